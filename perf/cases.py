@@ -248,9 +248,10 @@ def tolerance(case):
         return "exact"
     # The path computes the softmax weights in e4m3 (3 mantissa bits, about 2.5 % of each weight) after a
     # piecewise-linear exp2: against float64 the outputs are about 3 % off, and orders that quantise the weights against
-    # another running maximum differ by more than that from each other. The largest difference of one element is a few
-    # e4m3 steps (2^-3) of a row that few keys decide.
-    return {"rel": 0.03, "max": 0.5}
+    # another running maximum differ by up to 4 % from each other (measured at 2048 keys). The largest difference of one
+    # element, over the outputs' root mean square, belongs to a row that few keys decide: 0.43 between two such orders,
+    # and 0.62 against float64 under the causal mask, whose first rows see one to a few keys.
+    return {"rel": 0.03, "max": 0.9 if case["causal"] else 0.5}
 
 
 def _attention64(q, k, v, causal, scale, lse):
