@@ -125,10 +125,10 @@ int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, in
     if (bytes_q < elems) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "q: buffer smaller than B*SK*HK*128 bytes");
     if (bytes_scale < fmha_mxfp8_seq32_scale_bytes(B, SK, HK))
         return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "scale: buffer smaller than B*ceil(SK/32)*HK*128 bytes");
-    const uint64_t lanes = (uint64_t)B * nblk * (uint64_t)HK * 16u;
-    if ((lanes + 255) / 256 > 0xFFFFFFFFull) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
+    const uint64_t tiles = (uint64_t)B * nblk * (uint64_t)HK;   // one wave each, four to a workgroup
+    if ((tiles + 3) / 4 > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
     QuantSeq32Args a = {x, q, scale, (uint32_t)B, (uint32_t)SK, (uint32_t)HK, nblk};
-    return g_quant.launch(Q_SEQ32, &a, sizeof(a), (uint32_t)((lanes + 255) / 256), 1, 1, 256, stream, err, errlen);
+    return g_quant.launch(Q_SEQ32, &a, sizeof(a), (uint32_t)((tiles + 3) / 4), 1, 1, 256, stream, err, errlen);
 }
 
 }  // extern "C"

@@ -11,7 +11,7 @@
 // rule and layout; these kernels follow the FMHA generator so their bytes are the FMHA's inputs bit for bit.
 //
 // All three are HBM-bound streaming kernels: every lane moves 16-byte bf16 chunks (8 elements) in and 8-byte e4m3
-// chunks out; a 32-element block lives in 4 adjacent lanes (rows) or in one lane (sequence blocks).
+// chunks out; a 32-element block lives in 4 adjacent lanes (rows) or spread over a wave (sequence blocks).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -228,13 +228,15 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_tensor(QuantT
     if (blockIdx.x == 0 && threadIdx.x == 0) a.descale[0] = d;
 }
 
-// Sequence blocks: one lane per (b, 32-key block, kv head, 8-column chunk). Pass 1 takes the lane's 8 column maxima
-// over the block's keys, pass 2 reads the same 32 chunks again (from L2) and writes their e4m3 bytes, then the lane
-// writes its 8 scale bytes. A ragged last block (SK % 32 != 0) takes its maxima over the keys that exist.
+// Sequence blocks: one wave per tile of 32 keys x 128 columns of one (b, kv head). Lane l takes columns 8 (l & 15) .. +7 of
+// keys (l >> 4) + 4 j, j = 0..7: its eight 16-byte loads go out together (one wave instruction reads four 256-byte row
+// pieces) and stay in registers, so the tile is read once. The column maxima meet over the lanes l, l ^ 16, l ^ 32,
+// l ^ 48; each lane writes its eight 8-byte pieces, lanes 0..15 the 128 scale bytes. The heads of one 32-key block are
+// consecutive waves, so a workgroup reads up to 1 KiB of each key's row. Rows past a ragged last block (SK % 32 != 0)
+// re-read its last key, which changes no maximum, and are not stored.
 extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_seq32(QuantSeq32Args a) {
-    const uint64_t gid = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    const uint32_t c = (uint32_t)(gid & 15u);
-    uint64_t t = gid >> 4;
+    const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, r0 = lane >> 4;
+    uint64_t t = (uint64_t)blockIdx.x * 4u + (threadIdx.x >> 6);
     const uint32_t hk = (uint32_t)(t % a.HK);
     t /= a.HK;
     const uint32_t blk = (uint32_t)(t % a.nblk);
@@ -244,32 +246,43 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_seq32(QuantSe
     const uint32_t nk = min(32u, a.SK - k0);
     const uint64_t row_stride = (uint64_t)a.HK * 128u;
     const uint64_t base = ((uint64_t)b * a.SK + k0) * row_stride + (uint64_t)hk * 128u + c * 8u;
+    u32x4 w[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j)
+        w[j] = *reinterpret_cast<const u32x4*>(a.x + base + min(r0 + 4u * j, nk - 1u) * row_stride);
     float m[8];
-    for (int j = 0; j < 8; ++j) m[j] = 0.0f;
-    for (uint32_t k = 0; k < nk; ++k) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(a.x + base + k * row_stride);
-        for (int j = 0; j < 4; ++j) {
-            m[2 * j] = fmaxf(m[2 * j], fabsf(bf16_lo(w[j])));
-            m[2 * j + 1] = fmaxf(m[2 * j + 1], fabsf(bf16_hi(w[j])));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            m[2 * i] = fmaxf(m[2 * i], fabsf(bf16_lo(w[j][i])));   // fmaxf drops NaN, as in the rows kernel
+            m[2 * i + 1] = fmaxf(m[2 * i + 1], fabsf(bf16_hi(w[j][i])));
         }
-    }
     uint32_t e[8];
     float s[8];
-    for (int j = 0; j < 8; ++j) {
-        e[j] = e8m0_of_amax(m[j]);
-        s[j] = inv_scale(e[j]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        m[i] = fmaxf(m[i], __shfl_xor(m[i], 16, 64));
+        m[i] = fmaxf(m[i], __shfl_xor(m[i], 32, 64));
+        e[i] = e8m0_of_amax(m[i]);
+        s[i] = inv_scale(e[i]);
     }
-    for (uint32_t k = 0; k < nk; ++k) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(a.x + base + k * row_stride);
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) {
+        const uint32_t r = r0 + 4u * j;
         u32x2 out;
-        out[0] = pack4_e4m3(sat448(scaled(bf16_lo(w[0]), s[0])), sat448(scaled(bf16_hi(w[0]), s[1])),
-                            sat448(scaled(bf16_lo(w[1]), s[2])), sat448(scaled(bf16_hi(w[1]), s[3])));
-        out[1] = pack4_e4m3(sat448(scaled(bf16_lo(w[2]), s[4])), sat448(scaled(bf16_hi(w[2]), s[5])),
-                            sat448(scaled(bf16_lo(w[3]), s[6])), sat448(scaled(bf16_hi(w[3]), s[7])));
-        *reinterpret_cast<u32x2*>(a.q + base + k * row_stride) = out;
+        out[0] = pack4_e4m3(sat448(scaled(bf16_lo(w[j][0]), s[0])), sat448(scaled(bf16_hi(w[j][0]), s[1])),
+                            sat448(scaled(bf16_lo(w[j][1]), s[2])), sat448(scaled(bf16_hi(w[j][1]), s[3])));
+        out[1] = pack4_e4m3(sat448(scaled(bf16_lo(w[j][2]), s[4])), sat448(scaled(bf16_hi(w[j][2]), s[5])),
+                            sat448(scaled(bf16_lo(w[j][3]), s[6])), sat448(scaled(bf16_hi(w[j][3]), s[7])));
+        if (r < nk) store8_system(a.q + base + r * row_stride, out);
     }
-    u32x2 sc;
-    sc[0] = e[0] | (e[1] << 8) | (e[2] << 16) | (e[3] << 24);
-    sc[1] = e[4] | (e[5] << 8) | (e[6] << 16) | (e[7] << 24);
-    *reinterpret_cast<u32x2*>(a.scale + (((uint64_t)b * a.nblk + blk) * a.HK + hk) * 128u + c * 8u) = sc;
+    if (r0 == 0u) {
+        u32x2 sc;
+        sc[0] = e[0] | (e[1] << 8) | (e[2] << 16) | (e[3] << 24);
+        sc[1] = e[4] | (e[5] << 8) | (e[6] << 16) | (e[7] << 24);
+        *reinterpret_cast<u32x2*>(a.scale + (((uint64_t)b * a.nblk + blk) * a.HK + hk) * 128u + c * 8u) = sc;
+    }
 }

@@ -154,6 +154,22 @@ def test_seq32_matches_oracle(gpu, B, SK, HK):
     assert np.array_equal(_host(q), q_ref)
 
 
+@pytest.mark.parametrize("B,SK,HK", [(1, 31, 2), (2, 33, 5), (1, 4, 1), (3, 69, 3)])
+def test_seq32_special_values(gpu, B, SK, HK):
+    """Ragged 32-key blocks, a head count that leaves a workgroup's last waves idle, and every special bf16 value in
+    the columns (NaN, infinities, zeros of both signs, subnormals): bytes equal to the oracle's."""
+    rng = np.random.default_rng(SK * 31 + HK)
+    bits = _bf16_bits(rng.standard_normal(B * SK * HK * D).astype(np.float32))
+    special = np.array([0x7fc0, 0xffc1, 0x7f80, 0xff80, 0x0000, 0x8000, 0x0001, 0x8001, 0x7f7f], dtype=bits.dtype)
+    at = rng.choice(bits.size, bits.size // 5, replace=False)
+    bits[at] = rng.choice(special, at.size)
+    q, sc = ops.quantize_v_seq32(_dev(bits, gpu).view(B, SK, HK, D))
+    torch.cuda.synchronize()
+    q_ref, s_ref = oracle.quant_seq32_bf16(bits, B, SK, HK)
+    assert np.array_equal(_host(sc), s_ref)
+    assert np.array_equal(_host(q), q_ref)
+
+
 def test_rejections(gpu):
     x = torch.zeros(16, D, dtype=torch.bfloat16, device=gpu)
     q = torch.empty(16 * D, dtype=torch.uint8, device=gpu)
