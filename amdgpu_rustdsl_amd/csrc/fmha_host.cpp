@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -16,6 +17,7 @@
 
 #include "../../include/fmha_mxfp8.h"
 #include "module_cache.h"
+#include "packed_args.h"
 
 static_assert(sizeof(fmha_mxfp8_args) == 656, "kernarg size (vs128_abi.h:126)");
 static_assert(sizeof(fmha_mxfp8_params) == 192, "params layout (lib.py mirrors it)");
@@ -79,7 +81,7 @@ namespace {
 using fmha_internal::fail;
 using fmha_internal::set_err;
 
-const char* const kKernelNames[10] = {
+const char* const kKernelNames[13] = {
     "fmha_fwd_hd128_mxfp8_v3_vs128",
     "fmha_fwd_hd128_mxfp8_v3_t128",
     "fmha_fwd_hd128_mxfp8_v3_kvsplit",
@@ -93,9 +95,13 @@ const char* const kKernelNames[10] = {
     "fmha_fwd_hd128_mxfp8_v3_t128_split_tiles_scaled",
     // extension kernel: the combine with the splits spread over 4 waves (more than 8 partials per row)
     "fmha_fwd_hd128_mxfp8_v3_kvsplit_combine_wide",
+    // extension kernels: short query ranges, the rows of a KV head's query heads packed; the merge with the LSE output
+    "fmha_fwd_hd128_mxfp8_v3_packed",
+    "fmha_fwd_hd128_mxfp8_v3_packed_scaled",
+    "fmha_fwd_hd128_mxfp8_v3_combine_lse",
 };
 enum { K_VS128 = 0, K_T128 = 1, K_KVSPLIT = 2, K_COMBINE = 3, K_VS128_SC = 4, K_T128_SC = 5, K_KVSPLIT_SC = 6, K_T128ST = 7,
-       K_T128ST_SC = 8, K_COMBINE_WIDE = 9 };
+       K_T128ST_SC = 8, K_COMBINE_WIDE = 9, K_PACKED = 10, K_PACKED_SC = 11, K_COMBINE_LSE = 12 };
 
 // The 128-row grids (t128's shapes, and vs128's half-chip and causal ones below) run on the split-tile kernel (512
 // threads) from 7 key tiles on, and on the one-wave-per-SIMD kernel (256 threads, the reference's order) below that:
@@ -126,7 +132,7 @@ bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool caus
     return (S + 255) / 256 * H * B <= 128 || (causal && (SK + 127) / 128 >= 4);
 }
 
-fmha_internal::ModuleCache<10> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
+fmha_internal::ModuleCache<13> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
 
 int get_functions(hipFunction_t** out, char* err, size_t errlen) { return g_fmha.get(out, err, errlen); }
 
@@ -258,6 +264,100 @@ i64 kv_fill(i64 B, i64 H, i64 S, i64 SK, i64 splits) {
     while (sub < 8 && blocks * sub * 2 <= (i64)cu_count() && tiles >= 4 * splits * sub * 2 && !empty_split(SK, splits * sub * 2))
         sub *= 2;
     return sub;
+}
+
+// The packed-rows kernel (extension) for short query ranges: the shares `sub` that each of the `parts` key ranges is cut
+// into, or 0 to keep the path's own kernel. The rule compares estimated times (us, measured on MI355X):
+// - a block costs kBlock besides its tiles: arguments, first loads, epilogue;
+// - a 128-key tile costs a split-tile block kTile (less with idle waves: up to 96 rows), the 256-row kernel kTileWhole, and at
+//   least what its 32 KiB take at the 5 TB/s that the chip reads when `readers` blocks stream distinct keys;
+// - a merge that the path would not run anyway costs kMerge, and the partials their bytes, written and read back.
+// Measured against the path's own kernels (kernel times without / with it): B8 H32 HK8 S1 SK8192 96 / 32.1 + merge 3.9,
+// SK1024 19.0 / 10.0 + 3.4; B8 H32 HK8 S16 SK2048 28.3 / 14.0 + 3.8; KV split B1 H32 HK8 S1 SK16384 23.1 / 12.0,
+// B4 H16 HK4 S16 SK5000 17.9 / 11.3, B4 H8 HK1 S64 SK8192 16.5 / 12.4, B1 H8 S128 SK16000 15.3 / 13.7.
+// No gain, so the rule keeps the own kernel: full grids of 128-row blocks (B8 H8 S128 SK4096: 18.0 either way).
+i64 packed_sub(i64 B, i64 H, i64 HK, i64 S, i64 SK, i64 parts, bool whole, bool split_path, bool f32, i64 own_blocks, i64 max_parts) {
+    constexpr double kBlock = 6.0, kTile = 1.05, kTileIdle = 0.9, kTileWhole = 1.5, kMerge = 5.0, kReadTile = 0.0065, kBytes = 1.0e7;
+    const i64 tiles = (SK + 127) / 128, cus = cu_count(), rows = S * (H / HK), qtiles = (rows + 127) / 128;
+    if (S > 128 || tiles < 8) return 0;
+    const i64 t = (tiles + parts - 1) / parts, n = qtiles * HK * B * parts;
+    auto cost = [&](i64 blocks, i64 sharers, i64 per, double tile, i64 partials, double merge) {
+        const double readers = (double)std::min(blocks, cus) / (double)sharers;
+        const double bytes = partials ? 2.0 * (double)(partials * B * S * H) * (f32 ? 512.0 : 256.0) : 0.0;
+        return (double)((blocks + cus - 1) / cus) * ((double)per * std::max(tile, readers * kReadTile) + kBlock) + merge + bytes / kBytes;
+    };
+    double best = cost(own_blocks, H / HK, t, whole ? kTileWhole : kTile, split_path ? parts : 0, 0.0) - 0.5;
+    i64 sub = 0;
+    for (i64 s = 1; s <= 16 && s <= t && s * parts <= max_parts; ++s) {
+        const double c = cost(n * s, qtiles, (t + s - 1) / s, rows <= 96 ? kTileIdle : kTile, parts * s, split_path ? 0.0 : kMerge);
+        if (c < best) {
+            best = c;
+            sub = s;
+        }
+    }
+    return sub;
+}
+
+// What the one-call entry runs for a shape: the resolved path, and for the packed-rows kernel its shares.
+struct Plan {
+    int path, splits;   // as the entry reports them
+    i64 parts;          // KV-split partials (chunks x fill), 1 off the KV split
+    i64 sub;            // packed-rows shares of each partial's range; 0: the path's own kernel
+    bool whole;         // packed rows: the softmax reference over whole tiles
+    int kern;           // the path's own kernel (full-sequence paths)
+    uint32_t block, gx;
+};
+
+int kernel_of(int path, i64 B, i64 H, i64 S, i64 SK, bool causal, bool scaled, uint32_t* block, uint32_t* gx) {
+    if (path == FMHA_PATH_VS128 && !vs128_on_128row_grid(B, H, S, SK, causal)) {
+        *block = 512u;
+        *gx = (uint32_t)((S + 255) / 256);
+        return scaled ? K_VS128_SC : K_VS128;
+    }
+    // t128, or vs128 on the 128-row grid (same kernarg layout): the split-tile kernel or the 256-thread one
+    const bool st = use_split_tiles(B, H, S, SK, causal);
+    *block = st ? 512u : 256u;
+    *gx = (uint32_t)((S + 127) / 128);
+    return st ? (scaled ? K_T128ST_SC : K_T128ST) : (scaled ? K_T128_SC : K_T128);
+}
+
+// Fills the plan of a shape whose path (and, for the KV split, chunk count) is resolved. `workspace` is what the call may
+// use: partials that do not fit lower the fill, then the shares. `any_path` (fmha_fwd_hd128_mxfp8_auto_ws): shares, and a
+// workspace on the full-sequence paths too; the other entries keep the kernels and the bits that they had.
+void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspace, bool any_path) {
+    const i64 B = p.B, H = p.H, HK = p.HK, S = p.S, SK = p.SK;
+    const size_t one = fmha_mxfp8_workspace_bytes(B, H, S, 1);
+    const i64 fits = (i64)std::min<size_t>(workspace / one, 256);
+    pl.parts = 1;
+    pl.sub = 0;
+    pl.kern = -1;
+    if (pl.path == FMHA_PATH_KVSPLIT) {
+        i64 fill = p.kv_fill ? 1 : kv_fill(B, H, S, SK, pl.splits);
+        while (fill > 1 && fits < pl.splits * fill) fill /= 2;
+        pl.parts = pl.splits * fill;
+        pl.whole = false;
+        // kv_fill = 1 asks for the reference's grid
+        if (any_path && !p.kv_fill) pl.sub = packed_sub(B, H, HK, S, SK, pl.parts, false, true, p.f32_partials != 0, H * B * pl.parts, fits);
+    } else {
+        pl.kern = kernel_of(pl.path, B, H, S, SK, p.causal != 0, scaled, &pl.block, &pl.gx);
+        pl.whole = pl.kern != K_T128ST && pl.kern != K_T128ST_SC;
+        // a forced path keeps its kernel (and its bits)
+        if (any_path && p.path < 0 && p.kv_fill == 0)
+            pl.sub = packed_sub(B, H, HK, S, SK, 1, pl.whole, false, true, (i64)pl.gx * H * B, fits);
+    }
+    if (pl.sub > 0 && pl.parts * pl.sub * B * S * H * 512 >= (1LL << 32)) pl.sub = 0;   // the combines' 32-bit partial offsets
+}
+
+// path / splits as the entry resolves them from the params (no checks)
+void resolve_path(Plan& pl, const fmha_mxfp8_params& p) {
+    pl.splits = 0;
+    pl.path = p.path;
+    if (pl.path < 0) {
+        pl.path = fmha_mxfp8_select_path(p.B, p.H, p.S, p.SK, &pl.splits);
+        if (p.causal && pl.path == FMHA_PATH_KVSPLIT) pl.path = ((i64)(p.S + 255) / 256 * p.H * p.B <= 64) ? FMHA_PATH_T128 : FMHA_PATH_VS128;
+    } else if (pl.path == FMHA_PATH_KVSPLIT) {
+        pl.splits = p.splits > 0 ? p.splits : 4;
+    }
 }
 
 }  // namespace
@@ -416,22 +516,104 @@ int fmha_mxfp8_launch_combine_wide(const fmha_mxfp8_combine_args* a, uint32_t gx
     return launch_raw(K_COMBINE_WIDE, a, sizeof(*a), gx, 1, 1, 256, stream, nullptr, 0);
 }
 
-int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes, void* stream, int* path_out,
-                              int* splits_out, char* err, size_t errlen) {
+// The slot of the workspace that this call's partials go to, and the caller's turn word advanced.
+// Workspace slots: a workspace of k >= 2 times the need (rounded to 256 B) holds min(k, FMHA_WORKSPACE_SLOTS) sets
+// of partials, and consecutive calls take them in turn. The split kernel then writes lines that the previous
+// call's combine did not just read: writing over partials that the combine read in the kernel before cost
+// B1H8S2048 (4 splits) 25.6 -> 19.1 us per call with 4 slots (2 slots: 21.2, 8: 19.1, 16: 20.0).
+static uint8_t* workspace_slot(const fmha_mxfp8_params& p, void* workspace, size_t workspace_bytes, size_t need) {
+    const size_t stride = (need + 255u) & ~(size_t)255u;
+    size_t nslots = workspace_bytes / stride;
+    if (nslots < 1) nslots = 1;
+    if (nslots > FMHA_WORKSPACE_SLOTS) nslots = FMHA_WORKSPACE_SLOTS;
+    size_t slot = 0;
+    if (nslots > 1 && p.ws_turn) slot = (size_t)((*p.ws_turn)++ % nslots);
+    return (uint8_t*)workspace + slot * stride;
+}
+
+// The merge of `parts` partials per row into the output rows (and the LSE, when `lse` is not null).
+static int run_combine(const fmha_mxfp8_params& p, const uint8_t* ohat, const uint8_t* lse, i64 parts, bool f32, float* lse_out, void* stream,
+                       char* err, size_t errlen) {
+    const i64 rows_total = (i64)p.B * p.S * p.H;
+    struct LseArgs {
+        fmha_mxfp8_combine_args c;
+        uint32_t pad;
+        float* lse_out;
+        uint32_t S, H;
+    } la;
+    static_assert(sizeof(LseArgs) == 56 && offsetof(LseArgs, lse_out) == 40, "combine_lse kernarg");
+    fmha_mxfp8_combine_args& ca = la.c;
+    ca.ptr_ohat = const_cast<uint8_t*>(ohat);
+    ca.ptr_lse = const_cast<uint8_t*>(lse);
+    ca.ptr_out = p.o;
+    ca.rows_total = (uint32_t)rows_total;
+    ca.d = 128;
+    ca.splits = (uint32_t)parts | (f32 ? FMHA_KVS_F32_PARTIALS : 0u);
+    if (!p.no_check) {
+        fmha_mxfp8_buffer_sizes csz;
+        std::memset(&csz, 0, sizeof(csz));
+        csz.ptr_ohat = (uint64_t)parts * rows_total * 512;
+        csz.ptr_lse = (uint64_t)parts * rows_total * 4;
+        csz.ptr_o = p.bytes_o;
+        const int rc = fmha_mxfp8_validate_combine(&ca, &csz, 0, 1, 1, err, errlen);
+        if (rc != FMHA_OK) return rc;
+    }
+    // more than 8 partials per row: the combine with the splits spread over 4 waves (64 groups per block)
+    const bool wide = parts > 8 || lse_out;
+    const uint64_t cgrid = ((uint64_t)rows_total * 128 / 8 + (wide ? 63 : 255)) / (wide ? 64 : 256);
+    const uint32_t gx = (uint32_t)(cgrid ? cgrid : 1);
+    if (lse_out) {
+        la.pad = 0;
+        la.lse_out = lse_out;
+        la.S = (uint32_t)p.S;
+        la.H = (uint32_t)p.H;
+        return launch_raw(K_COMBINE_LSE, &la, sizeof(la), gx, 1, 1, 256, stream, err, errlen);
+    }
+    return launch_raw(wide ? K_COMBINE_WIDE : K_COMBINE, &ca, sizeof(ca), gx, 1, 1, 256, stream, err, errlen);
+}
+
+// The packed-rows kernel and its merge, for a plan with pl.sub > 0 (make_plan checked that the workspace holds the
+// partials, and the caller the extents).
+static int run_packed(const fmha_mxfp8_params& p, const Plan& pl, const fmha_mxfp8_args& a, void* workspace, size_t workspace_bytes, void* stream,
+                      char* err, size_t errlen) {
+    const i64 rows_total = (i64)p.B * p.S * p.H, parts = pl.parts * pl.sub;
+    // the full-sequence paths hold O and the row sums in f32 to the end, so their partials stay in f32
+    const bool f32 = pl.path != FMHA_PATH_KVSPLIT || p.f32_partials;
+    uint8_t* ohat = workspace_slot(p, workspace, workspace_bytes, fmha_mxfp8_workspace_bytes(p.B, p.H, p.S, (int)parts));
+    uint8_t* lse = ohat + (size_t)parts * rows_total * 512;
+    fmha_packed_args ka;
+    std::memset(&ka, 0, sizeof(ka));
+    ka.q = p.q; ka.k = p.k; ka.v = p.v;
+    ka.qs = p.q_descale; ka.ks = p.k_descale; ka.vd = p.v_descale;
+    ka.ohat = ohat;
+    ka.lse = lse;
+    ka.S = (uint32_t)p.S; ka.SK = (uint32_t)p.SK; ka.H = (uint32_t)p.H; ka.HK = (uint32_t)p.HK;
+    std::memcpy(&ka.softmax_scale, &a.softmax_scale, 4);
+    while ((p.HK << ka.gshift) < p.H) ++ka.gshift;
+    ka.parts = (uint32_t)pl.parts;
+    ka.sub = (uint32_t)pl.sub;
+    ka.groups = (uint32_t)(p.B * parts);
+    ka.rows_total = (uint32_t)rows_total;
+    ka.flags = (a.flags & (FMHA_FLAG_CAUSAL | FMHA_FLAG_V_SEQ32)) | (f32 ? kPackedF32 : 0u) | (pl.whole ? kPackedWhole : 0u);
+    const i64 qtiles = ((i64)p.S * (p.H / p.HK) + 127) / 128;
+    const int rc = launch_raw((a.flags & FMHA_FLAG_SCALE) ? K_PACKED_SC : K_PACKED, &ka, sizeof(ka), (uint32_t)(qtiles * p.HK * p.B * parts), 1, 1, 512,
+                              stream, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    return run_combine(p, ohat, lse, parts, f32, pl.path == FMHA_PATH_KVSPLIT ? nullptr : (float*)p.lse, stream, err, errlen);
+}
+
+// any_path: as in make_plan
+static int run_entry(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes, bool any_path, void* stream, int* path_out,
+                     int* splits_out, char* err, size_t errlen) {
     if (!p) return fail(err, errlen, FMHA_ERR_PATH, "GV-HOST-ARGS", "null params");
     const i64 B = p->B, H = p->H, HK = p->HK, S = p->S, SK = p->SK;
     if (B < 1 || H < 1 || HK < 1 || S < 1 || SK < 1)
         return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "B, H, HK, S, SK must be >= 1");
     if (H % HK != 0 || ((H / HK) & (H / HK - 1)) != 0 || H / HK > 16)
         return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "H must be a power-of-two multiple (<= 16) of HK");
-    int splits = 0;
-    int path = p->path;
-    if (path < 0) {
-        path = fmha_mxfp8_select_path(B, H, S, SK, &splits);
-        if (p->causal && path == FMHA_PATH_KVSPLIT) path = ((S + 255) / 256 * H * B <= 64) ? FMHA_PATH_T128 : FMHA_PATH_VS128;
-    } else if (path == FMHA_PATH_KVSPLIT) {
-        splits = p->splits > 0 ? p->splits : 4;
-    }
+    Plan pl;
+    resolve_path(pl, *p);
+    const int path = pl.path, splits = pl.splits;
     if (path != FMHA_PATH_VS128 && path != FMHA_PATH_T128 && path != FMHA_PATH_KVSPLIT)
         return fail(err, errlen, FMHA_ERR_PATH, "GV-HOST-PATH", "unknown path");
     if (path == FMHA_PATH_KVSPLIT) {
@@ -458,13 +640,9 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
     std::memset(&sz, 0, sizeof(sz));
     sz.ptr_q = p->bytes_q; sz.ptr_k = p->bytes_k; sz.ptr_v = p->bytes_v; sz.ptr_o = p->bytes_o;
     sz.ptr_q_descale = p->bytes_q_descale; sz.ptr_k_descale = p->bytes_k_descale; sz.ptr_v_descale = p->bytes_v_descale;
-    // the KV split's partial count: the chunks times the fill, as far as the workspace holds it
-    i64 parts = splits;
-    if (path == FMHA_PATH_KVSPLIT) {
-        i64 sub = p->kv_fill ? 1 : kv_fill(B, H, S, SK, splits);
-        while (sub > 1 && workspace_bytes < fmha_mxfp8_workspace_bytes(B, H, S, (int)(splits * sub))) sub /= 2;
-        parts = splits * sub;
-    }
+    // the KV split's partial count: the chunks times the fill, as far as the workspace holds it; the packed-rows shares
+    make_plan(pl, *p, scaled, workspace ? workspace_bytes : 0, any_path);
+    i64 parts = pl.parts;
     if (path == FMHA_PATH_KVSPLIT && parts * B * S * H * 512 >= (1LL << 32))
         // a kernel-contract limit (32-bit partial offsets), checked with or without no_check
         return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "ka(0x284) outside contract (partials of 4 GiB or more)");
@@ -481,17 +659,10 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
                                                    : fmha_mxfp8_validate_t128(&a, &sz, gx, gy, (uint32_t)B, HK, err, errlen);
             if (rc != FMHA_OK) return rc;
         }
-        uint32_t block = 512u, kgx = gx;
-        int kern;
-        if (path == FMHA_PATH_VS128 && !vs128_on_128row_grid(B, H, S, SK, p->causal != 0)) {
-            kern = scaled ? K_VS128_SC : K_VS128;
-        } else {
-            // t128, or vs128 on the 128-row grid (same kernarg layout): the split-tile kernel or the 256-thread one
-            const bool st = use_split_tiles(B, H, S, SK, p->causal != 0);
-            kern = st ? (scaled ? K_T128ST_SC : K_T128ST) : (scaled ? K_T128_SC : K_T128);
-            block = st ? 512u : 256u;
-            kgx = (uint32_t)((S + 127) / 128);
-        }
+        if (pl.sub > 0) return run_packed(*p, pl, a, workspace, workspace_bytes, stream, err, errlen);
+        const int kern = pl.kern;
+        const uint32_t block = pl.block;
+        uint32_t kgx = pl.gx;
         // the causal q-tile pairing when the grid would take more than one wave of blocks (the extension's flag; the
         // reference pairs its causal kernels' tiles always, grid.rs:94-111), or when the caller asks for it
         const bool pair = p->causal && kern != K_VS128 && kern != K_VS128_SC && kgx > 1 &&
@@ -509,17 +680,7 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
         set_err(err, errlen, "GV-HOST-WORKSPACE: KV split needs %zu workspace bytes, got %zu", need, workspace_bytes);
         return FMHA_ERR_WORKSPACE;
     }
-    // Workspace slots: a workspace of k >= 2 times the need (rounded to 256 B) holds min(k, FMHA_WORKSPACE_SLOTS) sets
-    // of partials, and consecutive calls take them in turn. The split kernel then writes lines that the previous
-    // call's combine did not just read: writing over partials that the combine read in the kernel before cost
-    // B1H8S2048 (4 splits) 25.6 -> 19.1 us per call with 4 slots (2 slots: 21.2, 8: 19.1, 16: 20.0).
-    const size_t stride = (need + 255u) & ~(size_t)255u;
-    size_t nslots = workspace_bytes / stride;
-    if (nslots < 1) nslots = 1;
-    if (nslots > FMHA_WORKSPACE_SLOTS) nslots = FMHA_WORKSPACE_SLOTS;
-    size_t slot = 0;
-    if (nslots > 1 && p->ws_turn) slot = (size_t)((*p->ws_turn)++ % nslots);
-    uint8_t* ohat = (uint8_t*)workspace + slot * stride;
+    uint8_t* ohat = pl.sub > 0 ? (uint8_t*)workspace : workspace_slot(*p, workspace, workspace_bytes, need);
     uint8_t* lse = ohat + (size_t)parts * rows_total * 512;
     fmha_mxfp8_kvsplit_args ka;
     std::memcpy(&ka, &a, 0x270);
@@ -533,26 +694,30 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
     const uint32_t gx = (uint32_t)((S + 255) / 256), gz = (uint32_t)(B * parts);
     int rc = p->no_check ? FMHA_OK : fmha_mxfp8_validate_kvsplit(&ka, &sz, gx, gy, gz, B, HK, 0, err, errlen);
     if (rc != FMHA_OK) return rc;
+    if (pl.sub > 0) return run_packed(*p, pl, a, workspace, workspace_bytes, stream, err, errlen);
     rc = launch_raw(scaled ? K_KVSPLIT_SC : K_KVSPLIT, &ka, sizeof(ka), gx, gy, gz, 512, stream, err, errlen);
     if (rc != FMHA_OK) return rc;
-    fmha_mxfp8_combine_args ca;
-    ca.ptr_ohat = ohat;
-    ca.ptr_lse = lse;
-    ca.ptr_out = p->o;
-    ca.rows_total = (uint32_t)rows_total;
-    ca.d = 128;
-    ca.splits = (uint32_t)parts | part_fmt;
-    fmha_mxfp8_buffer_sizes csz = sz;
-    csz.ptr_o = p->bytes_o;
-    if (!p->no_check) {
-        rc = fmha_mxfp8_validate_combine(&ca, &csz, 0, 1, 1, err, errlen);
-        if (rc != FMHA_OK) return rc;
-    }
-    // more than 8 partials per row: the combine with the splits spread over 4 waves (64 groups per block)
-    const bool wide = parts > 8;
-    const uint64_t cgrid = ((uint64_t)rows_total * 128 / 8 + (wide ? 63 : 255)) / (wide ? 64 : 256);
-    return launch_raw(wide ? K_COMBINE_WIDE : K_COMBINE, &ca, sizeof(ca), (uint32_t)(cgrid ? cgrid : 1), 1, 1, 256, stream, err,
-                      errlen);
+    return run_combine(*p, ohat, lse, parts, p->f32_partials != 0, nullptr, stream, err, errlen);
+}
+
+int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes, void* stream, int* path_out,
+                              int* splits_out, char* err, size_t errlen) {
+    return run_entry(p, workspace, workspace_bytes, false, stream, path_out, splits_out, err, errlen);
+}
+
+int fmha_fwd_hd128_mxfp8_auto_ws(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes, void* stream, int* path_out,
+                                 int* splits_out, char* err, size_t errlen) {
+    return run_entry(p, workspace, workspace_bytes, true, stream, path_out, splits_out, err, errlen);
+}
+
+size_t fmha_mxfp8_auto_workspace_bytes(const fmha_mxfp8_params* p) {
+    if (!p || p->B < 1 || p->H < 1 || p->HK < 1 || p->S < 1 || p->SK < 1 || p->H % p->HK != 0) return 0;
+    Plan pl;
+    resolve_path(pl, *p);
+    if (pl.path != FMHA_PATH_VS128 && pl.path != FMHA_PATH_T128 && pl.path != FMHA_PATH_KVSPLIT) return 0;
+    make_plan(pl, *p, p->softmax_scale != 0.0f, ~(size_t)0, true);
+    if (pl.sub > 0) return fmha_mxfp8_workspace_bytes(p->B, p->H, p->S, (int)(pl.parts * pl.sub));
+    return pl.path == FMHA_PATH_KVSPLIT ? fmha_mxfp8_workspace_bytes(p->B, p->H, p->S, (int)pl.parts) : 0;
 }
 
 }  // extern "C"

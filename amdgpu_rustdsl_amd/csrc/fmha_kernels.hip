@@ -32,6 +32,7 @@
 #include <stdint.h>
 
 #include "../../include/fmha_mxfp8.h"
+#include "packed_args.h"
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -105,6 +106,11 @@ struct Prm {
     float qk_m, qk_rm;
     int32_t qk_e;
     uint32_t qk_scaled;
+    // the packed-rows kernel (extension): rows of one KV head, row r = query r >> pk_sh, head (KV head << pk_sh) + the
+    // low bits of r; pk_rows of them. seed_key: the first key of the tile the softmax reference comes from (-1: none)
+    uint32_t pk_rows, pk_sh;
+    int32_t seed_key;
+    uint32_t seed_whole;
 #ifdef FMHA_TRACE
     uint64_t* trace;   // debug builds only: per (block, wave) timestamps, pointer at kernarg 0x288
     uint64_t t_entry;  // timestamp of the kernel's first instruction
@@ -603,6 +609,8 @@ struct Wave {
     // (16 VGPRs) for the whole key range: re-reading them from LDS every tile cost 32 KiB of LDS reads per tile and block.
     // rwave: the wave's 32-row block in the block's rows (its wave index, or wave % 4 when the two groups share rows);
     // rb: query rows per block (ROWS, or 128 for the full-sequence split-tile kernel)
+    // PK: packed rows (Prm::pk_sh); `head` is then the KV head's first query head
+    template <bool PK = false>
     __device__ __forceinline__ void init(const Prm& p, uint32_t lds_, uint32_t qtile, uint32_t head, uint32_t bidx, uint32_t key_hi_,
                                          uint32_t rwave, uint32_t rb = ROWS) {
         lane = threadIdx.x & 63u;
@@ -612,8 +620,10 @@ struct Wave {
         lds = lds_;
         key_hi = key_hi_;
         row0 = qtile * rb + rwave * 32u;
-        const uint32_t row = row0 + n;
-        const uint32_t row_c = min(row, p.S - 1u);
+        const uint32_t prow = PK ? min(row0 + n, p.pk_rows - 1u) : 0u;
+        if (PK) head += prow & ((1u << p.pk_sh) - 1u);
+        const uint32_t row = PK ? prow >> p.pk_sh : row0 + n;
+        const uint32_t row_c = PK ? row : min(row, p.S - 1u);
         kfo = n * 128u + ((hh ^ swz(n)) << 4);
         kso = hh * 512u + n * 4u;
         vso = hh * 128u + n;
@@ -630,8 +640,9 @@ struct Wave {
         if (p.flags & 1u) {
             const int off = (int)p.SK - (int)p.S + 1;
             lim_row = (uint32_t)max(0, min((int)key_hi, (int)row + off));
-            lim_wave_min = (uint32_t)max(0, min((int)key_hi, (int)row0 + off));
-            lim_wave_max = (uint32_t)max(0, min((int)key_hi, (int)row0 + 31 + off));
+            const int first = PK ? (int)(min(row0, p.pk_rows - 1u) >> p.pk_sh) : (int)row0;
+            lim_wave_min = (uint32_t)max(0, min((int)key_hi, first + off));
+            lim_wave_max = (uint32_t)max(0, min((int)key_hi, first + 31 + off));
         }
         {
             // ds_read_b64_tr_b8 source lane (g, jj, pp) reads key 16 r + rlo of the 64-key half, dims
@@ -1036,7 +1047,9 @@ __device__ __forceinline__ v4i merge_finish(const MergeState& st) {
 // before staging over the ring, comes after B's stores are issued. (The 256-thread kernel's waves end together:
 // there the two rounds cost more than the barrier saves.) DCH: the dims the wave writes: 0 all, 1 dims 0..63 (dc 0, 1),
 // 2 dims 64..127 (dc 2, 3; the LSE is left to the DCH 1 wave of the same rows).
-template <bool SPLIT, int NT, bool TAIL = false, int DCH = 0>
+// PK: the packed-rows kernel's partials (SPLIT): row r of the wave's KV head is query r >> pk_sh of head
+// `head` + (r & (2^pk_sh - 1)).
+template <bool SPLIT, int NT, bool TAIL = false, int DCH = 0, bool PK = false>
 __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32_t head, uint32_t bidx, uint32_t split, const Recipe& rc,
                                          bool sync) {
     // lane-derived values recomputed here from an opaque lane id: kept from the prologue they would be live (and
@@ -1045,6 +1058,11 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
     asm volatile("" : "+s"(all));   // an opaque mask, so the lane index is computed here (see lane_addr on inline asm)
     const uint32_t lane = __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
     const uint32_t hh = lane >> 5, n = lane & 31u, row = w.row0 + n;
+    static_assert(!PK || SPLIT, "packed rows are written as partials");
+    const uint32_t nrows = PK ? p.pk_rows : p.S;
+    auto pk_prow = [&](uint32_t r) -> size_t {   // partial row of packed row r
+        return (size_t)split * p.rows_total + ((size_t)bidx * p.S + (r >> p.pk_sh)) * p.H + head + (r & ((1u << p.pk_sh) - 1u));
+    };
     const float l = row_sum(w.lacc, lane);
     const uint32_t dbase = 4u * hh;
     const bool f32 = SPLIT && p.f32_partials;
@@ -1071,8 +1089,8 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
     }
     if (f32) {
         // extension: f32 rows of 512 B (the workspace's rows are fp32-sized either way), stored directly
-        if (row < p.S) {
-            uint8_t* orow = obase + (size_t)n * ostride;
+        if (row < nrows) {
+            uint8_t* orow = PK ? p.ohat + pk_prow(row) * 512u : obase + (size_t)n * ostride;
 #pragma unroll
             for (int dc = kDc0; dc < kDc1; ++dc)
 #pragma unroll
@@ -1132,8 +1150,8 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
                 for (int k = 0; k < 4; ++k) {
                     const uint32_t r = 8u * k + (lane >> 3);
                     const v4i x = lds_read16(sbase + r * kEpiRow + c8 * 16u);
-                    if (w.row0 + r < p.S) {
-                        store16_system(obase + (size_t)r * ostride + c8 * 16u, x);
+                    if (w.row0 + r < nrows) {
+                        store16_system((PK ? p.ohat + pk_prow(w.row0 + r) * 256u : obase + (size_t)r * ostride) + c8 * 16u, x);
                     }
                 }
             }
@@ -1164,7 +1182,7 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
             if (sync) block_barrier();   // pairs with A's barrier before its staging
         }
     }
-    if (row >= p.S || hh != 0 || DCH == 2) return;
+    if (row >= nrows || hh != 0 || DCH == 2) return;
     if (!SPLIT) {
         if (p.lse_out) {
             // natural-log LSE of the scores (extension): P = 2^(S + 512 b - 127) / conv, l = sum P
@@ -1176,7 +1194,7 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
     } else {
         const float l_total = l * 0.0625f;
         const float hl = h2f(w.bw) + h2f(w.bw >> 16);
-        const size_t prow = (size_t)split * p.rows_total + ((size_t)bidx * p.S + row) * p.H + head;
+        const size_t prow = PK ? pk_prow(row) : (size_t)split * p.rows_total + ((size_t)bidx * p.S + row) * p.H + head;
         // an empty range (l = 0) gets -1e30: the combine gives it weight 0
         // a write-back store: the H words of a row are consecutive, and the KV split's one-query-tile grids put the
         // blocks of those H heads on one XCD (kvsplit_kernel), so its L2 merges them into whole lines (written through,
@@ -1248,7 +1266,13 @@ __device__ __forceinline__ void merge_halves(Wave<NT>& w, uint32_t lds) {
 // tile's keys instead, A keys 0..63 and B keys 64..127 (two of the four 32-key accumulators, half the MFMAs); the
 // schedule, the ring and the copies are unchanged. After the loop B hands its softmax state to A through LDS and A
 // merges the two (merge_halves).
-template <bool LUT, bool SPLIT, bool GB, bool VS, bool HV, bool SC>
+//
+// PK (the packed-rows kernel, HV): the block's rows are packed (Prm::pk_sh), and its key range may be a later part of a
+// range whose first tile fixes the softmax reference: before its own tiles it takes that tile's row max (K seed_key,
+// through K slot 3) exactly as the whole range's first tile would, so P is quantised on the same grid wherever the
+// range is cut. seed_whole: the reference is the maximum over the tile's 128 keys (the whole-tile kernels' order),
+// else over the group's own 64 keys (the split-tile order).
+template <bool LUT, bool SPLIT, bool GB, bool VS, bool HV, bool SC, bool PK = false>
 __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds, uint32_t qtile, uint32_t head, uint32_t bidx,
                                                       uint32_t split, uint32_t key_lo, uint32_t key_hi) {
     constexpr int NT = 512;
@@ -1257,7 +1281,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
     const Recipe rc = recipe(LUT);
     // rows per block: 256, or 128 for the full-sequence split-tile kernel (the KV split's split-tile blocks keep the
     // 256-row grid and use their first 128 rows)
-    constexpr uint32_t RB = HV && !SPLIT ? 128u : 256u;
+    constexpr uint32_t RB = HV && (!SPLIT || PK) ? 128u : 256u;
     const uint32_t tblk = ((bidx * p.splits + split) * p.H + head) * ((p.S + RB - 1u) / RB) + qtile;   // trace slot
     (void)tblk;
     FMHA_MARK(p, tblk, 0);
@@ -1265,12 +1289,12 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
     if (p.trace && (threadIdx.x & 63u) == 0u) p.trace[((size_t)tblk * 8u + (threadIdx.x >> 6)) * 8u + 7u] = p.t_entry;
 #endif
     Wave<NT> w;
-    w.init(p, lds, qtile, head, bidx, key_hi, HV ? wave_id() & 3u : wave_id(), RB);
+    w.template init<PK>(p, lds, qtile, head, bidx, key_hi, HV ? wave_id() & 3u : wave_id(), RB);
     FMHA_MARK(p, tblk, 1);
     const uint32_t kvh = head / p.gqa;
     const bool causal = (p.flags & 1u) != 0;
     uint32_t key_end = key_hi;   // the block's last useful key + 1
-    if (causal) key_end = (uint32_t)max(0, min((int)key_hi, (int)(qtile * RB + RB - 1) + (int)p.SK - (int)p.S + 1));
+    if (causal && !PK) key_end = (uint32_t)max(0, min((int)key_hi, (int)(qtile * RB + RB - 1) + (int)p.SK - (int)p.S + 1));
     const uint32_t ntiles = key_end > key_lo ? (key_end - key_lo + kTile - 1) / kTile : 0;
 
     Stager<NT> st;
@@ -1300,11 +1324,15 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         st.init_dma();
         const uint32_t ks0 = st.ks_word(key_of(0), true);
         const uint32_t ks1 = st.ks_word(key_of(1), ntiles > 1);
+        const bool seed = PK && p.seed_key >= 0;
+        const uint32_t kss = seed ? st.ks_word((uint32_t)p.seed_key, true) : 0u;
         st.load_ks(key_of(2), ntiles > 2);                              // stored by V(0)
         // The first barrier needs K 0, V 0 and K 1 (read in I(0)); V 1 and K 2 are first read in I(1), so barrier 0
         // waits for them and they stay out of the first barrier's burst.
         st.dma(key_of(0), true, 0, key_of(0), true, 0);                 // K 0, V 0
         st.dma(key_of(1), ntiles > 1, 1, key_of(1), false, 3);          // K 1 (V slot 3 gets zeros, nothing reads it yet)
+        // the seed tile's K, in slot 3 until V(0)'s copies (after the barrier below)
+        if (seed) st.dma((uint32_t)p.seed_key, true, 3, key_of(1), false, 3);
         if (VS) st.dma_vs(key_of(0), true, 0);                          // V scales of tile 0
         // The stores of the words wait for their loads. The compiler counts only its own loads (not the copies' inline
         // assembly), so its wait there leaves at most two VMEM operations of any kind in flight: placed before the
@@ -1312,6 +1340,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         // -2.4 %, cfg3 -0.6 %).
         st.store_ks_word(ks0, 0);
         st.store_ks_word(ks1, 1);
+        if (seed) st.store_ks_word(kss, 3);
         w.commit_q();   // (its wait for the Q scale word likewise comes before the copies of K 2 and V 1)
         st.dma(key_of(2), ntiles > 2, 2, key_of(1), ntiles > 1, 1);     // K 2, V 1
         if (VS) st.dma_vs(key_of(1), ntiles > 1, 1);                    // V scales of tile 1
@@ -1320,9 +1349,42 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         FMHA_MARK(p, tblk, 2);
         block_barrier();
         FMHA_MARK(p, tblk, 3);
-        w.template qk_all<KB0>(0, s);
-        float mrow = row_max(s);   // unmasked row max of the tile the next VALU phase decides on
-        {
+        if (seed) {
+            const uint32_t sk = (uint32_t)p.seed_key;
+            // row max of the seed tile's blocks B0 .. B0 + NA - 1, scaled and masked as V(t) does it
+            auto half_max = [&](auto b0) {
+                constexpr int B0 = decltype(b0)::value;
+                w.template qk_all<B0>(3, s);
+                float m = row_max(s);
+                if (SC) w.scale_s(s, m);
+                if (w.needs_mask(sk)) {
+                    w.template apply_mask<B0>(s, sk);
+                    m = row_max(s);
+                }
+                return m;
+            };
+            float m = half_max(std::integral_constant<int, KB0>{});
+            if (p.seed_whole) m = fmaxf(m, half_max(std::integral_constant<int, 2 - KB0>{}));
+            rebase<LUT>(rc, m, s, w.o, w.lacc, w.bias, w.bw, w.qrm);   // (O and the row sums are zero)
+            block_barrier();   // every wave has read K slot 3
+        }
+        // a wave without rows (decode-like row counts) only carries its share of the copies and the barriers
+        const bool idle = PK && w.row0 >= p.pk_rows;
+        if (idle) {
+            for (uint32_t t = 0; t < ntiles; ++t) {
+                st.store_ks(slot_of(t + 2));
+                st.dma(key_of(t + 3), t + 3 < ntiles, slot_of(t + 3), key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                st.load_ks(key_of(t + 3), t + 3 < ntiles);
+                block_barrier_keep_dma<0, kDmaOps>();
+            }
+        }
+        float mrow = 0.0f;
+        if (!idle) {
+            w.template qk_all<KB0>(0, s);
+            mrow = row_max(s);   // unmasked row max of the tile the next VALU phase decides on
+        }
+        if (!idle) {
             typename Wave<NT>::Ring ring;
             typename Wave<NT>::QkPre pre;
             // V(t)'s copies: K tile t+3 and V tile t+2 (and the per-32-key V scales), the K-scale words of tile t+3
@@ -1387,18 +1449,18 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         // HV: each group finishes half of every row's dims (A 0..63, B 64..127); the merge's barriers retired the ring
         merge_halves<GB>(w, lds);
         FMHA_MARK(p, tblk, 6);
-        epilogue<SPLIT, NT, false, GB ? 2 : 1>(p, w, head, bidx, split, rc, false);
+        epilogue<SPLIT, NT, false, GB ? 2 : 1, PK>(p, w, head, bidx, split, rc, false);
     }
     FMHA_MARK(p, tblk, 5);
 }
 
 // The whole routine is instantiated per group (the groups place their barrier differently; one body with a
 // group-dependent branch, or two loop copies sharing a prologue, made the register allocation spill).
-template <bool LUT, bool SPLIT, bool VS, bool HV, bool SC>
+template <bool LUT, bool SPLIT, bool VS, bool HV, bool SC, bool PK = false>
 __device__ __forceinline__ void attend_pingpong(const Prm& p, uint32_t lds, uint32_t qtile, uint32_t head, uint32_t bidx, uint32_t split,
                                 uint32_t key_lo, uint32_t key_hi) {
-    if (wave_id() >= 4u) attend_pingpong_group<LUT, SPLIT, true, VS, HV, SC>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
-    else attend_pingpong_group<LUT, SPLIT, false, VS, HV, SC>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
+    if (wave_id() >= 4u) attend_pingpong_group<LUT, SPLIT, true, VS, HV, SC, PK>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
+    else attend_pingpong_group<LUT, SPLIT, false, VS, HV, SC, PK>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
 }
 
 // One 4-wave block of 128 rows with one wave per SIMD (_t128 under its own 256-thread contract). Nothing else runs on
@@ -1666,6 +1728,61 @@ __device__ __forceinline__ void t128_split_tiles_kernel(uint32_t lds) {
     }
 }
 
+// The packed-rows kernel (extension): short query ranges (S <= 128) over long KV ranges, decode steps among them. The rows
+// of one KV head's query heads are packed into 128-row blocks (row r = query r / group, head r % group), so K and V are
+// read once per KV head instead of once per query head and a block's rows are not padding; each of the reference's
+// `parts` key ranges is cut into `sub` further ones, one block each, until the grid fills the CUs. Bound by HBM: a
+// split-tile block streams a 32 KiB key tile in ~1.05 us, 8 TB/s over 256 CUs.
+template <bool SC>
+__device__ __forceinline__ void packed_kernel(uint32_t lds) {
+    Prm p;
+#define PK_FIELD(T, field) ka<T>(offsetof(fmha_packed_args, field))
+    p.q = (const uint8_t*)PK_FIELD(uint64_t, q); p.k = (const uint8_t*)PK_FIELD(uint64_t, k); p.v = (const uint8_t*)PK_FIELD(uint64_t, v);
+    p.qs = (const uint8_t*)PK_FIELD(uint64_t, qs); p.ks = (const uint8_t*)PK_FIELD(uint64_t, ks);
+    p.vd = (const float*)PK_FIELD(uint64_t, vd);
+    p.ohat = (uint8_t*)PK_FIELD(uint64_t, ohat); p.lse = (float*)PK_FIELD(uint64_t, lse);
+    p.S = PK_FIELD(uint32_t, S); p.SK = PK_FIELD(uint32_t, SK); p.H = PK_FIELD(uint32_t, H);
+    const uint32_t HK = PK_FIELD(uint32_t, HK), parts = PK_FIELD(uint32_t, parts), sub = PK_FIELD(uint32_t, sub);
+    const uint32_t flags = PK_FIELD(uint32_t, flags), groups = PK_FIELD(uint32_t, groups);
+    p.pk_sh = PK_FIELD(uint32_t, gshift);
+    p.rows_total = PK_FIELD(uint32_t, rows_total);
+#undef PK_FIELD
+    p.gqa = 1u << p.pk_sh;
+    p.flags = flags & FMHA_FLAG_CAUSAL;
+    p.f32_partials = (flags & kPackedF32) ? 1u : 0u;
+    p.seed_whole = (flags & kPackedWhole) ? 1u : 0u;
+    p.q_seq = p.H * 128u; p.q_b = p.S * p.q_seq;
+    p.k_seq = p.v_seq = HK * 128u; p.k_b = p.v_b = p.SK * p.k_seq;
+    p.qs_b = p.S * p.H * 4u; p.ks_b = p.SK * HK * 4u;
+    p.o = nullptr; p.o_seq = p.o_b = 0u; p.lse_out = nullptr;
+    p.vs32 = (flags & FMHA_FLAG_V_SEQ32) ? (const uint8_t*)p.vd : nullptr;
+    p.vs_row = p.k_seq;
+    p.vs_b = ((p.SK + 31u) >> 5) * p.vs_row;
+    p.splits = parts * sub;
+    p.pk_rows = p.S << p.pk_sh;
+    set_qk_scale(p, SC);
+    // block -> (row tile, KV head, group), a group being one key range of one batch: the KV heads of a group are consecutive
+    // 128-byte pieces of the same K and V rows and LSE rows, and the row tiles of one head share its K and V, so a
+    // group's blocks go to one XCD when the groups are a multiple of 8 (the hardware deals blocks round-robin over them)
+    const uint32_t qtiles = (p.pk_rows + 127u) >> 7, L = blockIdx.x, gb = qtiles * HK;
+    const bool by_xcd = (groups & 7u) == 0u;
+    const uint32_t j = by_xcd ? L >> 3 : L;
+    const uint32_t qt = __builtin_amdgcn_readfirstlane(j % qtiles);
+    const uint32_t hk = __builtin_amdgcn_readfirstlane(j / qtiles % HK);
+    const uint32_t group = __builtin_amdgcn_readfirstlane(by_xcd ? (j / gb) * 8u + (L & 7u) : j / gb);
+    const uint32_t split = group % p.splits, bidx = group / p.splits;
+    // range `part` of the reference's chunks (its tiles as in kvsplit_kernel), of which this block runs the sub-th share
+    const uint32_t ntiles = (p.SK + 127u) / 128u, tps = (ntiles + parts - 1u) / parts;
+    const uint32_t lo = min(ntiles, split / sub * tps), hi = min(ntiles, lo + tps);
+    const uint32_t per = (hi - lo + sub - 1u) / sub;
+    const uint32_t t0 = min(hi, lo + split % sub * per), t1 = min(hi, t0 + per);
+    const uint32_t key_lo = t0 * 128u, key_hi = min(t1 * 128u, p.SK);
+    p.seed_key = p.seed_whole || t0 != lo ? (int32_t)(lo * 128u) : -1;
+    const uint32_t head = hk << p.pk_sh;
+    if (p.vs32) attend_pingpong<false, true, true, true, SC, true>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+    else attend_pingpong<false, true, false, true, SC, true>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+}
+
 }  // namespace
 
 #define FMHA_LDS_BASE(name)                                                 \
@@ -1724,6 +1841,19 @@ extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_t12
     t128_split_tiles_kernel<true>(smem_base);
 }
 
+// Extension kernels (no counterpart in the reference): packed rows, fmha_packed_args.
+extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_packed(fmha_packed_args a) {
+    FMHA_LDS_BASE(smem);
+    (void)a;
+    packed_kernel<false>(smem_base);
+}
+
+extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_packed_scaled(fmha_packed_args a) {
+    FMHA_LDS_BASE(smem);
+    (void)a;
+    packed_kernel<true>(smem_base);
+}
+
 // epilogue.rs:89-167 / io.rs:164-185: thread t -> 8 consecutive outputs of row t >> 4 (tail threads redo the last group)
 // The combines take the 36-byte layout (fmha_mxfp8_combine_args: three pointers, then rows_total, d and the split
 // field at 0x18, 0x1C, 0x20) as scalar parameters, which lay out the same bytes: as scalars the nine dwords are preloaded
@@ -1755,9 +1885,12 @@ extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_kvspli
 // the last group); wave p merges the p-th quarter of the splits (ceil(splits / 4) each, in order), and wave 0 merges
 // the quarters in order through LDS. With the reference kernel's layout one thread walks every split of its group in
 // turn: at 32 splits that is 4 dependent rounds of loads on 64 groups per block (13.7 us at 1024 rows on MI355X).
-extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_kvsplit_combine_wide(FMHA_COMBINE_PARAMS) {
-    (void)d;
-    __shared__ float part[3][10][64];
+// LSE: also the natural-log LSE [B, H, S] of each row, which the full-sequence paths write themselves when they are not
+// split: log2 l - 2048 (hi + lo) is the merged base-2 LSE plus 4 (the partials carry l / 16), and the constants are
+// those of the epilogue's LSE output (the lazy recipe).
+template <bool LSE>
+__device__ __forceinline__ void combine_wide(float (&part)[3][10][64], const uint8_t* ohat, const float* lse, uint8_t* out, uint32_t rows,
+                                             uint32_t split_field, float* lse_out, uint32_t S, uint32_t H) {
     const uint32_t splits = split_field & 0xffffu;
     const uint32_t groups = rows << 4;
     const uint32_t lane = threadIdx.x & 63u, p = threadIdx.x >> 6;
@@ -1791,4 +1924,25 @@ extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_kvspli
         merge_states(st, o);
     }
     store16_system(out + (size_t)t * 16u, merge_finish(st));
+    if (LSE && (t & 15u) == 0u) {
+        const uint32_t row = t >> 4, h = row % H, bs = row / H, s = bs % S, b = bs / S;
+        const Recipe rc = recipe(false);
+        const float lse2 = st.m > -1.0e30f ? st.m + __builtin_amdgcn_logf(st.den) + 4.0f + 127.0f + __builtin_amdgcn_logf(rc.conv) - rc.exp2_bias_log2
+                                           : -INFINITY;
+        store4_system(lse_out + ((size_t)b * H + h) * S + s, lse2 * 0.69314718055994531f);
+    }
+}
+
+extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_kvsplit_combine_wide(FMHA_COMBINE_PARAMS) {
+    (void)d;
+    __shared__ float part[3][10][64];
+    combine_wide<false>(part, ohat, lse, out, rows, split_field, nullptr, 1u, 1u);
+}
+
+extern "C" __global__ void __launch_bounds__(256)
+    fmha_fwd_hd128_mxfp8_v3_combine_lse(FMHA_COMBINE_PARAMS, uint32_t pad, float* lse_out, uint32_t S, uint32_t H) {
+    (void)d;
+    (void)pad;
+    __shared__ float part[3][10][64];
+    combine_wide<true>(part, ohat, lse, out, rows, split_field, lse_out, S, H);
 }

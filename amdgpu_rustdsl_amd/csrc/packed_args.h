@@ -1,0 +1,23 @@
+// packed_args.h - kernel arguments of the packed-rows attention kernel, shared by its host and device code.
+#ifndef FMHA_PACKED_ARGS_H
+#define FMHA_PACKED_ARGS_H
+
+#include <stdint.h>
+
+// `flags`: FMHA_FLAG_CAUSAL and FMHA_FLAG_V_SEQ32 as in fmha_mxfp8_args, and
+enum { kPackedF32 = 0x100u,      // partial rows in f32 (512 B) instead of fp16 (256 B)
+       kPackedWhole = 0x200u };  // the softmax reference is taken over whole 128-key tiles (else over each 64-key half)
+
+typedef struct fmha_packed_args {
+    const void *q, *k, *v, *qs, *ks, *vd;
+    void *ohat, *lse;        // partial rows and their base-2 LSE, row (b S + s) H + h of each of parts x sub splits
+    uint32_t S, SK, H, HK;
+    float softmax_scale;     // at 0x50, where the `_scaled` kernels read it
+    uint32_t gshift;         // log2(H / HK)
+    uint32_t parts, sub;     // the reference's key ranges, and how many blocks share each
+    uint32_t groups;         // B parts sub (the grid is HK x row tiles x groups)
+    uint32_t rows_total;     // B S H
+    uint32_t flags;
+} fmha_packed_args;
+
+#endif

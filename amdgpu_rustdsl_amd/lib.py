@@ -108,6 +108,9 @@ _L.fmha_mxfp8_launch_combine.argtypes = [_P(CombineArgs), _u32, _vp]
 _L.fmha_mxfp8_launch_combine_wide.argtypes = [_P(CombineArgs), _u32, _vp]
 _L.fmha_fwd_hd128_mxfp8_auto.argtypes = [_P(Params), _vp, _sz, _vp, _P(_c), _P(_c), _cp, _sz]
 _L.fmha_fwd_hd128_mxfp8_auto_noalloc.argtypes = [_P(Params), _vp, _P(_c), _P(_c), _cp, _sz]
+_L.fmha_fwd_hd128_mxfp8_auto_ws.argtypes = _L.fmha_fwd_hd128_mxfp8_auto.argtypes
+_L.fmha_mxfp8_auto_workspace_bytes.argtypes = [_P(Params)]
+_L.fmha_mxfp8_auto_workspace_bytes.restype = _sz
 _L.fmha_mxfp8_init.argtypes = [_cp, _sz]
 _L.fmha_mxfp8_version.restype = _cp
 _L.fmha_mxfp8_version.argtypes = []
@@ -121,7 +124,7 @@ _L.fmha_mxfp8_seq32_scale_bytes.restype = _sz
 EXPORTED = ["fmha_mxfp8_validate_vs128", "fmha_mxfp8_validate_t128", "fmha_mxfp8_validate_kvsplit", "fmha_mxfp8_validate_combine",
             "fmha_mxfp8_select_path", "fmha_mxfp8_uses_split_tiles", "fmha_mxfp8_fill_args", "fmha_mxfp8_workspace_bytes", "fmha_mxfp8_kv_partials", "fmha_mxfp8_launch_vs128",
             "fmha_mxfp8_launch_t128", "fmha_mxfp8_launch_t128_split_tiles", "fmha_mxfp8_launch_kvsplit", "fmha_mxfp8_launch_combine", "fmha_mxfp8_launch_combine_wide", "fmha_fwd_hd128_mxfp8_auto",
-            "fmha_fwd_hd128_mxfp8_auto_noalloc",
+            "fmha_fwd_hd128_mxfp8_auto_noalloc", "fmha_fwd_hd128_mxfp8_auto_ws", "fmha_mxfp8_auto_workspace_bytes",
             "fmha_mxfp8_init", "fmha_mxfp8_version",
             "fmha_mxfp8_quantize_rows", "fmha_mxfp8_quantize_tensor", "fmha_mxfp8_quantize_seq32", "fmha_mxfp8_seq32_scale_bytes"]
 
@@ -225,6 +228,16 @@ def _run(entry, params, *args):
 def run_auto(params, workspace=None, workspace_bytes=0, stream=None):
     """fmha_fwd_hd128_mxfp8_auto; returns Ran (path name, splits; .partials)."""
     return _run(_L.fmha_fwd_hd128_mxfp8_auto, params, workspace, workspace_bytes, stream)
+
+
+def run_auto_ws(params, workspace=None, workspace_bytes=0, stream=None):
+    """fmha_fwd_hd128_mxfp8_auto_ws: run_auto with a workspace that the full-sequence paths may use too."""
+    return _run(_L.fmha_fwd_hd128_mxfp8_auto_ws, params, workspace, workspace_bytes, stream)
+
+
+def auto_workspace_bytes(params):
+    """The workspace run_auto_ws can use for these params (one slot; 0 when it needs none)."""
+    return int(_L.fmha_mxfp8_auto_workspace_bytes(ctypes.byref(params)))
 
 
 NOALLOC_SCRATCH_BYTES = 33816576   # FMHA_NOALLOC_SCRATCH_BYTES

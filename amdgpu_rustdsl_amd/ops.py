@@ -138,13 +138,10 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
         if not float(softmax_scale) > 0.0:
             raise ValueError(f"fmha_fwd_mxfp8: softmax_scale must be positive, got {softmax_scale!r}")
         p.softmax_scale = float(softmax_scale)
-    # the workspace only matters for the KV split; size it for the split the dispatch will choose
-    want_path, want_splits = (select_path(B, H, S, SK) if path_id < 0 else (path, nsplit))
-    ws, ws_bytes = None, 0
-    if want_path == "kvsplit" and not causal:
-        # the entry's partials: the chunks, each spread over up to 8 blocks when the grid would leave CUs idle
-        parts = lib.kv_partials(B, H, S, SK, want_splits) if kv_fill else want_splits
-        ws_bytes = lib.workspace_bytes(B, H, S, parts)
+    # the workspace: the KV split's partials (the chunks, each spread over up to 8 blocks when the grid would leave CUs
+    # idle), or those of a short query range's shares
+    ws, ws_bytes = None, lib.auto_workspace_bytes(p)
+    if ws_bytes:
         # room for the entry's workspace slots (consecutive calls then write partials the previous combine did not
         # just read), unless that would take more than 512 MiB
         slotted = lib.WORKSPACE_SLOTS * ((ws_bytes + 255) // 256 * 256)
@@ -154,7 +151,7 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
         ws = buf.data_ptr()
         p.ws_turn = ctypes.pointer(turn)
     with torch.cuda.device(dev):
-        return lib.run_auto(p, ws, ws_bytes, st)
+        return lib.run_auto_ws(p, ws, ws_bytes, st)
 
 
 def alloc_scales(B, rows, H, device, fill=0):

@@ -305,6 +305,17 @@ typedef struct fmha_mxfp8_params {
 int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes,
                               void* stream, int* path_out, int* splits_out, char* err, size_t errlen);
 
+/* Extension (no counterpart in the reference): the same entry for callers whose workspace serves one stream and every
+ * shape. Same params, rules, errors and results; with path = -1 a short query range (S <= 128) over many key tiles may
+ * then use the workspace on the full-sequence paths too, and on the KV split be cut further: the query heads of a
+ * KV head are packed into one block's rows, and the key range is spread over several blocks whose f32 partials a merge
+ * kernel adds up. Every share starts from the softmax reference of the whole range's first tile, so P is quantised as
+ * the unsplit kernel does; the sums are taken in another order. Without enough workspace the path's own kernel runs.
+ * fmha_mxfp8_auto_workspace_bytes: the workspace the call can use (one slot; 0 when it needs none). */
+int fmha_fwd_hd128_mxfp8_auto_ws(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes,
+                                 void* stream, int* path_out, int* splits_out, char* err, size_t errlen);
+size_t fmha_mxfp8_auto_workspace_bytes(const fmha_mxfp8_params* p);
+
 /* Allocation-free variant of fmha_fwd_hd128_mxfp8_auto. No counterpart in the reference: it is for callers that
  * cannot allocate device memory or pass a workspace (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). The KV split's workspace is a device array of FMHA_NOALLOC_SCRATCH_BYTES inside the library
