@@ -123,13 +123,19 @@ bool use_split_tiles(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
 
 // The one-call entry also runs the vs128 path on the 128-row grid when its 256-row grid holds at most 128 blocks (half
 // of the 256 CUs or fewer): there the same shape fills twice the CUs. Causal (extension): always from 4 key tiles on,
-// so that the 128-row grid's causal q-tile pairing is available past one wave of blocks. The kernel is chosen as for
-// t128 (above). Below the split-tile threshold the 256-thread t128 kernel gives the vs128 kernel's order and bits
+// so that the 128-row grid's causal q-tile pairing is available past one wave of blocks, except square causal shapes whose
+// 256-row grid has more blocks than CUs: there the 256-row kernel with its heaviest query tiles first balances as well
+// and takes 1.5 us per 256 rows and key tile where the split-tile kernel takes 2.1 (us per call, split-tile / 256-row:
+// B1 H32 HK8 S6144 174.3 / 146.1, S4096 82.6 / 66.5, B3 H8 S3001 63.7 / 40.0, B8 H8 S2048 62.5 / 59.2; at one round of
+// blocks it loses: B1 H8 S8192 72.2 / 86.4, B2 H8 S4096 41.9 / 47.5). With many more keys than queries (chunked prefill,
+// S < SK) the split-tile order is kept: every row then averages many keys, and outputs of the two orders, though equally
+// close to float64, differ by 3 % from each other. The kernel is chosen as for t128 (above). Below the split-tile threshold the 256-thread t128 kernel gives the vs128 kernel's order and bits
 // (both take every tile whole) on twice the blocks; measured with the LUT recipe at B4H8S1024 SK256, B2H8S2048 SK384
 // and B1H8S4096 SK128: 10.4 / 12.6 / 7.7 us against 11.9 / 14.3 / 9.5 (above 128 blocks of 256 rows the vs128 kernel
 // stays ahead: B8H8S2048 SK256 25.4 against 36.4 us). The direct vs128 launcher keeps the 256-row kernel its grid names.
 bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
-    return (S + 255) / 256 * H * B <= 128 || (causal && (SK + 127) / 128 >= 4);
+    const int64_t blocks = (S + 255) / 256 * H * B;
+    return blocks <= 128 || (causal && (SK + 127) / 128 >= 4 && !(S == SK && blocks > (int64_t)cu_count()));
 }
 
 fmha_internal::ModuleCache<13> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);

@@ -1594,6 +1594,19 @@ __device__ inline void block_coords(uint32_t S, uint32_t H, uint32_t rows, uint3
     z = blockIdx.z;
 }
 
+// The causal order of the 256-row grid: the query tiles with the most keys first, so that the last blocks to start are the
+// shortest. Where the heads divide over the 8 XCDs, each XCD runs its heads' heaviest tiles together, then the next
+// ones (its own logical blocks, as block_coords deals them); else each head's tiles in descending order.
+__device__ inline void causal_coords(uint32_t S, uint32_t H, uint32_t& qt, uint32_t& head) {
+    const uint32_t gx = (S + 255u) / 256u;
+    if ((H & 7u) == 0u) {
+        const uint32_t per = H >> 3, i = (head % per) * gx + qt;
+        head = __builtin_amdgcn_readfirstlane(head - head % per + i % per);
+        qt = i / per;
+    }
+    qt = __builtin_amdgcn_readfirstlane(gx - 1u - qt);
+}
+
 // Inlined into its kernel, like everything that reads the kernel arguments: in a called (outlined) function the
 // kernarg segment pointer is not an ABI input and compiles to null. build.py rejects a code object with a call.
 // SC: the `_scaled` kernel of the pair (the softmax scale at 0x050 applied in the kernel).
@@ -1610,6 +1623,7 @@ __device__ __forceinline__ void full_kernel(uint32_t lds) {
     if constexpr (NT == 512) {
         uint32_t qt, head, z;
         block_coords(p.S, p.H, 256u, qt, head, z);
+        if (p.flags & FMHA_FLAG_CAUSAL) causal_coords(p.S, p.H, qt, head);
         if (p.vs32) {
             if (lut) attend_pingpong<true, false, true, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
             else attend_pingpong<false, false, true, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
