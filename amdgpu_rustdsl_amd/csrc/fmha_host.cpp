@@ -81,7 +81,7 @@ namespace {
 using fmha_internal::fail;
 using fmha_internal::set_err;
 
-const char* const kKernelNames[13] = {
+const char* const kKernelNames[16] = {
     "fmha_fwd_hd128_mxfp8_v3_vs128",
     "fmha_fwd_hd128_mxfp8_v3_t128",
     "fmha_fwd_hd128_mxfp8_v3_kvsplit",
@@ -99,9 +99,14 @@ const char* const kKernelNames[13] = {
     "fmha_fwd_hd128_mxfp8_v3_packed",
     "fmha_fwd_hd128_mxfp8_v3_packed_scaled",
     "fmha_fwd_hd128_mxfp8_v3_combine_lse",
+    // extension kernels: the 256-row kernel with split last blocks, and their merge
+    "fmha_fwd_hd128_mxfp8_v3_vs128_tail",
+    "fmha_fwd_hd128_mxfp8_v3_vs128_tail_scaled",
+    "fmha_fwd_hd128_mxfp8_v3_tail_combine",
 };
 enum { K_VS128 = 0, K_T128 = 1, K_KVSPLIT = 2, K_COMBINE = 3, K_VS128_SC = 4, K_T128_SC = 5, K_KVSPLIT_SC = 6, K_T128ST = 7,
-       K_T128ST_SC = 8, K_COMBINE_WIDE = 9, K_PACKED = 10, K_PACKED_SC = 11, K_COMBINE_LSE = 12 };
+       K_T128ST_SC = 8, K_COMBINE_WIDE = 9, K_PACKED = 10, K_PACKED_SC = 11, K_COMBINE_LSE = 12,
+       K_TAIL = 13, K_TAIL_SC = 14, K_TAIL_COMBINE = 15 };
 
 // The 128-row grids (t128's shapes, and vs128's half-chip and causal ones below) run on the split-tile kernel (512
 // threads) from 7 key tiles on, and on the one-wave-per-SIMD kernel (256 threads, the reference's order) below that:
@@ -138,7 +143,7 @@ bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool caus
     return blocks <= 128 || (causal && (SK + 127) / 128 >= 4 && !(S == SK && blocks > (int64_t)cu_count()));
 }
 
-fmha_internal::ModuleCache<13> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
+fmha_internal::ModuleCache<16> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
 
 int get_functions(hipFunction_t** out, char* err, size_t errlen) { return g_fmha.get(out, err, errlen); }
 
@@ -304,12 +309,38 @@ i64 packed_sub(i64 B, i64 H, i64 HK, i64 S, i64 SK, i64 parts, bool whole, bool 
     return sub;
 }
 
+// The 256-row grid with split last blocks (extension): the ranges `sub` that each block past the last whole round of CUs is
+// cut into, or 0. n blocks of t tiles on c CUs take ceil(n / c) rounds; with at most half the CUs busy in the last one,
+// cutting its blocks into up to c / (n mod c) ranges shortens that round, for a merge and the partials' bytes; the rule
+// takes the count with the least estimated time. Measured on MI355X, us per call whole / cut: B3 H8 S3001 (288 blocks
+// of 24 tiles) 81.0 / 67.3 with 4 ranges (2: 73.3, 8: 69.9), B1 H32 HK8 S2049 56.9 / 53.3, B1 H12 S6000 158.0 / 117.3,
+// B1 H9 S8192 183.8 / 139.3; where the rule keeps them whole a cut loses: 384 blocks of 24 tiles 79.8 / 83.3, 288 of 9
+// tiles 40.0 / 40.5, 320 of 16 57.0 / 57.3.
+i64 tail_sub(i64 blocks, i64 tiles) {
+    constexpr double kBlock = 6.0, kTile = 1.5, kMerge = 5.0, kBytes = 4.0e6;
+    const i64 cus = cu_count(), rem = blocks % cus;
+    if (blocks < cus || rem == 0 || tiles < 8) return 0;
+    double best = (double)tiles * kTile + kBlock - 1.0;
+    i64 sub = 0;
+    for (i64 s = 2; s <= 8 && s * rem <= cus; ++s) {
+        // the seed tile counts for one; each partial row is written and read back
+        const double c = (double)((tiles + s - 1) / s + 1) * kTile + kBlock + kMerge + (double)(rem * s * 256 * 1024) / kBytes;
+        if (c < best) {
+            best = c;
+            sub = s;
+        }
+    }
+    return sub;
+}
+size_t tail_bytes(i64 rem, i64 sub) { return (size_t)(rem * sub * 256) * 516u; }
+
 // What the one-call entry runs for a shape: the resolved path, and for the packed-rows kernel its shares.
 struct Plan {
     int path, splits;   // as the entry reports them
     i64 parts;          // KV-split partials (chunks x fill), 1 off the KV split
     i64 sub;            // packed-rows shares of each partial's range; 0: the path's own kernel
     bool whole;         // packed rows: the softmax reference over whole tiles
+    i64 tail, tail_blocks;   // 256-row grid: ranges per split last block (0: none) and how many blocks are split
     int kern;           // the path's own kernel (full-sequence paths)
     uint32_t block, gx;
 };
@@ -335,7 +366,7 @@ void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspa
     const size_t one = fmha_mxfp8_workspace_bytes(B, H, S, 1);
     const i64 fits = (i64)std::min<size_t>(workspace / one, 256);
     pl.parts = 1;
-    pl.sub = 0;
+    pl.sub = pl.tail = pl.tail_blocks = 0;
     pl.kern = -1;
     if (pl.path == FMHA_PATH_KVSPLIT) {
         i64 fill = p.kv_fill ? 1 : kv_fill(B, H, S, SK, pl.splits);
@@ -350,6 +381,12 @@ void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspa
         // a forced path keeps its kernel (and its bits)
         if (any_path && p.path < 0 && p.kv_fill == 0)
             pl.sub = packed_sub(B, H, HK, S, SK, 1, pl.whole, false, true, (i64)pl.gx * H * B, fits);
+        if (any_path && p.path < 0 && p.kv_fill == 0 && !p.causal && pl.sub == 0 && (pl.kern == K_VS128 || pl.kern == K_VS128_SC)) {
+            const i64 blocks = (i64)pl.gx * H * B;
+            pl.tail = tail_sub(blocks, (SK + 127) / 128);
+            pl.tail_blocks = pl.tail ? blocks % cu_count() : 0;
+            if (pl.tail && tail_bytes(pl.tail_blocks, pl.tail) > workspace) pl.tail = pl.tail_blocks = 0;
+        }
     }
     if (pl.sub > 0 && pl.parts * pl.sub * B * S * H * 512 >= (1LL << 32)) pl.sub = 0;   // the combines' 32-bit partial offsets
 }
@@ -608,6 +645,31 @@ static int run_packed(const fmha_mxfp8_params& p, const Plan& pl, const fmha_mxf
     return run_combine(p, ohat, lse, parts, f32, pl.path == FMHA_PATH_KVSPLIT ? nullptr : (float*)p.lse, stream, err, errlen);
 }
 
+// The 256-row kernel with split last blocks and their merge, for a plan with pl.tail > 0 (make_plan checked the workspace).
+static int run_tail(const fmha_mxfp8_params& p, const Plan& pl, const fmha_mxfp8_args& a, void* workspace, size_t workspace_bytes, void* stream,
+                    char* err, size_t errlen) {
+    const i64 blocks = (i64)pl.gx * p.H * p.B, nfull = blocks - pl.tail_blocks;
+    uint8_t* ohat = workspace_slot(p, workspace, workspace_bytes, tail_bytes(pl.tail_blocks, pl.tail));
+    uint8_t* lse = ohat + (size_t)(pl.tail_blocks * pl.tail * 256) * 512u;
+    fmha_tail_args ta;
+    ta.base = a;
+    ta.ohat = ohat;
+    ta.lse = lse;
+    ta.nfull = (uint32_t)nfull;
+    ta.ntail = (uint32_t)pl.tail_blocks;
+    ta.sub = (uint32_t)pl.tail;
+    ta.pad = 0;
+    const int rc = launch_raw(pl.kern == K_VS128_SC ? K_TAIL_SC : K_TAIL, &ta, sizeof(ta), (uint32_t)(nfull + pl.tail_blocks * pl.tail), 1, 1,
+                              512, stream, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    struct {
+        const void *ohat, *lse;
+        void *out, *lse_out;
+        uint32_t ntail, sub, nfull, S, H, pad;
+    } ca = {ohat, lse, p.o, p.lse, ta.ntail, ta.sub, ta.nfull, (uint32_t)p.S, (uint32_t)p.H, 0u};
+    return launch_raw(K_TAIL_COMBINE, &ca, sizeof(ca), (uint32_t)(pl.tail_blocks * 16), 1, 1, 256, stream, err, errlen);
+}
+
 // any_path: as in make_plan
 static int run_entry(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes, bool any_path, void* stream, int* path_out,
                      int* splits_out, char* err, size_t errlen) {
@@ -666,6 +728,7 @@ static int run_entry(const fmha_mxfp8_params* p, void* workspace, size_t workspa
             if (rc != FMHA_OK) return rc;
         }
         if (pl.sub > 0) return run_packed(*p, pl, a, workspace, workspace_bytes, stream, err, errlen);
+        if (pl.tail > 0) return run_tail(*p, pl, a, workspace, workspace_bytes, stream, err, errlen);
         const int kern = pl.kern;
         const uint32_t block = pl.block;
         uint32_t kgx = pl.gx;
@@ -723,6 +786,7 @@ size_t fmha_mxfp8_auto_workspace_bytes(const fmha_mxfp8_params* p) {
     if (pl.path != FMHA_PATH_VS128 && pl.path != FMHA_PATH_T128 && pl.path != FMHA_PATH_KVSPLIT) return 0;
     make_plan(pl, *p, p->softmax_scale != 0.0f, ~(size_t)0, true);
     if (pl.sub > 0) return fmha_mxfp8_workspace_bytes(p->B, p->H, p->S, (int)(pl.parts * pl.sub));
+    if (pl.tail > 0) return tail_bytes(pl.tail_blocks, pl.tail);
     return pl.path == FMHA_PATH_KVSPLIT ? fmha_mxfp8_workspace_bytes(p->B, p->H, p->S, (int)pl.parts) : 0;
 }
 

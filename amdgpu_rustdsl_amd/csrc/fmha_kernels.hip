@@ -111,6 +111,7 @@ struct Prm {
     uint32_t pk_rows, pk_sh;
     int32_t seed_key;
     uint32_t seed_whole;
+    int64_t tl_row;   // the 256-row kernel's split blocks: partial row of query row 0 of the block's (batch, head)
 #ifdef FMHA_TRACE
     uint64_t* trace;   // debug builds only: per (block, wave) timestamps, pointer at kernarg 0x288
     uint64_t t_entry;  // timestamp of the kernel's first instruction
@@ -944,6 +945,9 @@ struct Wave {
 
 };
 
+// Where a kernel's partial rows go (epilogue)
+enum { kRowsOfAll = 0, kRowsPacked = 1, kRowsOfBlock = 2 };
+
 // The row sum of this lane's query (the ones pattern puts it in D dword (lane / 16) % 2).
 __device__ __forceinline__ float row_sum(const v4f& lacc, uint32_t lane) { return ((lane >> 4) & 1u) ? lacc[1] : lacc[0]; }
 
@@ -1047,9 +1051,10 @@ __device__ __forceinline__ v4i merge_finish(const MergeState& st) {
 // before staging over the ring, comes after B's stores are issued. (The 256-thread kernel's waves end together:
 // there the two rounds cost more than the barrier saves.) DCH: the dims the wave writes: 0 all, 1 dims 0..63 (dc 0, 1),
 // 2 dims 64..127 (dc 2, 3; the LSE is left to the DCH 1 wave of the same rows).
-// PK: the packed-rows kernel's partials (SPLIT): row r of the wave's KV head is query r >> pk_sh of head
-// `head` + (r & (2^pk_sh - 1)).
-template <bool SPLIT, int NT, bool TAIL = false, int DCH = 0, bool PK = false>
+// PM, where the partials (SPLIT) of row r go: kRowsOfAll: row (b S + r) H + head of the split; kRowsPacked (the packed-rows
+// kernel): row r of the KV head is query r >> pk_sh of head `head` + (r & (2^pk_sh - 1)); kRowsOfBlock (the 256-row
+// kernel's split blocks): row tl_row + r.
+template <bool SPLIT, int NT, bool TAIL = false, int DCH = 0, int PM = kRowsOfAll>
 __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32_t head, uint32_t bidx, uint32_t split, const Recipe& rc,
                                          bool sync) {
     // lane-derived values recomputed here from an opaque lane id: kept from the prologue they would be live (and
@@ -1058,9 +1063,11 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
     asm volatile("" : "+s"(all));   // an opaque mask, so the lane index is computed here (see lane_addr on inline asm)
     const uint32_t lane = __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
     const uint32_t hh = lane >> 5, n = lane & 31u, row = w.row0 + n;
-    static_assert(!PK || SPLIT, "packed rows are written as partials");
-    const uint32_t nrows = PK ? p.pk_rows : p.S;
-    auto pk_prow = [&](uint32_t r) -> size_t {   // partial row of packed row r
+    static_assert(PM == kRowsOfAll || SPLIT, "only partials go elsewhere");
+    constexpr bool PK = PM != kRowsOfAll;
+    const uint32_t nrows = PM == kRowsPacked ? p.pk_rows : p.S;
+    auto pk_prow = [&](uint32_t r) -> size_t {   // partial row of row r
+        if (PM == kRowsOfBlock) return (size_t)(p.tl_row + (int64_t)r);
         return (size_t)split * p.rows_total + ((size_t)bidx * p.S + (r >> p.pk_sh)) * p.H + head + (r & ((1u << p.pk_sh) - 1u));
     };
     const float l = row_sum(w.lacc, lane);
@@ -1140,7 +1147,7 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
                     const uint32_t r = 4u * k + (lane >> 4);
                     const v4i x = lds_read16(sbase + r * kEpiRow + c16 * 16u);
                     if (w.row0 + r < p.S) {
-                        store16_system(obase + (size_t)r * ostride + c16 * 16u, x);
+                        store16_system((PK ? p.ohat + pk_prow(w.row0 + r) * 256u : obase + (size_t)r * ostride) + c16 * 16u, x);
                     }
                 }
             } else {
@@ -1174,7 +1181,7 @@ __device__ __forceinline__ void epilogue(const Prm& p, const Wave<NT>& w, uint32
                     const uint32_t r = 4u * k + (lane >> 4);
                     const v4i x = lds_read16(sbase + r * kEpiRow + c16 * 16u);
                     if (w.row0 + 16u * h + r < p.S) {
-                        store16_system(obase + (size_t)(16u * h + r) * ostride + c16 * 16u, x);
+                        store16_system((PK ? p.ohat + pk_prow(w.row0 + 16u * h + r) * 256u : obase + (size_t)(16u * h + r) * ostride) + c16 * 16u, x);
                     }
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // round h's reads are back before h + 1 writes
@@ -1267,12 +1274,12 @@ __device__ __forceinline__ void merge_halves(Wave<NT>& w, uint32_t lds) {
 // schedule, the ring and the copies are unchanged. After the loop B hands its softmax state to A through LDS and A
 // merges the two (merge_halves).
 //
-// PK (the packed-rows kernel, HV): the block's rows are packed (Prm::pk_sh), and its key range may be a later part of a
-// range whose first tile fixes the softmax reference: before its own tiles it takes that tile's row max (K seed_key,
+// PM != kRowsOfAll (the packed-rows kernel and the 256-row kernel's split blocks): the block's key range may be a later part
+// of a range whose first tile fixes the softmax reference: before its own tiles it takes that tile's row max (K seed_key,
 // through K slot 3) exactly as the whole range's first tile would, so P is quantised on the same grid wherever the
-// range is cut. seed_whole: the reference is the maximum over the tile's 128 keys (the whole-tile kernels' order),
-// else over the group's own 64 keys (the split-tile order).
-template <bool LUT, bool SPLIT, bool GB, bool VS, bool HV, bool SC, bool PK = false>
+// range is cut. HV with seed_whole: the reference is the maximum over the tile's 128 keys (the whole-tile kernels'
+// order), else over the group's own 64 keys (the split-tile order). kRowsPacked: the block's rows are packed (Prm::pk_sh).
+template <bool LUT, bool SPLIT, bool GB, bool VS, bool HV, bool SC, int PM = kRowsOfAll>
 __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds, uint32_t qtile, uint32_t head, uint32_t bidx,
                                                       uint32_t split, uint32_t key_lo, uint32_t key_hi) {
     constexpr int NT = 512;
@@ -1281,6 +1288,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
     const Recipe rc = recipe(LUT);
     // rows per block: 256, or 128 for the full-sequence split-tile kernel (the KV split's split-tile blocks keep the
     // 256-row grid and use their first 128 rows)
+    constexpr bool PK = PM == kRowsPacked, SEED = PM != kRowsOfAll;
     constexpr uint32_t RB = HV && (!SPLIT || PK) ? 128u : 256u;
     const uint32_t tblk = ((bidx * p.splits + split) * p.H + head) * ((p.S + RB - 1u) / RB) + qtile;   // trace slot
     (void)tblk;
@@ -1324,7 +1332,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         st.init_dma();
         const uint32_t ks0 = st.ks_word(key_of(0), true);
         const uint32_t ks1 = st.ks_word(key_of(1), ntiles > 1);
-        const bool seed = PK && p.seed_key >= 0;
+        const bool seed = SEED && p.seed_key >= 0;
         const uint32_t kss = seed ? st.ks_word((uint32_t)p.seed_key, true) : 0u;
         st.load_ks(key_of(2), ntiles > 2);                              // stored by V(0)
         // The first barrier needs K 0, V 0 and K 1 (read in I(0)); V 1 and K 2 are first read in I(1), so barrier 0
@@ -1364,7 +1372,9 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
                 return m;
             };
             float m = half_max(std::integral_constant<int, KB0>{});
-            if (p.seed_whole) m = fmaxf(m, half_max(std::integral_constant<int, 2 - KB0>{}));
+            if constexpr (HV) {
+                if (p.seed_whole) m = fmaxf(m, half_max(std::integral_constant<int, 2 - KB0>{}));
+            }
             rebase<LUT>(rc, m, s, w.o, w.lacc, w.bias, w.bw, w.qrm);   // (O and the row sums are zero)
             block_barrier();   // every wave has read K slot 3
         }
@@ -1444,23 +1454,23 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
     FMHA_MARK(p, tblk, 4);
     FMHA_LFLUSH(p, tblk);
     if (!HV) {
-        epilogue<SPLIT, NT, GB>(p, w, head, bidx, split, rc, true);
+        epilogue<SPLIT, NT, GB, 0, PM>(p, w, head, bidx, split, rc, true);
     } else {
         // HV: each group finishes half of every row's dims (A 0..63, B 64..127); the merge's barriers retired the ring
         merge_halves<GB>(w, lds);
         FMHA_MARK(p, tblk, 6);
-        epilogue<SPLIT, NT, false, GB ? 2 : 1, PK>(p, w, head, bidx, split, rc, false);
+        epilogue<SPLIT, NT, false, GB ? 2 : 1, PM>(p, w, head, bidx, split, rc, false);
     }
     FMHA_MARK(p, tblk, 5);
 }
 
 // The whole routine is instantiated per group (the groups place their barrier differently; one body with a
 // group-dependent branch, or two loop copies sharing a prologue, made the register allocation spill).
-template <bool LUT, bool SPLIT, bool VS, bool HV, bool SC, bool PK = false>
+template <bool LUT, bool SPLIT, bool VS, bool HV, bool SC, int PM = kRowsOfAll>
 __device__ __forceinline__ void attend_pingpong(const Prm& p, uint32_t lds, uint32_t qtile, uint32_t head, uint32_t bidx, uint32_t split,
                                 uint32_t key_lo, uint32_t key_hi) {
-    if (wave_id() >= 4u) attend_pingpong_group<LUT, SPLIT, true, VS, HV, SC, PK>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
-    else attend_pingpong_group<LUT, SPLIT, false, VS, HV, SC, PK>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
+    if (wave_id() >= 4u) attend_pingpong_group<LUT, SPLIT, true, VS, HV, SC, PM>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
+    else attend_pingpong_group<LUT, SPLIT, false, VS, HV, SC, PM>(p, lds, qtile, head, bidx, split, key_lo, key_hi);
 }
 
 // One 4-wave block of 128 rows with one wave per SIMD (_t128 under its own 256-thread contract). Nothing else runs on
@@ -1793,8 +1803,42 @@ __device__ __forceinline__ void packed_kernel(uint32_t lds) {
     const uint32_t key_lo = t0 * 128u, key_hi = min(t1 * 128u, p.SK);
     p.seed_key = p.seed_whole || t0 != lo ? (int32_t)(lo * 128u) : -1;
     const uint32_t head = hk << p.pk_sh;
-    if (p.vs32) attend_pingpong<false, true, true, true, SC, true>(p, lds, qt, head, bidx, split, key_lo, key_hi);
-    else attend_pingpong<false, true, false, true, SC, true>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+    if (p.vs32) attend_pingpong<false, true, true, true, SC, kRowsPacked>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+    else attend_pingpong<false, true, false, true, SC, kRowsPacked>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+}
+
+// The 256-row kernel with split last blocks (extension): a grid of n blocks of equal work on c CUs takes ceil(n / c) rounds, the
+// last of them on n mod c CUs. Here blocks 0 .. nfull - 1 (whole rounds) run as in the vs128 kernel, and each of the
+// ntail remaining ones is cut into `sub` key ranges, one block each, that write f32 partials (tail_combine merges them).
+// Every range starts from the reference of the first tile, so P is quantised as in the uncut block.
+template <bool SC>
+__device__ __forceinline__ void tail_kernel(uint32_t lds) {
+    Prm p = prm_from_kernarg<SC>();
+    const uint32_t nfull = ka<uint32_t>(offsetof(fmha_tail_args, nfull)), ntail = ka<uint32_t>(offsetof(fmha_tail_args, ntail));
+    const uint32_t sub = ka<uint32_t>(offsetof(fmha_tail_args, sub));
+    p.ohat = (uint8_t*)ka<uint64_t>(offsetof(fmha_tail_args, ohat));
+    p.lse = (float*)ka<uint64_t>(offsetof(fmha_tail_args, lse));
+    const uint32_t gx = (p.S + 255u) / 256u, L = blockIdx.x;
+    const bool tail = L >= nfull;
+    const uint32_t i = tail ? L - nfull : L;
+    // the whole rounds: consecutive blocks of one head on one XCD, as in block_coords
+    const uint32_t ti = tail ? i % ntail : 0u, part = tail ? i / ntail : 0u;
+    const uint32_t l = tail ? nfull + ti : ((nfull & 7u) == 0u ? (i & 7u) * (nfull >> 3) + (i >> 3) : i);
+    const uint32_t qt = __builtin_amdgcn_readfirstlane(l % gx), bh = l / gx;
+    const uint32_t head = __builtin_amdgcn_readfirstlane(bh % p.H), z = __builtin_amdgcn_readfirstlane(bh / p.H);
+    if (!tail) {
+        if (p.vs32) attend_pingpong<false, false, true, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
+        else attend_pingpong<false, false, false, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
+        return;
+    }
+    const uint32_t ntiles = (p.SK + 127u) / 128u, per = (ntiles + sub - 1u) / sub;
+    const uint32_t t0 = min(ntiles, part * per), t1 = min(ntiles, t0 + per);
+    const uint32_t key_lo = t0 * 128u, key_hi = min(t1 * 128u, p.SK);
+    p.seed_key = t0 != 0u ? 0 : -1;
+    p.f32_partials = 1u;
+    p.tl_row = (int64_t)(part * ntail + ti) * 256 - (int64_t)qt * 256;
+    if (p.vs32) attend_pingpong<false, true, true, false, SC, kRowsOfBlock>(p, lds, qt, head, z, 0, key_lo, key_hi);
+    else attend_pingpong<false, true, false, false, SC, kRowsOfBlock>(p, lds, qt, head, z, 0, key_lo, key_hi);
 }
 
 }  // namespace
@@ -1868,6 +1912,19 @@ extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_pac
     packed_kernel<true>(smem_base);
 }
 
+// Extension kernels: the 256-row kernel with split last blocks, fmha_tail_args.
+extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_vs128_tail(fmha_tail_args a) {
+    FMHA_LDS_BASE(smem);
+    (void)a;
+    tail_kernel<false>(smem_base);
+}
+
+extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_vs128_tail_scaled(fmha_tail_args a) {
+    FMHA_LDS_BASE(smem);
+    (void)a;
+    tail_kernel<true>(smem_base);
+}
+
 // epilogue.rs:89-167 / io.rs:164-185: thread t -> 8 consecutive outputs of row t >> 4 (tail threads redo the last group)
 // The combines take the 36-byte layout (fmha_mxfp8_combine_args: three pointers, then rows_total, d and the split
 // field at 0x18, 0x1C, 0x20) as scalar parameters, which lay out the same bytes: as scalars the nine dwords are preloaded
@@ -1894,14 +1951,37 @@ extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_kvspli
     store16_system(out + (size_t)t * 16u, merge_finish(st));
 }
 
+// The natural-log LSE of a merged row, which the full-sequence paths write themselves when they are not split: log2 l -
+// 2048 (hi + lo) is the merged base-2 LSE plus 4 (the partials carry l / 16), and the constants are those of the
+// epilogue's LSE output (the lazy recipe).
+__device__ __forceinline__ float merged_lse(const MergeState& st) {
+    const Recipe rc = recipe(false);
+    const float lse2 = st.m > -1.0e30f ? st.m + __builtin_amdgcn_logf(st.den) + 4.0f + 127.0f + __builtin_amdgcn_logf(rc.conv) - rc.exp2_bias_log2
+                                       : -INFINITY;
+    return lse2 * 0.69314718055994531f;
+}
+
+// The merge of the 256-row kernel's split blocks: thread t takes 8 outputs of row (t >> 4) & 255 of block nfull + (t >> 12).
+extern "C" __global__ void __launch_bounds__(256) fmha_fwd_hd128_mxfp8_v3_tail_combine(const uint8_t* ohat, const float* lse, uint8_t* out,
+                                                                                       float* lse_out, uint32_t ntail, uint32_t sub, uint32_t nfull,
+                                                                                       uint32_t S, uint32_t H) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;   // the grid is ntail x 16 blocks
+    MergeState st;
+    merge_init(st);
+    merge_splits<true>(lse, ohat, ntail * 256u, 0u, sub, t, st);
+    const uint32_t gx = (S + 255u) / 256u, l = nfull + (t >> 12), bh = l / gx;
+    const uint32_t row = (l % gx) * 256u + ((t >> 4) & 255u), head = bh % H, b = bh / H;
+    if (row >= S) return;
+    store16_system(out + (((size_t)b * S + row) * H + head) * 256u + (t & 15u) * 16u, merge_finish(st));
+    if (lse_out && (t & 15u) == 0u) store4_system(lse_out + ((size_t)b * H + head) * S + row, merged_lse(st));
+}
+
 // Extension (no counterpart in the reference): the same merge for many splits, with the splits spread over the block's
 // 4 waves. Lane l of every wave takes group 64 blockIdx.x + l (outputs 8 (g & 15) .. +7 of row g >> 4, tail lanes redo
 // the last group); wave p merges the p-th quarter of the splits (ceil(splits / 4) each, in order), and wave 0 merges
 // the quarters in order through LDS. With the reference kernel's layout one thread walks every split of its group in
 // turn: at 32 splits that is 4 dependent rounds of loads on 64 groups per block (13.7 us at 1024 rows on MI355X).
-// LSE: also the natural-log LSE [B, H, S] of each row, which the full-sequence paths write themselves when they are not
-// split: log2 l - 2048 (hi + lo) is the merged base-2 LSE plus 4 (the partials carry l / 16), and the constants are
-// those of the epilogue's LSE output (the lazy recipe).
+// LSE: also the natural-log LSE [B, H, S] of each row (merged_lse).
 template <bool LSE>
 __device__ __forceinline__ void combine_wide(float (&part)[3][10][64], const uint8_t* ohat, const float* lse, uint8_t* out, uint32_t rows,
                                              uint32_t split_field, float* lse_out, uint32_t S, uint32_t H) {
@@ -1940,10 +2020,7 @@ __device__ __forceinline__ void combine_wide(float (&part)[3][10][64], const uin
     store16_system(out + (size_t)t * 16u, merge_finish(st));
     if (LSE && (t & 15u) == 0u) {
         const uint32_t row = t >> 4, h = row % H, bs = row / H, s = bs % S, b = bs / S;
-        const Recipe rc = recipe(false);
-        const float lse2 = st.m > -1.0e30f ? st.m + __builtin_amdgcn_logf(st.den) + 4.0f + 127.0f + __builtin_amdgcn_logf(rc.conv) - rc.exp2_bias_log2
-                                           : -INFINITY;
-        store4_system(lse_out + ((size_t)b * H + h) * S + s, lse2 * 0.69314718055994531f);
+        store4_system(lse_out + ((size_t)b * H + h) * S + s, merged_lse(st));
     }
 }
 

@@ -1,4 +1,5 @@
-// packed_args.h - kernel arguments of the packed-rows attention kernel, shared by its host and device code.
+// packed_args.h - kernel arguments of the packed-rows kernel and of the 256-row kernel with split last blocks, shared by
+// host and device code. Include fmha_mxfp8.h first.
 #ifndef FMHA_PACKED_ARGS_H
 #define FMHA_PACKED_ARGS_H
 
@@ -19,5 +20,12 @@ typedef struct fmha_packed_args {
     uint32_t rows_total;     // B S H
     uint32_t flags;
 } fmha_packed_args;
+
+typedef struct fmha_tail_args {
+    fmha_mxfp8_args base;
+    void *ohat, *lse;        // f32 partial rows and base-2 LSE, row (range x ntail + block) x 256 + row of the block
+    uint32_t nfull, ntail;   // blocks that run whole, blocks cut into `sub` ranges
+    uint32_t sub, pad;
+} fmha_tail_args;
 
 #endif
