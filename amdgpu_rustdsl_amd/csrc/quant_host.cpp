@@ -50,20 +50,29 @@ struct QuantSeq32Args {
     void* scale;
     uint32_t B, SK, HK, nblk;
 };
+struct QuantQkvArgs {
+    QuantRowsArgs q, k;
+    QuantTensorArgs vt;
+    QuantSeq32Args vs;
+    void *q_slack, *k_slack;
+    uint32_t q_slack_words, k_slack_words;
+    uint32_t gq, gk, gv, seq32;
+};
+static_assert(sizeof(QuantQkvArgs) == 192, "qkv kernarg");
 static_assert(sizeof(QuantRowsArgs) == 40, "rows kernarg");
 static_assert(sizeof(QuantTensorArgs) == 32, "tensor kernarg");
 static_assert(sizeof(QuantSeq32Args) == 40, "seq32 kernarg");
 
-const char* const kQuantNames[4] = {
-    "fmha_mxfp8_quant_rows", "fmha_mxfp8_quant_amax", "fmha_mxfp8_quant_tensor", "fmha_mxfp8_quant_seq32",
+const char* const kQuantNames[5] = {
+    "fmha_mxfp8_quant_rows", "fmha_mxfp8_quant_amax", "fmha_mxfp8_quant_tensor", "fmha_mxfp8_quant_seq32", "fmha_mxfp8_quant_qkv",
 };
-enum { Q_ROWS = 0, Q_AMAX = 1, Q_TENSOR = 2, Q_SEQ32 = 3 };
+enum { Q_ROWS = 0, Q_AMAX = 1, Q_TENSOR = 2, Q_SEQ32 = 3, Q_QKV = 4 };
 // quant_kernels.hip: the amax pass runs exactly 512 workgroups and leaves one partial maximum each in descale words
 // [512, 1024); the descale buffer therefore spans 4096 bytes, the size the FMHA requires of it anyway.
 constexpr uint32_t kAmaxGroups = 512;
 constexpr uint64_t kDescaleBytes = 4096;
 
-fmha_internal::ModuleCache<4> g_quant(mxfp8_quant_hsaco_begin, mxfp8_quant_hsaco_end, kQuantNames);
+fmha_internal::ModuleCache<5> g_quant(mxfp8_quant_hsaco_begin, mxfp8_quant_hsaco_end, kQuantNames);
 
 bool aligned(const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 
@@ -74,12 +83,10 @@ uint32_t stride_grid(uint64_t chunks) {
     return (uint32_t)(g < 1 ? 1 : g > 1024 ? 1024 : g);
 }
 
-}  // namespace
+uint32_t rows_groups(int64_t rows) { return (uint32_t)((rows + 63) / 64); }   // 64 rows per workgroup
 
-extern "C" {
-
-int fmha_mxfp8_quantize_rows(const void* x, void* q, void* scale, int64_t rows, float mul, uint64_t bytes_x, uint64_t bytes_q,
-                             uint64_t bytes_scale, void* stream, char* err, size_t errlen) {
+int check_rows(const void* x, const void* q, const void* scale, int64_t rows, uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_scale,
+               char* err, size_t errlen) {
     if (rows < 1 || rows > (int64_t)0xFFFFFFFF * 64) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "rows outside [1, 2^38)");
     if (!x || !q || !scale) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "null pointer");
     if (!aligned(x, 16) || !aligned(q, 8) || !aligned(scale, 4))
@@ -88,12 +95,11 @@ int fmha_mxfp8_quantize_rows(const void* x, void* q, void* scale, int64_t rows, 
     if (bytes_x < r * 256) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "x: buffer smaller than rows * 256 bytes");
     if (bytes_q < r * 128) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "q: buffer smaller than rows * 128 bytes");
     if (bytes_scale < r * 4) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "scale: buffer smaller than rows * 4 bytes");
-    QuantRowsArgs a = {x, q, scale, r, mul, 0u};
-    return g_quant.launch(Q_ROWS, &a, sizeof(a), (uint32_t)((r + 63) / 64), 1, 1, 256, stream, err, errlen);   // 64 rows per workgroup
+    return FMHA_OK;
 }
 
-int fmha_mxfp8_quantize_tensor(const void* x, void* q, void* descale, int64_t n, uint64_t bytes_x, uint64_t bytes_q,
-                               uint64_t bytes_descale, void* stream, char* err, size_t errlen) {
+int check_tensor(const void* x, const void* q, const void* descale, int64_t n, uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_descale,
+                 char* err, size_t errlen) {
     if (n < 8 || n % 8 != 0) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "n must be a positive multiple of 8");
     if (!x || !q || !descale) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "null pointer");
     if (!aligned(x, 16) || !aligned(q, 8) || !aligned(descale, 4))
@@ -102,33 +108,98 @@ int fmha_mxfp8_quantize_tensor(const void* x, void* q, void* descale, int64_t n,
     if (bytes_x < un * 2) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "x: buffer smaller than n * 2 bytes");
     if (bytes_q < un) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "q: buffer smaller than n bytes");
     if (bytes_descale < kDescaleBytes) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "descale: buffer smaller than 4096 bytes");
-    QuantTensorArgs a = {x, q, descale, un};
-    int rc = g_quant.launch(Q_AMAX, &a, sizeof(a), kAmaxGroups, 1, 1, 256, stream, err, errlen);
-    if (rc == FMHA_OK) rc = g_quant.launch(Q_TENSOR, &a, sizeof(a), stride_grid(un / 8), 1, 1, 256, stream, err, errlen);
-    return rc;
+    return FMHA_OK;
 }
 
-size_t fmha_mxfp8_seq32_scale_bytes(int64_t B, int64_t SK, int64_t HK) {
+size_t seq32_bytes(int64_t B, int64_t SK, int64_t HK) {
     if (B < 1 || SK < 1 || HK < 1) return 0;
     return (size_t)((uint64_t)B * (uint64_t)((SK + 31) / 32) * (uint64_t)HK * 128u);
 }
 
-int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, int32_t SK, int32_t HK, uint64_t bytes_x,
-                              uint64_t bytes_q, uint64_t bytes_scale, void* stream, char* err, size_t errlen) {
+// one wave per 32-key tile, four to a workgroup
+uint64_t seq32_tiles(int64_t B, int64_t SK, int64_t HK) { return (uint64_t)B * (uint64_t)((SK + 31) / 32) * (uint64_t)HK; }
+uint32_t seq32_groups(int64_t B, int64_t SK, int64_t HK) { return (uint32_t)((seq32_tiles(B, SK, HK) + 3) / 4); }
+
+int check_seq32(const void* x, const void* q, const void* scale, int32_t B, int32_t SK, int32_t HK, uint64_t bytes_x, uint64_t bytes_q,
+                uint64_t bytes_scale, char* err, size_t errlen) {
     if (B < 1 || SK < 1 || HK < 1) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "B, SK, HK must be >= 1");
     if (!x || !q || !scale) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "null pointer");
     if (!aligned(x, 16) || !aligned(q, 8) || !aligned(scale, 8))
         return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "x needs 16-byte, q and scale 8-byte alignment");
     const uint64_t elems = (uint64_t)B * (uint64_t)SK * (uint64_t)HK * 128u;
-    const uint32_t nblk = (uint32_t)((SK + 31) / 32);
     if (bytes_x < elems * 2) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "x: buffer smaller than B*SK*HK*256 bytes");
     if (bytes_q < elems) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "q: buffer smaller than B*SK*HK*128 bytes");
-    if (bytes_scale < fmha_mxfp8_seq32_scale_bytes(B, SK, HK))
+    if (bytes_scale < seq32_bytes(B, SK, HK))
         return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "scale: buffer smaller than B*ceil(SK/32)*HK*128 bytes");
-    const uint64_t tiles = (uint64_t)B * nblk * (uint64_t)HK;   // one wave each, four to a workgroup
-    if ((tiles + 3) / 4 > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
-    QuantSeq32Args a = {x, q, scale, (uint32_t)B, (uint32_t)SK, (uint32_t)HK, nblk};
-    return g_quant.launch(Q_SEQ32, &a, sizeof(a), (uint32_t)((tiles + 3) / 4), 1, 1, 256, stream, err, errlen);
+    if ((seq32_tiles(B, SK, HK) + 3) / 4 > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
+    return FMHA_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int fmha_mxfp8_quantize_rows(const void* x, void* q, void* scale, int64_t rows, float mul, uint64_t bytes_x, uint64_t bytes_q,
+                             uint64_t bytes_scale, void* stream, char* err, size_t errlen) {
+    const int rc = check_rows(x, q, scale, rows, bytes_x, bytes_q, bytes_scale, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    QuantRowsArgs a = {x, q, scale, (uint64_t)rows, mul, 0u};
+    return g_quant.launch(Q_ROWS, &a, sizeof(a), rows_groups(rows), 1, 1, 256, stream, err, errlen);
+}
+
+int fmha_mxfp8_quantize_tensor(const void* x, void* q, void* descale, int64_t n, uint64_t bytes_x, uint64_t bytes_q,
+                               uint64_t bytes_descale, void* stream, char* err, size_t errlen) {
+    int rc = check_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    QuantTensorArgs a = {x, q, descale, (uint64_t)n};
+    rc = g_quant.launch(Q_AMAX, &a, sizeof(a), kAmaxGroups, 1, 1, 256, stream, err, errlen);
+    if (rc == FMHA_OK) rc = g_quant.launch(Q_TENSOR, &a, sizeof(a), stride_grid((uint64_t)n / 8), 1, 1, 256, stream, err, errlen);
+    return rc;
+}
+
+size_t fmha_mxfp8_seq32_scale_bytes(int64_t B, int64_t SK, int64_t HK) { return seq32_bytes(B, SK, HK); }
+
+int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, int32_t SK, int32_t HK, uint64_t bytes_x,
+                              uint64_t bytes_q, uint64_t bytes_scale, void* stream, char* err, size_t errlen) {
+    const int rc = check_seq32(x, q, scale, B, SK, HK, bytes_x, bytes_q, bytes_scale, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    QuantSeq32Args a = {x, q, scale, (uint32_t)B, (uint32_t)SK, (uint32_t)HK, (uint32_t)((SK + 31) / 32)};
+    return g_quant.launch(Q_SEQ32, &a, sizeof(a), seq32_groups(B, SK, HK), 1, 1, 256, stream, err, errlen);
+}
+
+int fmha_mxfp8_quantize_qkv(const fmha_mxfp8_qkv_params* p, void* stream, char* err, size_t errlen) {
+    if (!p) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "null params");
+    if (p->B < 1 || p->S < 1 || p->H < 1 || p->SK < 1 || p->HK < 1)
+        return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "B, S, H, SK, HK must be >= 1");
+    const int64_t rq = (int64_t)p->B * p->S * p->H, rk = (int64_t)p->B * p->SK * p->HK;
+    int rc = check_rows(p->q, p->q8, p->q_scale, rq, p->bytes_q, p->bytes_q8, p->bytes_q_scale, err, errlen);
+    if (rc == FMHA_OK) rc = check_rows(p->k, p->k8, p->k_scale, rk, p->bytes_k, p->bytes_k8, p->bytes_k_scale, err, errlen);
+    if (rc == FMHA_OK)
+        rc = p->v_seq32 ? check_seq32(p->v, p->v8, p->v_scale, p->B, p->SK, p->HK, p->bytes_v, p->bytes_v8, p->bytes_v_scale, err, errlen)
+                        : check_tensor(p->v, p->v8, p->v_scale, rk * 128, p->bytes_v, p->bytes_v8, p->bytes_v_scale, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    const uint64_t qsl = (p->bytes_q_scale - (uint64_t)rq * 4) / 4, ksl = (p->bytes_k_scale - (uint64_t)rk * 4) / 4;
+    if (qsl > 0xFFFFFFFFull || ksl > 0xFFFFFFFFull) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "scale slack too large");
+    QuantQkvArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.q = {p->q, p->q8, p->q_scale, (uint64_t)rq, p->q_mul, 0u};
+    a.k = {p->k, p->k8, p->k_scale, (uint64_t)rk, 1.0f, 0u};
+    a.vt = {p->v, p->v8, p->v_scale, (uint64_t)rk * 128};
+    a.vs = {p->v, p->v8, p->v_scale, (uint32_t)p->B, (uint32_t)p->SK, (uint32_t)p->HK, (uint32_t)((p->SK + 31) / 32)};
+    a.q_slack = (char*)p->q_scale + rq * 4;
+    a.k_slack = (char*)p->k_scale + rk * 4;
+    a.q_slack_words = (uint32_t)qsl;
+    a.k_slack_words = (uint32_t)ksl;
+    a.gq = rows_groups(rq);
+    a.gk = rows_groups(rk);
+    a.gv = p->v_seq32 ? seq32_groups(p->B, p->SK, p->HK) : kAmaxGroups;
+    a.seq32 = p->v_seq32 ? 1u : 0u;
+    const uint64_t grid = (uint64_t)a.gq + a.gk + a.gv + (qsl + 1023) / 1024 + (ksl + 1023) / 1024;
+    if (grid > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensors too large");
+    rc = g_quant.launch(Q_QKV, &a, sizeof(a), (uint32_t)grid, 1, 1, 256, stream, err, errlen);
+    if (rc == FMHA_OK && !p->v_seq32)
+        rc = g_quant.launch(Q_TENSOR, &a.vt, sizeof(a.vt), stride_grid((uint64_t)rk * 16), 1, 1, 256, stream, err, errlen);
+    return rc;
 }
 
 }  // extern "C"

@@ -100,10 +100,10 @@ struct QuantSeq32Args {
 // (64 bytes in flight per lane). Lane 0 of a row writes the row's 4 scale bytes as one word.
 constexpr uint32_t kRowsPerGroup = 64;
 
-extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_rows(QuantRowsArgs a) {
+__device__ __forceinline__ void quant_rows_group(const QuantRowsArgs& a, uint32_t group) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t c = threadIdx.x & 15u;   // 8-element chunk of the row
-    const uint64_t row0 = (uint64_t)blockIdx.x * kRowsPerGroup + (threadIdx.x >> 4);
+    const uint64_t row0 = (uint64_t)group * kRowsPerGroup + (threadIdx.x >> 4);
     u32x4 w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -137,16 +137,17 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_rows(QuantRow
     }
 }
 
+extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_rows(QuantRowsArgs a) { quant_rows_group(a, blockIdx.x); }
+
 // Tensor scale, pass 1: kQuantAmaxGroups workgroups stride over the tensor; workgroup g stores its maximum |x| into
 // descale[kQuantPartial + g] (plain stores: every slot is rewritten by every call, so nothing needs clearing and no
 // two workgroups touch one address). NaN elements are skipped (fmaxf), as std::max skips them in the generator's
 // running maximum.
-extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_amax(QuantTensorArgs a) {
-    __shared__ float part[4];
+__device__ __forceinline__ void quant_amax_group(const QuantTensorArgs& a, uint32_t group, float (&part)[4]) {
     const uint64_t nchunk = a.n / 8u;
-    const uint64_t stride = (uint64_t)gridDim.x * 256u;
+    const uint64_t stride = (uint64_t)kQuantAmaxGroups * 256u;
     float m = 0.0f;
-    uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    uint64_t i = (uint64_t)group * 256u + threadIdx.x;
     for (; i + 3 * stride < nchunk; i += 4 * stride) {   // four 16-byte loads in flight per lane
         u32x4 w[4];
 #pragma unroll
@@ -162,7 +163,12 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_amax(QuantTen
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) a.descale[kQuantPartial + blockIdx.x] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+    if (threadIdx.x == 0) a.descale[kQuantPartial + group] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+}
+
+extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_amax(QuantTensorArgs a) {
+    __shared__ float part[4];
+    quant_amax_group(a, blockIdx.x, part);
 }
 
 // Tensor scale, pass 2: every workgroup reduces the kQuantAmaxGroups partial maxima, then d = amax / 448 and
@@ -225,7 +231,9 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_tensor(QuantT
             if (c < nchunk) store8_system(a.q + c * 8u, out);
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.descale[0] = d;
+    // descale[0] = d, and zeros up to the partial maxima (the buffer's contents do not depend on what it held)
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < kQuantPartial; i += 256u) a.descale[i] = i == 0u ? d : 0.0f;
 }
 
 // Sequence blocks: one wave per tile of 32 keys x 128 columns of one (b, kv head). Lane l takes columns 8 (l & 15) .. +7 of
@@ -234,9 +242,9 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_tensor(QuantT
 // l ^ 48; each lane writes its eight 8-byte pieces, lanes 0..15 the 128 scale bytes. The heads of one 32-key block are
 // consecutive waves, so a workgroup reads up to 1 KiB of each key's row. Rows past a ragged last block (SK % 32 != 0)
 // re-read its last key, which changes no maximum, and are not stored.
-extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_seq32(QuantSeq32Args a) {
+__device__ __forceinline__ void quant_seq32_group(const QuantSeq32Args& a, uint32_t group) {
     const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, r0 = lane >> 4;
-    uint64_t t = (uint64_t)blockIdx.x * 4u + (threadIdx.x >> 6);
+    uint64_t t = (uint64_t)group * 4u + (threadIdx.x >> 6);
     const uint32_t hk = (uint32_t)(t % a.HK);
     t /= a.HK;
     const uint32_t blk = (uint32_t)(t % a.nblk);
@@ -284,5 +292,46 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_seq32(QuantSe
         sc[0] = e[0] | (e[1] << 8) | (e[2] << 16) | (e[3] << 24);
         sc[1] = e[4] | (e[5] << 8) | (e[6] << 16) | (e[7] << 24);
         *reinterpret_cast<u32x2*>(a.scale + (((uint64_t)b * a.nblk + blk) * a.HK + hk) * 128u + c * 8u) = sc;
+    }
+}
+
+extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_seq32(QuantSeq32Args a) { quant_seq32_group(a, blockIdx.x); }
+
+// Q, K and V of one attention layer in one launch: workgroups [0, gq) quantise Q's rows, [gq, gq + gk) K's, the next gv
+// V (seq32 tiles, or the kQuantAmaxGroups of the tensor scale's first pass), and the rest clear the slack behind the two
+// scale tensors (whole dwords, 4 KiB per workgroup). Every workgroup is one of the kernels above, so the bytes are
+// theirs. Bound by HBM and, at small layers, by the launch: at B2 H8 S2048 (8.4 MB each) the three separate launches and
+// the two fills took 5.8 + 5.8 + 3.8 + 2 x 2.1 us with a gap behind each; this one takes 10.2.
+struct QuantQkvArgs {
+    QuantRowsArgs q, k;
+    QuantTensorArgs vt;
+    QuantSeq32Args vs;
+    uint32_t* q_slack;
+    uint32_t* k_slack;
+    uint32_t q_slack_words, k_slack_words;
+    uint32_t gq, gk, gv, seq32;
+};
+
+extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_qkv(QuantQkvArgs a) {
+    __shared__ float part[4];
+    uint32_t g = blockIdx.x;
+    if (g < a.gq) return quant_rows_group(a.q, g);
+    g -= a.gq;
+    if (g < a.gk) return quant_rows_group(a.k, g);
+    g -= a.gk;
+    if (g < a.gv) {
+        if (a.seq32) quant_seq32_group(a.vs, g);
+        else quant_amax_group(a.vt, g, part);
+        return;
+    }
+    g -= a.gv;
+    const uint32_t qg = (a.q_slack_words + 1023u) >> 10;
+    uint32_t* dst = g < qg ? a.q_slack : a.k_slack;
+    const uint32_t n = g < qg ? a.q_slack_words : a.k_slack_words;
+    if (g >= qg) g -= qg;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t w = g * 1024u + i * 256u + threadIdx.x;
+        if (w < n) dst[w] = 0u;
     }
 }

@@ -69,6 +69,14 @@ class CombineArgs(ctypes.Structure):
     _fields_ = [("ptr_ohat", _vp), ("ptr_lse", _vp), ("ptr_out", _vp), ("rows_total", _u32), ("d", _u32), ("splits", _u32)]
 
 
+class QkvParams(ctypes.Structure):
+    """fmha_mxfp8_qkv_params (include/mxfp8_quant.h)."""
+    _fields_ = [(n, _vp) for n in ("q", "k", "v", "q8", "k8", "v8", "q_scale", "k_scale", "v_scale")] + \
+               [(n, _u64) for n in ("bytes_q", "bytes_k", "bytes_v", "bytes_q8", "bytes_k8", "bytes_v8", "bytes_q_scale",
+                                    "bytes_k_scale", "bytes_v_scale")] + \
+               [(n, ctypes.c_int32) for n in ("B", "S", "H", "SK", "HK", "v_seq32")] + [("q_mul", ctypes.c_float), ("pad", ctypes.c_int32)]
+
+
 class BufferSizes(ctypes.Structure):
     _fields_ = [(n, _u64) for n in ("ptr_q", "ptr_k", "ptr_v", "ptr_o", "ptr_q_descale", "ptr_k_descale", "ptr_v_descale",
                                     "ptr_ohat", "ptr_lse")]
@@ -118,6 +126,7 @@ _L.fmha_mxfp8_version.argtypes = []
 _L.fmha_mxfp8_quantize_rows.argtypes = [_vp, _vp, _vp, _i64, ctypes.c_float, _u64, _u64, _u64, _vp, _cp, _sz]
 _L.fmha_mxfp8_quantize_tensor.argtypes = [_vp, _vp, _vp, _i64, _u64, _u64, _u64, _vp, _cp, _sz]
 _L.fmha_mxfp8_quantize_seq32.argtypes = [_vp, _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _u64, _u64, _u64, _vp, _cp, _sz]
+_L.fmha_mxfp8_quantize_qkv.argtypes = [_P(QkvParams), _vp, _cp, _sz]
 _L.fmha_mxfp8_seq32_scale_bytes.argtypes = [_i64, _i64, _i64]
 _L.fmha_mxfp8_seq32_scale_bytes.restype = _sz
 
@@ -126,7 +135,7 @@ EXPORTED = ["fmha_mxfp8_validate_vs128", "fmha_mxfp8_validate_t128", "fmha_mxfp8
             "fmha_mxfp8_launch_t128", "fmha_mxfp8_launch_t128_split_tiles", "fmha_mxfp8_launch_kvsplit", "fmha_mxfp8_launch_combine", "fmha_mxfp8_launch_combine_wide", "fmha_fwd_hd128_mxfp8_auto",
             "fmha_fwd_hd128_mxfp8_auto_noalloc", "fmha_fwd_hd128_mxfp8_auto_ws", "fmha_mxfp8_auto_workspace_bytes",
             "fmha_mxfp8_init", "fmha_mxfp8_version",
-            "fmha_mxfp8_quantize_rows", "fmha_mxfp8_quantize_tensor", "fmha_mxfp8_quantize_seq32", "fmha_mxfp8_seq32_scale_bytes"]
+            "fmha_mxfp8_quantize_rows", "fmha_mxfp8_quantize_tensor", "fmha_mxfp8_quantize_seq32", "fmha_mxfp8_quantize_qkv", "fmha_mxfp8_seq32_scale_bytes"]
 
 raw = _L
 
@@ -261,6 +270,11 @@ def quantize_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, stream=No
 def quantize_seq32(x, q, scale, B, SK, HK, bytes_x, bytes_q, bytes_scale, stream=None):
     buf = _errbuf()
     check(_L.fmha_mxfp8_quantize_seq32(x, q, scale, B, SK, HK, bytes_x, bytes_q, bytes_scale, stream, buf, 512), buf)
+
+
+def quantize_qkv(params, stream=None):
+    buf = _errbuf()
+    check(_L.fmha_mxfp8_quantize_qkv(ctypes.byref(params), stream, buf, 512), buf)
 
 
 def seq32_scale_bytes(B, SK, HK):

@@ -198,7 +198,7 @@ def quantize_v(x, stream=None):
     argument). x may have any shape whose element count is a multiple of 8. Runs fmha_mxfp8_quantize_tensor."""
     xb = _bf16(x, "x", rows=False)
     q = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    vs = torch.zeros(1024, dtype=torch.float32, device=x.device)
+    vs = torch.empty(1024, dtype=torch.float32, device=x.device)   # written whole: d, zeros, the partial maxima
     with torch.cuda.device(x.device):
         lib.quantize_tensor(xb.data_ptr(), q.data_ptr(), vs.data_ptr(), xb.numel(), _cap(xb), _cap(q), _cap(vs), _stream(x.device, stream))
     return q, vs
@@ -219,6 +219,35 @@ def quantize_v_seq32(x, stream=None):
     return q, sc
 
 
+def _quantize_qkv(q, k, v, mul, seq32, stream):
+    """quantize_mxfp8 of q (with ``mul``) and k, and quantize_v or quantize_v_seq32 of v, as one call: the same bytes in
+    one launch (two with the tensor scale), the slack behind the scales cleared by it."""
+    B, S, H, _ = q.shape
+    _, SK, HK, _ = k.shape
+    if not (q.device == k.device == v.device):   # each tensor on its own device
+        qs, ks = alloc_scales(B, S, H, q.device), alloc_scales(B, SK, HK, k.device)
+        q8, k8 = quantize_mxfp8(q, qs, mul=mul, stream=stream), quantize_mxfp8(k, ks, stream=stream)
+        v8, vs = (quantize_v_seq32 if seq32 else quantize_v)(v, stream=stream)
+        return q8, k8, v8, qs, ks, vs
+    for t, name in ((k, "k"), (v, "v")):
+        if tuple(t.shape) != (B, SK, HK, D):
+            raise ValueError(f"{name}: expected shape {(B, SK, HK, D)}, got {tuple(t.shape)}")
+    qb, kb, vb = _bf16(q, "x"), _bf16(k, "x"), _bf16(v, "x")
+    dev = q.device
+    empty = lambda n: torch.empty(n, dtype=torch.uint8, device=dev)   # noqa: E731
+    nq, nk = B * S * H, B * SK * HK
+    q8, k8, v8 = empty(nq * D), empty(nk * D), empty(nk * D)
+    qs, ks = empty(nq * 4 + 640 * H * 4), empty(nk * 4 + 640 * HK * 4)   # alloc_scales' sizes
+    vs = empty(B * ((SK + 31) // 32) * HK * D) if seq32 else torch.empty(1024, dtype=torch.float32, device=dev)
+    p = lib.QkvParams(qb.data_ptr(), kb.data_ptr(), vb.data_ptr(), q8.data_ptr(), k8.data_ptr(), v8.data_ptr(), qs.data_ptr(),
+                      ks.data_ptr(), vs.data_ptr(), _cap(qb), _cap(kb), _cap(vb), nq * D, nk * D, nk * D, qs.numel(), ks.numel(),
+                      vs.numel() * vs.element_size(), B, S, H, SK, HK, int(seq32), mul, 0)
+    with torch.cuda.device(dev):
+        lib.quantize_qkv(p, _stream(dev, stream))
+    return (q8.view(B, S, H, D), k8.view(B, SK, HK, D), v8.view(B, SK, HK, D), qs[:nq * 4].view(B, S, H, 4), ks[:nk * 4].view(B, SK, HK, 4),
+            vs.view(B, (SK + 31) // 32, HK, D) if seq32 else vs)
+
+
 LOG2E_OVER_SQRT_D = 1.4426950408889634 / math.sqrt(D)
 
 
@@ -233,16 +262,9 @@ def fmha_fwd_bf16_via_mxfp8(q, k, v, out=None, *, softmax_scale=None, causal=Fal
     _, SK, HK, _ = k.shape
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
     mul = 1.0 if scale_in_kernel else (LOG2E_OVER_SQRT_D if softmax_scale is None else 1.4426950408889634 * scale)
-    qs = alloc_scales(B, S, H, q.device)
-    ks = alloc_scales(B, SK, HK, k.device)
-    q8 = quantize_mxfp8(q, qs, mul=mul, stream=stream)
-    k8 = quantize_mxfp8(k, ks, stream=stream)
-    if v_scales == "seq32":
-        v8, vs = quantize_v_seq32(v, stream=stream)
-    elif v_scales == "tensor":
-        v8, vs = quantize_v(v, stream=stream)
-    else:
+    if v_scales not in ("tensor", "seq32"):
         raise ValueError(f"v_scales must be 'tensor' or 'seq32', got {v_scales!r}")
+    q8, k8, v8, qs, ks, vs = _quantize_qkv(q, k, v, mul, v_scales == "seq32", stream)
     if out is None:
         out = torch.empty(B, S, H, D, dtype=torch.bfloat16, device=q.device)
     fmha_fwd_mxfp8(q8, k8, v8, qs, ks, vs, out, path=path, splits=splits, stream=stream, lse=lse, causal=causal,

@@ -51,6 +51,22 @@ int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, in
 /* Bytes of the seq32 scale tensor: B * ceil(SK/32) * HK * 128. */
 size_t fmha_mxfp8_seq32_scale_bytes(int64_t B, int64_t SK, int64_t HK);
 
+/* Q, K and V of one attention layer from bf16 (extension): the same bytes as fmha_mxfp8_quantize_rows of Q (with
+ * q_mul) and of K and fmha_mxfp8_quantize_tensor (or, v_seq32 != 0, _seq32) of V, in one launch (two with the tensor
+ * scale). bytes_q_scale and bytes_k_scale are the whole allocations: what lies behind the scales is cleared (the slack
+ * that the attention requires to be zero). v_scale: 4096 bytes of f32, or E8M0 [B, ceil(SK/32), HK, 128]. */
+typedef struct fmha_mxfp8_qkv_params {
+    const void* q; const void* k; const void* v;        /* bf16 [B,S,H,128], [B,SK,HK,128] twice */
+    void* q8; void* k8; void* v8;                       /* e4m3, same shapes */
+    void* q_scale; void* k_scale; void* v_scale;
+    uint64_t bytes_q, bytes_k, bytes_v, bytes_q8, bytes_k8, bytes_v8;
+    uint64_t bytes_q_scale, bytes_k_scale, bytes_v_scale;
+    int32_t B, S, H, SK, HK, v_seq32;
+    float q_mul;
+    int32_t pad;
+} fmha_mxfp8_qkv_params;
+int fmha_mxfp8_quantize_qkv(const fmha_mxfp8_qkv_params* p, void* stream, char* err, size_t errlen);
+
 #ifdef __cplusplus
 }
 #endif

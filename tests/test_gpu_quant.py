@@ -170,6 +170,31 @@ def test_seq32_special_values(gpu, B, SK, HK):
     assert np.array_equal(_host(q), q_ref)
 
 
+@pytest.mark.parametrize("seq32", [False, True], ids=["tensor", "seq32"])
+@pytest.mark.parametrize("B,S,H,SK,HK", [(1, 1, 1, 1, 1), (2, 33, 3, 65, 3), (1, 300, 8, 77, 2), (3, 64, 5, 1030, 1)])
+def test_qkv_matches_separate_quantisers(gpu, B, S, H, SK, HK, seq32):
+    """The one-launch quantiser of a layer gives the separate kernels' bytes and clears the slack behind the scales."""
+    g = torch.Generator(device=gpu)
+    g.manual_seed(S * 7 + SK)
+    r = lambda *shape: torch.randn(*shape, generator=g, device=gpu, dtype=torch.bfloat16)   # noqa: E731
+    q, k, v = r(B, S, H, D), r(B, SK, HK, D) * 3, r(B, SK, HK, D)
+    trash = torch.full((1 << 20,), 0xa5, dtype=torch.uint8, device=gpu)   # so that fresh allocations are not zero by luck
+    del trash
+    q8, k8, v8, qs, ks, vs = ops._quantize_qkv(q, k, v, 0.125, seq32, None)
+    qs2, ks2 = ops.alloc_scales(B, S, H, gpu), ops.alloc_scales(B, SK, HK, gpu)
+    q2, k2 = ops.quantize_mxfp8(q, qs2, mul=0.125), ops.quantize_mxfp8(k, ks2)
+    v2, vs2 = ops.quantize_v_seq32(v) if seq32 else ops.quantize_v(v)
+    for x, y in ((q8, q2), (k8, k2), (v8, v2), (qs, qs2), (ks, ks2), (vs, vs2)):
+        assert x.shape == y.shape and x.dtype == y.dtype
+        assert np.array_equal(_host(x), _host(y))
+    for x, heads in ((qs, H), (ks, HK)):
+        n = x.numel()
+        whole = torch.empty(0, dtype=torch.uint8, device=gpu).set_(x.untyped_storage(), 0, (n + 640 * heads * 4,))
+        assert not whole[n:].any()
+    if not seq32:
+        assert not vs2[1:512].any() and not vs[1:512].any()
+
+
 def test_rejections(gpu):
     x = torch.zeros(16, D, dtype=torch.bfloat16, device=gpu)
     q = torch.empty(16 * D, dtype=torch.uint8, device=gpu)
