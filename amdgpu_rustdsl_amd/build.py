@@ -7,6 +7,8 @@ Outputs (in-tree, git-ignored, shipped with the source tree):
     amdgpu_rustdsl_amd/_build/mxfp8_quant_gfx950.hsaco  the quantisers
     amdgpu_rustdsl_amd/_build/libfmha_mxfp8.so          include/fmha_mxfp8.h + include/mxfp8_quant.h, both code
                                                         objects embedded
+    amdgpu_rustdsl_amd/_build/_fmha_ops.so              the torch-facing calls of ops.py (a CPython module over
+                                                        libfmha_mxfp8.so and torch's C++ libraries)
 """
 import os
 import subprocess
@@ -21,6 +23,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HSACO = os.path.join(OUT, "fmha_mxfp8_gfx950.hsaco")
 QHSACO = os.path.join(OUT, "mxfp8_quant_gfx950.hsaco")
 LIB = os.path.join(OUT, "libfmha_mxfp8.so")
+OPS = os.path.join(OUT, "_fmha_ops.so")
 
 # Packed FP32 VALU forms are kept out of the kernels (their results have been unreliable on this hardware pool);
 # the host pass warns that it does not know the feature, which is harmless.
@@ -112,6 +115,15 @@ def build(verbose=False):
           "-I" + os.path.join(ROCM, "include"), '-DFMHA_HSACO_PATH="%s"' % HSACO, '-DMXQ_HSACO_PATH="%s"' % QHSACO,
           os.path.join(CSRC, "fmha_host.cpp"), os.path.join(CSRC, "quant_host.cpp"), noalloc_o, "-L" + os.path.join(ROCM, "lib"), "-lamdhip64",
           "-Wl,-rpath," + os.path.join(ROCM, "lib"), "-o", LIB])
+    import sysconfig
+
+    import torch
+    tdir = os.path.dirname(torch.__file__)
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-isystem", os.path.join(tdir, "include"),
+          "-isystem", os.path.join(ROCM, "include"), "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "ops_binding.cpp"),
+          "-L" + OUT, "-lfmha_mxfp8", "-L" + os.path.join(tdir, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+          "-lamdhip64", "-Wl,-rpath,$ORIGIN", "-o", OPS])
     if verbose:
         print("built", HSACO, os.path.getsize(HSACO), "bytes;", LIB, os.path.getsize(LIB), "bytes")
     return LIB

@@ -3,11 +3,23 @@
 include/fmha_mxfp8.h (``amdgpu_rustdsl_amd.lib``). torch is used for device memory and the current stream only.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import math
+import os
 
 import torch
 
 from . import lib
+
+# The native form of the calls below (csrc/ops_binding.cpp): it serves well-formed calls on plain tensors and returns None
+# for any other, which the Python code here then serves or reports.
+_OPS_PATH = os.path.join(os.path.dirname(lib.LIB_PATH), "_fmha_ops.so")
+if not os.path.exists(_OPS_PATH):
+    raise ImportError(f"{_OPS_PATH} is missing: build it with `python amdgpu_rustdsl_amd/build.py` (or __graft_entry__.build())")
+_loader = importlib.machinery.ExtensionFileLoader("_fmha_ops", _OPS_PATH)
+_native = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fmha_ops", _loader))
+_native.set_error(lib.FmhaError)
 
 D = 128
 FMHA_VS128 = "fmha_fwd_hd128_mxfp8_v3_vs128"
@@ -40,6 +52,10 @@ def _expect(t, name, shape, esize, align=1):
     if t.data_ptr() % align:
         raise ValueError(f"{name}: expected {align}-byte alignment")
 
+
+_PATH_CODES = {"auto": -1, "vs128": lib.PATH_VS128, "t128": lib.PATH_T128, "kvsplit": lib.PATH_KVSPLIT}
+_PAIR_MODES = {"auto": 0, True: 1, False: 2}
+_PARTIAL_FORMATS = {"fp16": 0, "fp32": 1}
 
 _workspace = {}
 
@@ -87,7 +103,16 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
     so its output bits differ from the reference grid's by a few ULP; which fill runs depends on the device's CU
     count.
     """
-    pair_modes = {"auto": 0, True: 1, False: 2}
+    if path in _PATH_CODES and causal_pair in _PAIR_MODES and partials in _PARTIAL_FORMATS:
+        split_path = path == "kvsplit"
+        nsplit = (splits or 4) if split_path else 0
+        if (not split_path or nsplit in (2, 4, 8)) and (softmax_scale is None or float(softmax_scale) > 0.0):
+            ran = _native.attend(q, k, v, q_scale, k_scale, v_scale, out, lse, _PATH_CODES[path], nsplit, 1 if causal else 0,
+                                 _PARTIAL_FORMATS[partials], softmax_scale or 0.0, 0 if check else 1, _PAIR_MODES[causal_pair],
+                                 0 if kv_fill else 1, stream)
+            if ran is not None:
+                return lib.Ran(lib.PATH_NAMES[ran[0]], ran[1], ran[2])
+    pair_modes = _PAIR_MODES
     if causal_pair not in pair_modes:
         raise ValueError(f"fmha_fwd_mxfp8: causal_pair must be 'auto', True or False, got {causal_pair!r}")
     if partials not in ("fp16", "fp32"):
@@ -182,6 +207,9 @@ def quantize_mxfp8(x, scale_out, mul=1.0, stream=None):
     the block of ``x * mul`` (f32), elements e4m3 round-to-nearest-even saturating at 448. Writes the scales into
     ``scale_out`` (uint8, shape x.shape[:-1] + (4,); ``alloc_scales`` gives one with the FMHA's zeroed slack) and
     returns the e4m3 bytes (uint8, shape of x). Runs fmha_mxfp8_quantize_rows (include/mxfp8_quant.h)."""
+    done = _native.quantize_rows(x, scale_out, mul, stream)
+    if done is not None:
+        return done
     xb = _bf16(x, "x")
     rows = xb.numel() // D
     _expect(scale_out, "scale_out", tuple(x.shape[:-1]) + (4,), 1, align=4)
@@ -196,6 +224,9 @@ def quantize_v(x, stream=None):
     """On-GPU V quantisation with one f32 descale per tensor (ref_host.cpp:248-251): d = amax / 448, q = e4m3(x / d).
     Returns (q uint8 of x's shape, v_scale: a 4096-byte f32 buffer with d in element 0, the FMHA's V descale
     argument). x may have any shape whose element count is a multiple of 8. Runs fmha_mxfp8_quantize_tensor."""
+    done = _native.quantize_v(x, False, stream)
+    if done is not None:
+        return done
     xb = _bf16(x, "x", rows=False)
     q = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
     vs = torch.empty(1024, dtype=torch.float32, device=x.device)   # written whole: d, zeros, the partial maxima
@@ -208,6 +239,9 @@ def quantize_v_seq32(x, stream=None):
     """On-GPU V quantisation with one E8M0 per 32 keys along the sequence and per head_dim column (an extension; the
     reference's V scale is one f32 per tensor). x [B, SK, HK, 128] -> (q uint8 [B, SK, HK, 128],
     scale uint8 [B, ceil(SK/32), HK, 128]). Runs fmha_mxfp8_quantize_seq32."""
+    done = _native.quantize_v(x, True, stream)
+    if done is not None:
+        return done
     if x.dim() != 4:
         raise ValueError(f"x: expected [B, SK, HK, 128], got {tuple(x.shape)}")
     B, SK, HK, _ = x.shape
@@ -222,6 +256,9 @@ def quantize_v_seq32(x, stream=None):
 def _quantize_qkv(q, k, v, mul, seq32, stream):
     """quantize_mxfp8 of q (with ``mul``) and k, and quantize_v or quantize_v_seq32 of v, as one call: the same bytes in
     one launch (two with the tensor scale), the slack behind the scales cleared by it."""
+    done = _native.quantize_qkv(q, k, v, mul, seq32, stream)
+    if done is not None:
+        return done
     B, S, H, _ = q.shape
     _, SK, HK, _ = k.shape
     if not (q.device == k.device == v.device):   # each tensor on its own device

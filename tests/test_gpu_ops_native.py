@@ -1,0 +1,140 @@
+"""The native form of the torch-facing calls (csrc/ops_binding.cpp) against their Python form, and the workspace that it
+keeps: other streams, threads on one stream, graphs that outlive its growth."""
+import threading
+
+import pytest
+import torch
+
+from amdgpu_rustdsl_amd import lib, ops
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+class _Declines:
+    """In place of the native module: every call goes to the Python form."""
+
+    @staticmethod
+    def _none(*a):
+        return None
+
+    attend = quantize_rows = quantize_v = quantize_qkv = _none
+
+
+def _case(gpu, B, H, HK, S, SK, seed=0):
+    g = torch.Generator(device=gpu)
+    g.manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g, device=gpu, dtype=torch.bfloat16)   # noqa: E731
+    qs = torch.zeros(B * S * H * 4 + 2048 * H, dtype=torch.uint8, device=gpu)[: B * S * H * 4].view(B, S, H, 4)
+    ks = torch.zeros(B * SK * HK * 4 + 2560 * H, dtype=torch.uint8, device=gpu)[: B * SK * HK * 4].view(B, SK, HK, 4)
+    q, k = ops.quantize_mxfp8(r(B, S, H, D), qs, mul=ops.LOG2E_OVER_SQRT_D), ops.quantize_mxfp8(r(B, SK, HK, D), ks)
+    v, vs = ops.quantize_v(r(B, SK, HK, D))
+    return q, k, v, qs, ks, vs
+
+
+def _out(t):
+    return torch.full(t[0].shape, float("nan"), dtype=torch.bfloat16, device=t[0].device)
+
+
+SHAPES = [(1, 1, 1, 256, 256), (1, 8, 8, 256, 2048), (2, 8, 2, 3, 1500), (8, 32, 8, 1, 2048), (1, 4, 4, 300, 129)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
+@pytest.mark.parametrize("kw", [{}, {"lse": True, "causal": True}, {"softmax_scale": 0.1, "partials": "fp32", "kv_fill": False}],
+                         ids=["default", "lse_causal", "scaled_f32_nofill"])
+def test_native_call_equals_python_call(gpu, monkeypatch, shape, kw):
+    t = _case(gpu, *shape)
+    kw = dict(kw)
+    want_lse = kw.pop("lse", False)
+    got = []
+    for native in (True, False):
+        if native:
+            assert ops._native.attend.__name__ == "attend"
+        else:
+            monkeypatch.setattr(ops, "_native", _Declines)
+        out, lse = _out(t), torch.zeros(t[0].shape[0], t[0].shape[2], t[0].shape[1], device=gpu) if want_lse else None
+        ran = ops.fmha_fwd_mxfp8(*t, out, lse=lse, **kw)
+        torch.cuda.synchronize()
+        got.append((tuple(ran), ran.partials, out, lse))
+    a, b = got
+    assert a[:2] == b[:2]
+    assert torch.equal(a[2].view(torch.int16), b[2].view(torch.int16))
+    assert not want_lse or torch.equal(a[3], b[3])
+
+
+def test_native_declines_what_python_reports(gpu):
+    t = _case(gpu, 1, 4, 4, 64, 300)
+    out = _out(t)
+    bad = [(0, t[0].transpose(1, 2)), (0, t[0].cpu()), (1, t[1][:, :, :3]), (6, out.float()), (3, t[3][:, :-1])]
+    for i, x in bad:
+        args = list(t) + [out]
+        args[i] = x
+        assert ops._native.attend(*args, None, -1, 0, 0, 0, 0.0, 0, 0, 0, None) is None
+        with pytest.raises(ValueError):
+            ops.fmha_fwd_mxfp8(*args)
+    short = torch.zeros(64 * 16, dtype=torch.uint8, device=gpu).view(1, 64, 4, 4)   # no slack behind the scales
+    with pytest.raises(lib.FmhaError, match="GV-HOST-EXTENT") as e:
+        ops.fmha_fwd_mxfp8(t[0], t[1], t[2], short, *t[4:], out)
+    assert e.value.code == lib.FMHA_ERR_EXTENT
+    with pytest.raises(RuntimeError):   # a batched tensor has no memory of its own: refused, not a crash
+        torch.vmap(lambda q: (ops.fmha_fwd_mxfp8(q, *t[1:], out), q)[1])(t[0].unsqueeze(0))
+
+
+def test_threads_and_streams_share_nothing_they_should_not(gpu):
+    """Calls that use the workspace from four threads, two on one stream: every output is the single-threaded one."""
+    cases = [_case(gpu, 2, 8, 2, 4, 3000, seed=i) for i in range(4)]
+    want = []
+    for t in cases:
+        o = _out(t)
+        ops.fmha_fwd_mxfp8(*t, o)
+        want.append(o)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)]
+    outs = [[_out(t) for _ in range(12)] for t in cases]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(streams[i % 2]):
+                for o in outs[i]:
+                    ops.fmha_fwd_mxfp8(*cases[i], o)
+        except Exception as e:   # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [x.start() for x in threads]
+    [x.join() for x in threads]
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(4):
+        for o in outs[i]:
+            assert torch.equal(o.view(torch.int16), want[i].view(torch.int16)), i
+
+
+def test_graph_survives_workspace_growth(gpu):
+    """A captured call's workspace stays its own when a later, larger call grows the stream's workspace."""
+    small, large = _case(gpu, 2, 8, 2, 4, 3000, seed=1), _case(gpu, 8, 32, 8, 4, 4096, seed=2)
+    eager = _out(small)
+    ops.fmha_fwd_mxfp8(*small, eager)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream(gpu)
+    out = _out(small)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        ops.fmha_fwd_mxfp8(*small, out)   # the stream's workspace and the code objects, before the capture
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            ops.fmha_fwd_mxfp8(*small, out)
+        big = _out(large)
+        ops.fmha_fwd_mxfp8(*large, big)
+        s.synchronize()
+        trash = [torch.full((1 << 22,), 0xff, dtype=torch.uint8, device=gpu) for _ in range(8)]   # would take a freed workspace
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
+        trash[0].add_(1)
+    del trash
