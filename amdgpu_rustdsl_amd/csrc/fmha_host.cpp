@@ -17,7 +17,7 @@
 
 #include "../../include/fmha_mxfp8.h"
 #include "module_cache.h"
-#include "packed_args.h"
+#include "pre_args.h"
 
 static_assert(sizeof(fmha_mxfp8_args) == 656, "kernarg size (vs128_abi.h:126)");
 static_assert(sizeof(fmha_mxfp8_params) == 192, "params layout (lib.py mirrors it)");
@@ -81,7 +81,7 @@ namespace {
 using fmha_internal::fail;
 using fmha_internal::set_err;
 
-const char* const kKernelNames[16] = {
+const char* const kKernelNames[27] = {
     "fmha_fwd_hd128_mxfp8_v3_vs128",
     "fmha_fwd_hd128_mxfp8_v3_t128",
     "fmha_fwd_hd128_mxfp8_v3_kvsplit",
@@ -96,17 +96,31 @@ const char* const kKernelNames[16] = {
     // extension kernel: the combine with the splits spread over 4 waves (more than 8 partials per row)
     "fmha_fwd_hd128_mxfp8_v3_kvsplit_combine_wide",
     // extension kernels: short query ranges, the rows of a KV head's query heads packed; the merge with the LSE output
-    "fmha_fwd_hd128_mxfp8_v3_packed",
-    "fmha_fwd_hd128_mxfp8_v3_packed_scaled",
+    "fmha_fwd_hd128_mxfp8_pre_packed",
+    "fmha_fwd_hd128_mxfp8_pre_packed_scaled",
     "fmha_fwd_hd128_mxfp8_v3_combine_lse",
     // extension kernels: the 256-row kernel with split last blocks, and their merge
-    "fmha_fwd_hd128_mxfp8_v3_vs128_tail",
-    "fmha_fwd_hd128_mxfp8_v3_vs128_tail_scaled",
+    "fmha_fwd_hd128_mxfp8_pre_vs128_tail",
+    "fmha_fwd_hd128_mxfp8_pre_vs128_tail_scaled",
     "fmha_fwd_hd128_mxfp8_v3_tail_combine",
+    // extension kernels: the bodies of the kernels above on preloaded parameters (fmha_pre_args)
+    "fmha_fwd_hd128_mxfp8_pre_vs128",
+    "fmha_fwd_hd128_mxfp8_pre_vs128_scaled",
+    "fmha_fwd_hd128_mxfp8_pre_split_tiles",
+    "fmha_fwd_hd128_mxfp8_pre_split_tiles_scaled",
+    "fmha_fwd_hd128_mxfp8_pre_t128",
+    "fmha_fwd_hd128_mxfp8_pre_t128_lut",
+    "fmha_fwd_hd128_mxfp8_pre_kvsplit",
+    "fmha_fwd_hd128_mxfp8_pre_packed_seq32",
+    "fmha_fwd_hd128_mxfp8_pre_packed_scaled_seq32",
+    "fmha_fwd_hd128_mxfp8_pre_vs128_tail_seq32",
+    "fmha_fwd_hd128_mxfp8_pre_vs128_tail_scaled_seq32",
 };
 enum { K_VS128 = 0, K_T128 = 1, K_KVSPLIT = 2, K_COMBINE = 3, K_VS128_SC = 4, K_T128_SC = 5, K_KVSPLIT_SC = 6, K_T128ST = 7,
        K_T128ST_SC = 8, K_COMBINE_WIDE = 9, K_PACKED = 10, K_PACKED_SC = 11, K_COMBINE_LSE = 12,
-       K_TAIL = 13, K_TAIL_SC = 14, K_TAIL_COMBINE = 15 };
+       K_TAIL = 13, K_TAIL_SC = 14, K_TAIL_COMBINE = 15, K_PRE_VS128 = 16, K_PRE_VS128_SC = 17, K_PRE_T128ST = 18, K_PRE_T128ST_SC = 19,
+       K_PRE_T128 = 20, K_PRE_T128_LUT = 21, K_PRE_KVSPLIT = 22, K_PACKED_VS = 23, K_PACKED_SC_VS = 24,
+       K_TAIL_VS = 25, K_TAIL_SC_VS = 26 };
 
 // The 128-row grids (t128's shapes, and vs128's half-chip and causal ones below) run on the split-tile kernel (512
 // threads) from 7 key tiles on, and on the one-wave-per-SIMD kernel (256 threads, the reference's order) below that:
@@ -143,7 +157,7 @@ bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool caus
     return blocks <= 128 || (causal && (SK + 127) / 128 >= 4 && !(S == SK && blocks > (int64_t)cu_count()));
 }
 
-fmha_internal::ModuleCache<16> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
+fmha_internal::ModuleCache<27> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
 
 int get_functions(hipFunction_t** out, char* err, size_t errlen) { return g_fmha.get(out, err, errlen); }
 
@@ -334,6 +348,48 @@ i64 tail_sub(i64 blocks, i64 tiles) {
 }
 size_t tail_bytes(i64 rem, i64 sub) { return (size_t)(rem * sub * 256) * 516u; }
 
+// The preloaded parameters of a call (pre_args.h), or false where they cannot hold it: more than 65535 heads (the grid's
+// limit too), or an address past 48 bits.
+bool fill_pre(fmha_pre_args& x, const fmha_mxfp8_params& p, uint32_t flags, void* o, void* lse) {
+    const uint64_t a[6] = {(uint64_t)(uintptr_t)p.q,         (uint64_t)(uintptr_t)p.k,         (uint64_t)(uintptr_t)p.v,
+                           (uint64_t)(uintptr_t)p.q_descale, (uint64_t)(uintptr_t)p.k_descale, (uint64_t)(uintptr_t)p.v_descale};
+    for (uint64_t u : a)
+        if (u >> 48) return false;
+    if (p.H > 65535) return false;
+    std::memset(&x, 0, sizeof(x));
+    x.q_lo = (uint32_t)a[0]; x.k_lo = (uint32_t)a[1]; x.v_lo = (uint32_t)a[2];
+    x.qs_lo = (uint32_t)a[3]; x.ks_lo = (uint32_t)a[4]; x.vd_lo = (uint32_t)a[5];
+    x.hi_qk = (uint32_t)(a[0] >> 32) | (uint32_t)(a[1] >> 32) << 16;
+    x.hi_vqs = (uint32_t)(a[2] >> 32) | (uint32_t)(a[3] >> 32) << 16;
+    x.hi_ksvd = (uint32_t)(a[4] >> 32) | (uint32_t)(a[5] >> 32) << 16;
+    x.S = (uint32_t)p.S;
+    x.SK = (uint32_t)p.SK;
+    uint32_t sh = 0;
+    while ((p.HK << sh) < p.H) ++sh;
+    x.heads = (uint32_t)p.H | sh << 16 | flags << 24;
+    x.scale = p.softmax_scale;
+    x.o = o;
+    x.lse = lse;
+    x.rows_total = (uint32_t)((i64)p.B * p.S * p.H);
+    return true;
+}
+static_assert(sizeof(fmha_pre_args) == 96 && offsetof(fmha_pre_args, o) == 56 && offsetof(fmha_pre_args, out) == 80, "preloaded kernarg");
+
+// The preloaded kernel that runs the body of a full-sequence kernel, or -1: the short recipe (fewer than 4 key tiles), the
+// per-32-key V scales, the causal pairing and the causal single-wave blocks stay with the packed ABI's kernels.
+int pre_kernel(int kern, i64 tiles, uint32_t flags) {
+    if (flags & (FMHA_FLAG_V_SEQ32 | FMHA_FLAG_CAUSAL_PAIR)) return -1;
+    if (kern == K_T128) return (flags & FMHA_FLAG_CAUSAL) ? -1 : tiles < 4 ? K_PRE_T128_LUT : K_PRE_T128;
+    if (tiles < 4) return -1;
+    switch (kern) {
+        case K_VS128: return K_PRE_VS128;
+        case K_VS128_SC: return K_PRE_VS128_SC;
+        case K_T128ST: return K_PRE_T128ST;
+        case K_T128ST_SC: return K_PRE_T128ST_SC;
+        default: return -1;
+    }
+}
+
 // What the one-call entry runs for a shape: the resolved path, and for the packed-rows kernel its shares.
 struct Plan {
     int path, splits;   // as the entry reports them
@@ -363,6 +419,8 @@ int kernel_of(int path, i64 B, i64 H, i64 S, i64 SK, bool causal, bool scaled, u
 // workspace on the full-sequence paths too; the other entries keep the kernels and the bits that they had.
 void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspace, bool any_path) {
     const i64 B = p.B, H = p.H, HK = p.HK, S = p.S, SK = p.SK;
+    fmha_pre_args fits_pre;   // the packed rows and the split last blocks exist on preloaded parameters only
+    any_path = any_path && fill_pre(fits_pre, p, 0u, nullptr, nullptr);
     const size_t one = fmha_mxfp8_workspace_bytes(B, H, S, 1);
     const i64 fits = (i64)std::min<size_t>(workspace / one, 256);
     pl.parts = 1;
@@ -385,10 +443,10 @@ void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspa
             const i64 blocks = (i64)pl.gx * H * B;
             pl.tail = tail_sub(blocks, (SK + 127) / 128);
             pl.tail_blocks = pl.tail ? blocks % cu_count() : 0;
-            if (pl.tail && tail_bytes(pl.tail_blocks, pl.tail) > workspace) pl.tail = pl.tail_blocks = 0;
+            if (pl.tail && (tail_bytes(pl.tail_blocks, pl.tail) > workspace || pl.tail_blocks > 255 || blocks >= (1 << 20))) pl.tail = pl.tail_blocks = 0;
         }
     }
-    if (pl.sub > 0 && pl.parts * pl.sub * B * S * H * 512 >= (1LL << 32)) pl.sub = 0;   // the combines' 32-bit partial offsets
+    if (pl.sub > 0 && (pl.parts > 255 || pl.parts * pl.sub * B * S * H * 512 >= (1LL << 32))) pl.sub = 0;   // the combines' 32-bit partial offsets
 }
 
 // path / splits as the entry resolves them from the params (no checks)
@@ -624,23 +682,14 @@ static int run_packed(const fmha_mxfp8_params& p, const Plan& pl, const fmha_mxf
     const bool f32 = pl.path != FMHA_PATH_KVSPLIT || p.f32_partials;
     uint8_t* ohat = workspace_slot(p, workspace, workspace_bytes, fmha_mxfp8_workspace_bytes(p.B, p.H, p.S, (int)parts));
     uint8_t* lse = ohat + (size_t)parts * rows_total * 512;
-    fmha_packed_args ka;
-    std::memset(&ka, 0, sizeof(ka));
-    ka.q = p.q; ka.k = p.k; ka.v = p.v;
-    ka.qs = p.q_descale; ka.ks = p.k_descale; ka.vd = p.v_descale;
-    ka.ohat = ohat;
-    ka.lse = lse;
-    ka.S = (uint32_t)p.S; ka.SK = (uint32_t)p.SK; ka.H = (uint32_t)p.H; ka.HK = (uint32_t)p.HK;
-    std::memcpy(&ka.softmax_scale, &a.softmax_scale, 4);
-    while ((p.HK << ka.gshift) < p.H) ++ka.gshift;
-    ka.parts = (uint32_t)pl.parts;
-    ka.sub = (uint32_t)pl.sub;
-    ka.groups = (uint32_t)(p.B * parts);
-    ka.rows_total = (uint32_t)rows_total;
-    ka.flags = (a.flags & (FMHA_FLAG_CAUSAL | FMHA_FLAG_V_SEQ32)) | (f32 ? kPackedF32 : 0u) | (pl.whole ? kPackedWhole : 0u);
+    fmha_pre_args ka;
+    if (!fill_pre(ka, p, a.flags & (FMHA_FLAG_CAUSAL | FMHA_FLAG_V_SEQ32), ohat, lse)) return FMHA_ERR_KA_RANGE;   // (make_plan checked)
+    ka.extra = (uint32_t)pl.parts | (uint32_t)pl.sub << 8 | (f32 ? kPreF32 : 0u) | (pl.whole ? kPreWhole : 0u) |
+               ((p.B * parts) % 8 == 0 ? kPreByXcd : 0u);
     const i64 qtiles = ((i64)p.S * (p.H / p.HK) + 127) / 128;
-    const int rc = launch_raw((a.flags & FMHA_FLAG_SCALE) ? K_PACKED_SC : K_PACKED, &ka, sizeof(ka), (uint32_t)(qtiles * p.HK * p.B * parts), 1, 1, 512,
-                              stream, err, errlen);
+    const int rc = launch_raw(p.v_seq32 ? ((a.flags & FMHA_FLAG_SCALE) ? K_PACKED_SC_VS : K_PACKED_VS)
+                                       : ((a.flags & FMHA_FLAG_SCALE) ? K_PACKED_SC : K_PACKED), &ka, sizeof(ka), (uint32_t)(qtiles * p.HK * p.B * parts), 1, 1,
+                              512, stream, err, errlen);
     if (rc != FMHA_OK) return rc;
     return run_combine(p, ohat, lse, parts, f32, pl.path == FMHA_PATH_KVSPLIT ? nullptr : (float*)p.lse, stream, err, errlen);
 }
@@ -651,22 +700,19 @@ static int run_tail(const fmha_mxfp8_params& p, const Plan& pl, const fmha_mxfp8
     const i64 blocks = (i64)pl.gx * p.H * p.B, nfull = blocks - pl.tail_blocks;
     uint8_t* ohat = workspace_slot(p, workspace, workspace_bytes, tail_bytes(pl.tail_blocks, pl.tail));
     uint8_t* lse = ohat + (size_t)(pl.tail_blocks * pl.tail * 256) * 512u;
-    fmha_tail_args ta;
-    ta.base = a;
-    ta.ohat = ohat;
-    ta.lse = lse;
-    ta.nfull = (uint32_t)nfull;
-    ta.ntail = (uint32_t)pl.tail_blocks;
-    ta.sub = (uint32_t)pl.tail;
-    ta.pad = 0;
-    const int rc = launch_raw(pl.kern == K_VS128_SC ? K_TAIL_SC : K_TAIL, &ta, sizeof(ta), (uint32_t)(nfull + pl.tail_blocks * pl.tail), 1, 1,
+    fmha_pre_args ta;
+    if (!fill_pre(ta, p, a.flags & FMHA_FLAG_V_SEQ32, ohat, lse)) return FMHA_ERR_KA_RANGE;   // (make_plan checked)
+    ta.extra = (uint32_t)nfull << 12 | (uint32_t)pl.tail_blocks << 4 | (uint32_t)pl.tail;
+    ta.out = p.o;
+    ta.lse_out = p.lse;
+    const int rc = launch_raw(p.v_seq32 ? (pl.kern == K_VS128_SC ? K_TAIL_SC_VS : K_TAIL_VS) : (pl.kern == K_VS128_SC ? K_TAIL_SC : K_TAIL), &ta, sizeof(ta), (uint32_t)(nfull + pl.tail_blocks * pl.tail), 1, 1,
                               512, stream, err, errlen);
     if (rc != FMHA_OK) return rc;
     struct {
         const void *ohat, *lse;
         void *out, *lse_out;
         uint32_t ntail, sub, nfull, S, H, pad;
-    } ca = {ohat, lse, p.o, p.lse, ta.ntail, ta.sub, ta.nfull, (uint32_t)p.S, (uint32_t)p.H, 0u};
+    } ca = {ohat, lse, p.o, p.lse, (uint32_t)pl.tail_blocks, (uint32_t)pl.tail, (uint32_t)nfull, (uint32_t)p.S, (uint32_t)p.H, 0u};
     return launch_raw(K_TAIL_COMBINE, &ca, sizeof(ca), (uint32_t)(pl.tail_blocks * 16), 1, 1, 256, stream, err, errlen);
 }
 
@@ -740,6 +786,9 @@ static int run_entry(const fmha_mxfp8_params* p, void* workspace, size_t workspa
             a.flags |= FMHA_FLAG_CAUSAL_PAIR;
             kgx = (kgx + 1) / 2;
         }
+        const int pk = pre_kernel(kern, (SK + 127) / 128, a.flags);
+        fmha_pre_args pre;
+        if (pk >= 0 && fill_pre(pre, *p, a.flags, p->o, p->lse)) return launch_raw(pk, &pre, sizeof(pre), kgx, gy, (uint32_t)B, block, stream, err, errlen);
         return launch_raw(kern, &a, sizeof(a), kgx, gy, (uint32_t)B, block, stream, err, errlen);
     }
     // KV split: partials (fp32-sized rows, as ref_host.cpp:149 / ops.py:133) then the LSE, both in the workspace
@@ -764,7 +813,13 @@ static int run_entry(const fmha_mxfp8_params* p, void* workspace, size_t workspa
     int rc = p->no_check ? FMHA_OK : fmha_mxfp8_validate_kvsplit(&ka, &sz, gx, gy, gz, B, HK, 0, err, errlen);
     if (rc != FMHA_OK) return rc;
     if (pl.sub > 0) return run_packed(*p, pl, a, workspace, workspace_bytes, stream, err, errlen);
-    rc = launch_raw(scaled ? K_KVSPLIT_SC : K_KVSPLIT, &ka, sizeof(ka), gx, gy, gz, 512, stream, err, errlen);
+    fmha_pre_args pre;
+    if (!scaled && !p->v_seq32 && (SK + 127) / 128 >= 4 && fill_pre(pre, *p, 0u, ohat, lse)) {
+        pre.extra = (uint32_t)parts | (p->f32_partials ? kPreF32 : 0u) | (gx == 1u && gz % 8u == 0u ? kPreByXcd : 0u);
+        rc = launch_raw(K_PRE_KVSPLIT, &pre, sizeof(pre), gx, gy, gz, 512, stream, err, errlen);
+    } else {
+        rc = launch_raw(scaled ? K_KVSPLIT_SC : K_KVSPLIT, &ka, sizeof(ka), gx, gy, gz, 512, stream, err, errlen);
+    }
     if (rc != FMHA_OK) return rc;
     return run_combine(*p, ohat, lse, parts, p->f32_partials != 0, nullptr, stream, err, errlen);
 }

@@ -32,7 +32,7 @@
 #include <stdint.h>
 
 #include "../../include/fmha_mxfp8.h"
-#include "packed_args.h"
+#include "pre_args.h"
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -185,13 +185,13 @@ __device__ __forceinline__ void kernarg_lines_touch() {
     (void)t0; (void)t1; (void)t2; (void)t3; (void)t4; (void)t5; (void)t6; (void)t7; (void)t8; (void)t9;
 }
 
-// c = f32(softmax scale (kernarg 0x050) x log2 e) split into 2^e m (the host checked that it is a positive normal)
-__device__ inline void set_qk_scale(Prm& p, bool on) {
+// c = f32(softmax scale x log2 e) split into 2^e m (the host checked that it is a positive normal)
+__device__ inline void set_qk_scale(Prm& p, bool on, float scale) {
     p.qk_scaled = on ? 1u : 0u;
     p.qk_e = 0;
     p.qk_m = p.qk_rm = 1.0f;
     if (!on) return;
-    const float c = ka<float>(0x050) * 1.44269504088896340736f;
+    const float c = scale * 1.44269504088896340736f;
     const uint32_t u = __builtin_bit_cast(uint32_t, c);
     p.qk_e = (int32_t)((u >> 23) & 0xffu) - 127;
     p.qk_m = __builtin_bit_cast(float, (u & 0x007fffffu) | (127u << 23));
@@ -219,12 +219,56 @@ __device__ inline Prm prm_from_kernarg() {
     p.vs_row = p.k_seq;
     p.vs_b = ((p.SK + 31u) >> 5) * p.vs_row;
     p.ohat = nullptr; p.lse = nullptr; p.splits = 1; p.rows_total = 0; p.f32_partials = 0;
-    set_qk_scale(p, SC);
+    set_qk_scale(p, SC, SC ? ka<float>(0x050) : 0.0f);
 #ifdef FMHA_TRACE
     // the trace buffer: 0x288 of the 656-byte layout; the KV split's 648-byte layout ends there, so it reads the
     // unused 0x040 slot instead
     if (KVS) p.trace = (uint64_t*)(uintptr_t)ka<uint64_t>(0x040);
     else p.trace = (uint64_t*)(uintptr_t)(ka<uint32_t>(0x288) | ((uint64_t)ka<uint32_t>(0x28C) << 32));
+#endif
+    return p;
+}
+
+// The parameters of the kernels that the one-call entry launches itself: fourteen dwords that the hardware puts into SGPRs at
+// wave launch (the build's -amdgpu-kernarg-preload-count; they are all the user SGPRs beside the kernarg pointer), enough
+// for every address before the first tile, then the output pointers, which are read while the tiles are on their way. A
+// kernel with the packed ABI's ten kernarg lines first waits a memory round trip for them. Against that, the same bodies on one
+// box, us per launch: B2H8S2048 split tiles 21.9 -> 20.8, B1H8S1000 SK1337 15.4 -> 14.6, B1H1S256 7.1 -> 6.8, B4H8S2048
+// 32.2 -> 32.0.
+#define FMHA_PRE_PARAMS                                                                                                 \
+    uint32_t q_lo, uint32_t k_lo, uint32_t v_lo, uint32_t qs_lo, uint32_t ks_lo, uint32_t vd_lo, uint32_t hi_qk, uint32_t hi_vqs, \
+        uint32_t hi_ksvd, uint32_t S, uint32_t SK, uint32_t heads, uint32_t scale, uint32_t extra, uint8_t *o, float *lse, uint32_t rows_total
+#define FMHA_PRE_ARGS q_lo, k_lo, v_lo, qs_lo, ks_lo, vd_lo, hi_qk, hi_vqs, hi_ksvd, S, SK, heads, scale, extra, o, lse, rows_total
+
+// Prm of the preloaded parameters (fmha_pre_args): tensors are packed, so every stride follows from the sizes. PART: o and
+// lse are partial rows and their base-2 LSE.
+template <bool SC, bool PART>
+__device__ __forceinline__ Prm prm_from_preload(FMHA_PRE_PARAMS) {
+    auto ptr = [](uint32_t lo, uint32_t hi) { return (const uint8_t*)(uintptr_t)(((uint64_t)(hi & 0xffffu) << 32) | lo); };
+    Prm p;
+    p.q = ptr(q_lo, hi_qk); p.k = ptr(k_lo, hi_qk >> 16); p.v = ptr(v_lo, hi_vqs);
+    p.qs = ptr(qs_lo, hi_vqs >> 16); p.ks = ptr(ks_lo, hi_ksvd); p.vd = (const float*)ptr(vd_lo, hi_ksvd >> 16);
+    p.S = S; p.SK = SK;
+    p.H = heads & 0xffffu;
+    p.pk_sh = (heads >> 16) & 0xfu;
+    p.gqa = 1u << p.pk_sh;
+    p.flags = heads >> 24;
+    p.q_seq = p.H * 128u; p.q_b = S * p.q_seq;
+    p.k_seq = p.v_seq = (p.H >> p.pk_sh) * 128u; p.k_b = p.v_b = SK * p.k_seq;
+    p.o_seq = p.H * 256u; p.o_b = S * p.o_seq;
+    p.qs_b = S * p.H * 4u; p.ks_b = SK * (p.H >> p.pk_sh) * 4u;
+    p.vs32 = (p.flags & FMHA_FLAG_V_SEQ32) ? (const uint8_t*)p.vd : nullptr;
+    p.vs_row = p.k_seq;
+    p.vs_b = ((SK + 31u) >> 5) * p.vs_row;
+    p.o = PART ? nullptr : o; p.lse_out = PART ? nullptr : lse;
+    p.ohat = PART ? o : nullptr; p.lse = PART ? lse : nullptr;
+    p.splits = 1; p.rows_total = rows_total; p.f32_partials = 0;
+    p.pk_rows = 0; p.seed_key = -1; p.seed_whole = 0; p.tl_row = 0;
+    set_qk_scale(p, SC, __builtin_bit_cast(float, scale));
+    (void)extra;
+#ifdef FMHA_TRACE
+    p.trace = nullptr;
+    p.t_entry = 0;
 #endif
     return p;
 }
@@ -1664,6 +1708,35 @@ __device__ __forceinline__ void full_kernel(uint32_t lds) {
     }
 }
 
+// KV split: block -> (q tile, head, z = batch splits + split). one_tile: one query tile per (batch, head, split) and B x splits a
+// multiple of 8.
+__device__ __forceinline__ void kvsplit_coords(const Prm& p, bool one_tile, uint32_t& qt, uint32_t& head, uint32_t& z) {
+    if (one_tile) {
+        // No two blocks share K/V rows, so the XCD placement serves the LSE
+        // words instead. Block L of the (H, gz) grid goes to XCD L mod 8; L -> z = (L mod 8) + 8 ((L / 8) / H),
+        // head = (L / 8) mod H puts the H heads of one split on one XCD, and the H consecutive LSE words of a row
+        // (row index (b S + s) H + h) meet in one L2, which writes them back as whole lines.
+        const uint32_t L = blockIdx.y + p.H * blockIdx.z, j = L >> 3;
+        qt = 0;
+        head = __builtin_amdgcn_readfirstlane(j % p.H);
+        z = __builtin_amdgcn_readfirstlane((L & 7u) + 8u * (j / p.H));
+    } else {
+        block_coords(p.S, p.H, 256u, qt, head, z);
+    }
+}
+
+// components.rs:20-30 / 58-74: z = batch * splits + split; split s owns tiles [s tps, min(ntiles, (s+1) tps))
+__device__ __forceinline__ void kvsplit_range(const Prm& p, uint32_t z, uint32_t& bidx, uint32_t& split, uint32_t& key_lo, uint32_t& key_hi) {
+    bidx = z / p.splits;
+    split = z % p.splits;
+    const uint32_t ntiles = (p.SK + 127u) / 128u;
+    const uint32_t tps = (ntiles + p.splits - 1u) / p.splits;
+    const uint32_t tile_lo = split * tps;
+    const uint32_t tile_hi = min(ntiles, tile_lo + tps);
+    key_lo = tile_lo * 128u;
+    key_hi = min(tile_hi * 128u, p.SK);
+}
+
 // The KV-split kernel body (SC as in full_kernel).
 template <bool SC>
 __device__ __forceinline__ void kvsplit_kernel(uint32_t smem_base) {
@@ -1685,26 +1758,10 @@ __device__ __forceinline__ void kvsplit_kernel(uint32_t smem_base) {
     p.rows_total = ka<uint32_t>(offsetof(fmha_mxfp8_kvsplit_args, kvs_rows_total));
     uint32_t qt, head, z;
     const uint32_t gz = p.rows_total / (p.S * p.H) * p.splits;   // B x splits (rows_total = B S H: validate's rule)
-    if ((p.S + 255u) / 256u == 1u && (gz & 7u) == 0u) {
-        // One query tile per (batch, head, split): no two blocks share K/V rows, so the XCD placement serves the LSE
-        // words instead. Block L of the (H, gz) grid goes to XCD L mod 8; L -> z = (L mod 8) + 8 ((L / 8) / H),
-        // head = (L / 8) mod H puts the H heads of one split on one XCD, and the H consecutive LSE words of a row
-        // (row index (b S + s) H + h) meet in one L2, which writes them back as whole lines.
-        const uint32_t L = blockIdx.y + p.H * blockIdx.z, j = L >> 3;
-        qt = 0;
-        head = __builtin_amdgcn_readfirstlane(j % p.H);
-        z = __builtin_amdgcn_readfirstlane((L & 7u) + 8u * (j / p.H));
-    } else {
-        block_coords(p.S, p.H, 256u, qt, head, z);
-    }
-    // components.rs:20-30 / 58-74: z = batch * splits + split; split s owns tiles [s tps, min(ntiles, (s+1) tps))
-    const uint32_t bidx = z / p.splits, split = z % p.splits;
-    const uint32_t ntiles = (p.SK + 127u) / 128u;
-    const uint32_t tps = (ntiles + p.splits - 1u) / p.splits;
-    const uint32_t tile_lo = split * tps;
-    const uint32_t tile_hi = min(ntiles, tile_lo + tps);
-    const uint32_t key_lo = tile_lo * 128u, key_hi = min(tile_hi * 128u, p.SK);
-    const bool lut = ntiles < 4u;
+    kvsplit_coords(p, (p.S + 255u) / 256u == 1u && (gz & 7u) == 0u, qt, head, z);
+    uint32_t bidx, split, key_lo, key_hi;
+    kvsplit_range(p, z, bidx, split, key_lo, key_hi);
+    const bool lut = (p.SK + 127u) / 128u < 4u;
     // a block with at most 128 query rows (decode-like S; the ragged last block) splits each tile's keys between the
     // two wave groups instead of leaving the second group on padding rows (the LUT recipe, SK < 512, keeps the plain
     // order)
@@ -1757,39 +1814,20 @@ __device__ __forceinline__ void t128_split_tiles_kernel(uint32_t lds) {
 // read once per KV head instead of once per query head and a block's rows are not padding; each of the reference's
 // `parts` key ranges is cut into `sub` further ones, one block each, until the grid fills the CUs. Bound by HBM: a
 // split-tile block streams a 32 KiB key tile in ~1.05 us, 8 TB/s over 256 CUs.
-template <bool SC>
-__device__ __forceinline__ void packed_kernel(uint32_t lds) {
-    Prm p;
-#define PK_FIELD(T, field) ka<T>(offsetof(fmha_packed_args, field))
-    p.q = (const uint8_t*)PK_FIELD(uint64_t, q); p.k = (const uint8_t*)PK_FIELD(uint64_t, k); p.v = (const uint8_t*)PK_FIELD(uint64_t, v);
-    p.qs = (const uint8_t*)PK_FIELD(uint64_t, qs); p.ks = (const uint8_t*)PK_FIELD(uint64_t, ks);
-    p.vd = (const float*)PK_FIELD(uint64_t, vd);
-    p.ohat = (uint8_t*)PK_FIELD(uint64_t, ohat); p.lse = (float*)PK_FIELD(uint64_t, lse);
-    p.S = PK_FIELD(uint32_t, S); p.SK = PK_FIELD(uint32_t, SK); p.H = PK_FIELD(uint32_t, H);
-    const uint32_t HK = PK_FIELD(uint32_t, HK), parts = PK_FIELD(uint32_t, parts), sub = PK_FIELD(uint32_t, sub);
-    const uint32_t flags = PK_FIELD(uint32_t, flags), groups = PK_FIELD(uint32_t, groups);
-    p.pk_sh = PK_FIELD(uint32_t, gshift);
-    p.rows_total = PK_FIELD(uint32_t, rows_total);
-#undef PK_FIELD
-    p.gqa = 1u << p.pk_sh;
-    p.flags = flags & FMHA_FLAG_CAUSAL;
-    p.f32_partials = (flags & kPackedF32) ? 1u : 0u;
-    p.seed_whole = (flags & kPackedWhole) ? 1u : 0u;
-    p.q_seq = p.H * 128u; p.q_b = p.S * p.q_seq;
-    p.k_seq = p.v_seq = HK * 128u; p.k_b = p.v_b = p.SK * p.k_seq;
-    p.qs_b = p.S * p.H * 4u; p.ks_b = p.SK * HK * 4u;
-    p.o = nullptr; p.o_seq = p.o_b = 0u; p.lse_out = nullptr;
-    p.vs32 = (flags & FMHA_FLAG_V_SEQ32) ? (const uint8_t*)p.vd : nullptr;
-    p.vs_row = p.k_seq;
-    p.vs_b = ((p.SK + 31u) >> 5) * p.vs_row;
+template <bool SC, bool VS>
+__device__ __forceinline__ void packed_kernel(uint32_t lds, FMHA_PRE_PARAMS) {
+    Prm p = prm_from_preload<SC, true>(FMHA_PRE_ARGS);
+    const uint32_t parts = extra & 0xffu, sub = (extra >> 8) & 0x1fu, HK = p.H >> p.pk_sh;
+    const bool by_xcd = (extra & kPreByXcd) != 0u;
+    p.f32_partials = (extra & kPreF32) ? 1u : 0u;
+    p.seed_whole = (extra & kPreWhole) ? 1u : 0u;
+    p.flags &= FMHA_FLAG_CAUSAL;
     p.splits = parts * sub;
     p.pk_rows = p.S << p.pk_sh;
-    set_qk_scale(p, SC);
     // block -> (row tile, KV head, group), a group being one key range of one batch: the KV heads of a group are consecutive
     // 128-byte pieces of the same K and V rows and LSE rows, and the row tiles of one head share its K and V, so a
     // group's blocks go to one XCD when the groups are a multiple of 8 (the hardware deals blocks round-robin over them)
     const uint32_t qtiles = (p.pk_rows + 127u) >> 7, L = blockIdx.x, gb = qtiles * HK;
-    const bool by_xcd = (groups & 7u) == 0u;
     const uint32_t j = by_xcd ? L >> 3 : L;
     const uint32_t qt = __builtin_amdgcn_readfirstlane(j % qtiles);
     const uint32_t hk = __builtin_amdgcn_readfirstlane(j / qtiles % HK);
@@ -1803,21 +1841,19 @@ __device__ __forceinline__ void packed_kernel(uint32_t lds) {
     const uint32_t key_lo = t0 * 128u, key_hi = min(t1 * 128u, p.SK);
     p.seed_key = p.seed_whole || t0 != lo ? (int32_t)(lo * 128u) : -1;
     const uint32_t head = hk << p.pk_sh;
-    if (p.vs32) attend_pingpong<false, true, true, true, SC, kRowsPacked>(p, lds, qt, head, bidx, split, key_lo, key_hi);
-    else attend_pingpong<false, true, false, true, SC, kRowsPacked>(p, lds, qt, head, bidx, split, key_lo, key_hi);
+    attend_pingpong<false, true, VS, true, SC, kRowsPacked>(p, lds, qt, head, bidx, split, key_lo, key_hi);
 }
 
 // The 256-row kernel with split last blocks (extension): a grid of n blocks of equal work on c CUs takes ceil(n / c) rounds, the
 // last of them on n mod c CUs. Here blocks 0 .. nfull - 1 (whole rounds) run as in the vs128 kernel, and each of the
 // ntail remaining ones is cut into `sub` key ranges, one block each, that write f32 partials (tail_combine merges them).
 // Every range starts from the reference of the first tile, so P is quantised as in the uncut block.
-template <bool SC>
-__device__ __forceinline__ void tail_kernel(uint32_t lds) {
-    Prm p = prm_from_kernarg<SC>();
-    const uint32_t nfull = ka<uint32_t>(offsetof(fmha_tail_args, nfull)), ntail = ka<uint32_t>(offsetof(fmha_tail_args, ntail));
-    const uint32_t sub = ka<uint32_t>(offsetof(fmha_tail_args, sub));
-    p.ohat = (uint8_t*)ka<uint64_t>(offsetof(fmha_tail_args, ohat));
-    p.lse = (float*)ka<uint64_t>(offsetof(fmha_tail_args, lse));
+template <bool SC, bool VS>
+__device__ __forceinline__ void tail_kernel(uint32_t lds, uint8_t* out, float* lse_out, FMHA_PRE_PARAMS) {
+    Prm p = prm_from_preload<SC, true>(FMHA_PRE_ARGS);
+    p.o = out;
+    p.lse_out = lse_out;
+    const uint32_t nfull = extra >> 12, ntail = (extra >> 4) & 0xffu, sub = extra & 0xfu;
     const uint32_t gx = (p.S + 255u) / 256u, L = blockIdx.x;
     const bool tail = L >= nfull;
     const uint32_t i = tail ? L - nfull : L;
@@ -1827,8 +1863,7 @@ __device__ __forceinline__ void tail_kernel(uint32_t lds) {
     const uint32_t qt = __builtin_amdgcn_readfirstlane(l % gx), bh = l / gx;
     const uint32_t head = __builtin_amdgcn_readfirstlane(bh % p.H), z = __builtin_amdgcn_readfirstlane(bh / p.H);
     if (!tail) {
-        if (p.vs32) attend_pingpong<false, false, true, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
-        else attend_pingpong<false, false, false, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
+        attend_pingpong<false, false, VS, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
         return;
     }
     const uint32_t ntiles = (p.SK + 127u) / 128u, per = (ntiles + sub - 1u) / sub;
@@ -1837,8 +1872,7 @@ __device__ __forceinline__ void tail_kernel(uint32_t lds) {
     p.seed_key = t0 != 0u ? 0 : -1;
     p.f32_partials = 1u;
     p.tl_row = (int64_t)(part * ntail + ti) * 256 - (int64_t)qt * 256;
-    if (p.vs32) attend_pingpong<false, true, true, false, SC, kRowsOfBlock>(p, lds, qt, head, z, 0, key_lo, key_hi);
-    else attend_pingpong<false, true, false, false, SC, kRowsOfBlock>(p, lds, qt, head, z, 0, key_lo, key_hi);
+    attend_pingpong<false, true, VS, false, SC, kRowsOfBlock>(p, lds, qt, head, z, 0, key_lo, key_hi);
 }
 
 }  // namespace
@@ -1899,31 +1933,99 @@ extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_t12
     t128_split_tiles_kernel<true>(smem_base);
 }
 
-// Extension kernels (no counterpart in the reference): packed rows, fmha_packed_args.
-extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_packed(fmha_packed_args a) {
+// The kernels of the one-call entry (extension: fmha_pre_args, no counterpart in the reference): the bodies of the kernels above
+// on preloaded parameters, each for one recipe and the per-tensor V descale, plus the packed rows and the split last
+// blocks. `extra` is the word that the kernel needs beside the shape.
+#define FMHA_PRE_KERNEL(name, threads) extern "C" __global__ void __launch_bounds__(threads, 1) fmha_fwd_hd128_mxfp8_pre_##name
+
+template <bool SC>
+__device__ __forceinline__ void pre_vs128(uint32_t lds, FMHA_PRE_PARAMS) {
+    const Prm p = prm_from_preload<SC, false>(FMHA_PRE_ARGS);
+    uint32_t qt, head, z;
+    block_coords(p.S, p.H, 256u, qt, head, z);
+    if (p.flags & FMHA_FLAG_CAUSAL) causal_coords(p.S, p.H, qt, head);
+    attend_pingpong<false, false, false, false, SC>(p, lds, qt, head, z, 0, 0, p.SK);
+}
+FMHA_PRE_KERNEL(vs128, 512)(FMHA_PRE_PARAMS) {
     FMHA_LDS_BASE(smem);
-    (void)a;
-    packed_kernel<false>(smem_base);
+    pre_vs128<false>(smem_base, FMHA_PRE_ARGS);
+}
+FMHA_PRE_KERNEL(vs128_scaled, 512)(FMHA_PRE_PARAMS) {
+    FMHA_LDS_BASE(smem);
+    pre_vs128<true>(smem_base, FMHA_PRE_ARGS);
 }
 
-extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_packed_scaled(fmha_packed_args a) {
+// not the causal pairing, whose pass loop takes registers (13 VGPRs and 20 SGPR spills) from every call: it stays with the
+// split-tile kernel of the packed ABI
+template <bool SC>
+__device__ __forceinline__ void pre_split_tiles(uint32_t lds, FMHA_PRE_PARAMS) {
+    const Prm p = prm_from_preload<SC, false>(FMHA_PRE_ARGS);
+    uint32_t qt, head, z;
+    block_coords(p.S, p.H, 128u, qt, head, z);
+    attend_pingpong<false, false, false, true, SC>(p, lds, qt, head, z, 0, 0, p.SK);
+}
+FMHA_PRE_KERNEL(split_tiles, 512)(FMHA_PRE_PARAMS) {
     FMHA_LDS_BASE(smem);
-    (void)a;
-    packed_kernel<true>(smem_base);
+    pre_split_tiles<false>(smem_base, FMHA_PRE_ARGS);
+}
+FMHA_PRE_KERNEL(split_tiles_scaled, 512)(FMHA_PRE_PARAMS) {
+    FMHA_LDS_BASE(smem);
+    pre_split_tiles<true>(smem_base, FMHA_PRE_ARGS);
 }
 
-// Extension kernels: the 256-row kernel with split last blocks, fmha_tail_args.
-extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_vs128_tail(fmha_tail_args a) {
+// not causal: the pairing stays with the t128 kernel
+template <bool LUT>
+__device__ __forceinline__ void pre_t128(uint32_t lds, FMHA_PRE_PARAMS) {
+    const Prm p = prm_from_preload<false, false>(FMHA_PRE_ARGS);
+    uint32_t qt, head, z;
+    block_coords(p.S, p.H, 128u, qt, head, z);
+    attend_single_wave<LUT, false, false>(p, lds, qt, head, z);
+}
+FMHA_PRE_KERNEL(t128, 256)(FMHA_PRE_PARAMS) {
     FMHA_LDS_BASE(smem);
-    (void)a;
-    tail_kernel<false>(smem_base);
+    pre_t128<false>(smem_base, FMHA_PRE_ARGS);
+}
+FMHA_PRE_KERNEL(t128_lut, 256)(FMHA_PRE_PARAMS) {
+    FMHA_LDS_BASE(smem);
+    pre_t128<true>(smem_base, FMHA_PRE_ARGS);
 }
 
-extern "C" __global__ void __launch_bounds__(512, 1) fmha_fwd_hd128_mxfp8_v3_vs128_tail_scaled(fmha_tail_args a) {
+// extra: the split count, kPreF32
+FMHA_PRE_KERNEL(kvsplit, 512)(FMHA_PRE_PARAMS) {
     FMHA_LDS_BASE(smem);
-    (void)a;
-    tail_kernel<true>(smem_base);
+    Prm p = prm_from_preload<false, true>(FMHA_PRE_ARGS);
+    p.splits = extra & 0xffffu;
+    p.f32_partials = (extra & kPreF32) ? 1u : 0u;
+    uint32_t qt, head, z;
+    kvsplit_coords(p, (extra & kPreByXcd) != 0u, qt, head, z);
+    uint32_t bidx, split, key_lo, key_hi;
+    kvsplit_range(p, z, bidx, split, key_lo, key_hi);
+    if (p.S - qt * 256u <= 128u) attend_pingpong<false, true, false, true, false>(p, smem_base, qt, head, bidx, split, key_lo, key_hi);
+    else attend_pingpong<false, true, false, false, false>(p, smem_base, qt, head, bidx, split, key_lo, key_hi);
 }
+
+// One kernel per recipe option: with the V-scale and scaled bodies behind branches of one kernel, its register allocation
+// (SGPR spills, VGPRs) and code size were those of the largest.
+#define FMHA_PACKED_KERNEL(name, SC, VS)                 \
+    FMHA_PRE_KERNEL(name, 512)(FMHA_PRE_PARAMS) {        \
+        FMHA_LDS_BASE(smem);                             \
+        packed_kernel<SC, VS>(smem_base, FMHA_PRE_ARGS); \
+    }
+FMHA_PACKED_KERNEL(packed, false, false)
+FMHA_PACKED_KERNEL(packed_scaled, true, false)
+FMHA_PACKED_KERNEL(packed_seq32, false, true)
+FMHA_PACKED_KERNEL(packed_scaled_seq32, true, true)
+
+#define FMHA_TAIL_KERNEL(name, SC, VS)                                                             \
+    FMHA_PRE_KERNEL(name, 512)(FMHA_PRE_PARAMS, uint32_t pad, uint8_t* out, float* lse_out) {      \
+        FMHA_LDS_BASE(smem);                                                                       \
+        (void)pad;                                                                                 \
+        tail_kernel<SC, VS>(smem_base, out, lse_out, FMHA_PRE_ARGS);                               \
+    }
+FMHA_TAIL_KERNEL(vs128_tail, false, false)
+FMHA_TAIL_KERNEL(vs128_tail_scaled, true, false)
+FMHA_TAIL_KERNEL(vs128_tail_seq32, false, true)
+FMHA_TAIL_KERNEL(vs128_tail_scaled_seq32, true, true)
 
 // epilogue.rs:89-167 / io.rs:164-185: thread t -> 8 consecutive outputs of row t >> 4 (tail threads redo the last group)
 // The combines take the 36-byte layout (fmha_mxfp8_combine_args: three pointers, then rows_total, d and the split
