@@ -146,7 +146,8 @@ bool use_split_tiles(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
 // 256-row grid has more blocks than CUs: there the 256-row kernel with its heaviest query tiles first balances as well
 // and takes 1.5 us per 256 rows and key tile where the split-tile kernel takes 2.1 (us per call, split-tile / 256-row:
 // B1 H32 HK8 S6144 174.3 / 146.1, S4096 82.6 / 66.5, B3 H8 S3001 63.7 / 40.0, B8 H8 S2048 62.5 / 59.2; at one round of
-// blocks it loses: B1 H8 S8192 72.2 / 86.4, B2 H8 S4096 41.9 / 47.5). With many more keys than queries (chunked prefill,
+// blocks it loses: B1 H8 S8192 72.2 / 86.4, B2 H8 S4096 41.9 / 47.5). 9 key tiles keep the split-tile kernel, which
+// fmha_mxfp8_uses_split_tiles has always named there (B8 H8 S1152 39.4 / 29.9). With many more keys than queries (chunked prefill,
 // S < SK) the split-tile order is kept: every row then averages many keys, and outputs of the two orders, though equally
 // close to float64, differ by 3 % from each other. The kernel is chosen as for t128 (above). Below the split-tile threshold the 256-thread t128 kernel gives the vs128 kernel's order and bits
 // (both take every tile whole) on twice the blocks; measured with the LUT recipe at B4H8S1024 SK256, B2H8S2048 SK384
@@ -154,7 +155,8 @@ bool use_split_tiles(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
 // stays ahead: B8H8S2048 SK256 25.4 against 36.4 us). The direct vs128 launcher keeps the 256-row kernel its grid names.
 bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
     const int64_t blocks = (S + 255) / 256 * H * B;
-    return blocks <= 128 || (causal && (SK + 127) / 128 >= 4 && !(S == SK && blocks > (int64_t)cu_count()));
+    const int64_t tiles = (SK + 127) / 128;
+    return blocks <= 128 || (causal && tiles >= 4 && !(S == SK && (tiles <= 8 || tiles >= 10) && blocks > (int64_t)cu_count()));
 }
 
 fmha_internal::ModuleCache<27> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
