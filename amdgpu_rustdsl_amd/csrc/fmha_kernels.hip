@@ -496,6 +496,41 @@ struct Stager {
             dma16(rv, vbase + g * 1024u, dmaoff, soff);
         }
     }
+    // The loop's copies as running state: base and remaining bytes of the next K, V and K-scale tiles, advanced by one tile per
+    // call. `limit` ends the block's last tile, so a tile past it finds no bytes left (its size is at most -stride + one
+    // row's bytes, never positive) and needs no test. From the tile index, the three resources took ~50 scalar
+    // instructions in a row per VALU phase, during which the wave converted nothing.
+    uint64_t ck, cv, cks;
+    int nk, nv, nks;
+    uint32_t cstep, csstep, woff;
+    __device__ __forceinline__ void init_cursors(uint32_t kkey, uint32_t vkey, uint32_t limit) {
+        ck = (uint64_t)(uintptr_t)kb + (uint64_t)kkey * k_seq;
+        cv = (uint64_t)(uintptr_t)vb + (uint64_t)vkey * k_seq;
+        cks = (uint64_t)(uintptr_t)ksb + (uint64_t)kkey * ks_row;
+        nk = ((int)limit - 1 - (int)kkey) * (int)k_seq + kD;
+        nv = ((int)limit - 1 - (int)vkey) * (int)k_seq + kD;
+        nks = ((int)limit - 1 - (int)kkey) * (int)ks_row + 4;
+        cstep = kTile * k_seq;
+        csstep = kTile * ks_row;
+        woff = __builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
+    }
+    // K's copies, then V's: alternating, or V first, cost the split-tile grids 1 % and 3 %
+    __device__ __forceinline__ void dma_next(uint32_t kslot, uint32_t vslot) {
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0));
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0));
+        const uint32_t kbase = slot_base(lds + woff, kLdsK, kslot, kTileBytes), vbase = slot_base(lds + woff, kLdsV, vslot, kTileBytes);
+#pragma unroll
+        for (int i = 0; i < kN; ++i) dma16(rk, kbase + (uint32_t)i * (NT * 16u), dmaoff, __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
+#pragma unroll
+        for (int i = 0; i < kN; ++i) dma16(rv, vbase + (uint32_t)i * (NT * 16u), dmaoff, __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
+        ck += cstep; cv += cstep;
+        nk -= (int)cstep; nv -= (int)cstep;
+    }
+    __device__ __forceinline__ void load_ks_next() {
+        ksr = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc((const void*)(uintptr_t)cks, (uint32_t)max(nks, 0)), ksoff, 0, 0);
+        cks += csstep;
+        nks -= (int)csstep;
+    }
     // The K-scale words of tile [kkey0, kkey0 + 128) into ksr (register-staged: the upper k-group's copy is shifted)
     __device__ __forceinline__ void load_ks(uint32_t kkey0, bool kvalid) {
         const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksb + (size_t)kkey0 * ks_row, tile_bytes(kkey0, kvalid, ks_row, 4));
@@ -508,8 +543,7 @@ struct Stager {
         return __builtin_amdgcn_raw_buffer_load_b32(rks, ksoff, 0, 0);
     }
     __device__ __forceinline__ void store_ks_word(uint32_t word, uint32_t kslot) const {
-        const uint32_t ksw_base = tid < 256u ? slot_base(lds, kLdsKs, kslot, kKsSlot) : lds + kLdsKsDummy;
-        lds_write4(ksw_base + kswoff, word >> ksshift);
+        lds_write4(slot_base(lds, kLdsKs, kslot, kKsSlot) + kswoff, word >> ksshift);   // (threads 0..255: group A)
     }
 
 };
@@ -1383,15 +1417,19 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         // slots written in I(t), K (t-1) & 3 and V (t-2) & 3, were last read in I(t-1). The K-scale words go through
         // registers: V(t) loads tile t+3's and stores tile t+2's (slot (t+2) & 3, last read in I(t-3)), published by
         // barrier t. A copy past the range (an empty resource) writes zeros into its slot, which is free as above.
-        constexpr int kDmaOps = 2 * Stager<NT>::kN + 1 + (VS ? 1 : 0);   // VMEM operations issued per VALU phase
+        // group A (threads 0..255) stages the K-scale words for both
+        constexpr int kDmaOps = 2 * Stager<NT>::kN + (GB ? 0 : 1) + (VS ? 1 : 0);   // VMEM operations issued per VALU phase
         // Every prologue load goes out at once (Q and its scales were issued by init): the K-scale words of tiles 0..2,
         // then the copies. One memory round trip to the first barrier (the stores of the words wait for their loads).
         st.init_dma();
-        const uint32_t ks0 = st.ks_word(key_of(0), true);
-        const uint32_t ks1 = st.ks_word(key_of(1), ntiles > 1);
         const bool seed = SEED && p.seed_key >= 0;
-        const uint32_t kss = seed ? st.ks_word((uint32_t)p.seed_key, true) : 0u;
-        st.load_ks(key_of(2), ntiles > 2);                              // stored by V(0)
+        uint32_t ks0 = 0, ks1 = 0, kss = 0;
+        if (!GB) {
+            ks0 = st.ks_word(key_of(0), true);
+            ks1 = st.ks_word(key_of(1), ntiles > 1);
+            if (seed) kss = st.ks_word((uint32_t)p.seed_key, true);
+            st.load_ks(key_of(2), ntiles > 2);                          // stored by V(0)
+        }
         // The first barrier needs K 0, V 0 and K 1 (read in I(0)); V 1 and K 2 are first read in I(1), so barrier 0
         // waits for them and they stay out of the first barrier's burst.
         st.dma(key_of(0), true, 0, key_of(0), true, 0);                 // K 0, V 0
@@ -1403,15 +1441,18 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         // assembly), so its wait there leaves at most two VMEM operations of any kind in flight: placed before the
         // copies of K 2 and V 1, it does not hold the first barrier for those two (kvsplit kernel alone at cfg5
         // -2.4 %, cfg3 -0.6 %).
-        st.store_ks_word(ks0, 0);
-        st.store_ks_word(ks1, 1);
-        if (seed) st.store_ks_word(kss, 3);
+        if (!GB) {
+            st.store_ks_word(ks0, 0);
+            st.store_ks_word(ks1, 1);
+            if (seed) st.store_ks_word(kss, 3);
+        }
         w.commit_q();   // (its wait for the Q scale word likewise comes before the copies of K 2 and V 1)
         st.dma(key_of(2), ntiles > 2, 2, key_of(1), ntiles > 1, 1);     // K 2, V 1
         if (VS) st.dma_vs(key_of(1), ntiles > 1, 1);                    // V scales of tile 1
         // everything but the copies of K 2 and V 1 (which barrier 0 waits for)
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * Stager<NT>::kN + (VS ? 1 : 0)) : "memory");
         FMHA_MARK(p, tblk, 2);
+        st.init_cursors(key_of(3), key_of(2), min(p.SK, key_lo + ntiles * kTile));
         block_barrier();
         FMHA_MARK(p, tblk, 3);
         if (seed) {
@@ -1439,10 +1480,12 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         const bool idle = PK && w.row0 >= p.pk_rows;
         if (idle) {
             for (uint32_t t = 0; t < ntiles; ++t) {
-                st.store_ks(slot_of(t + 2));
-                st.dma(key_of(t + 3), t + 3 < ntiles, slot_of(t + 3), key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                if (!GB) {
+                    st.store_ks(slot_of(t + 2));
+                    st.load_ks_next();
+                }
+                st.dma_next(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
-                st.load_ks(key_of(t + 3), t + 3 < ntiles);
                 block_barrier_keep_dma<0, kDmaOps>();
             }
         }
@@ -1456,13 +1499,17 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
             typename Wave<NT>::QkPre pre;
             // V(t)'s copies: K tile t+3 and V tile t+2 (and the per-32-key V scales), the K-scale words of tile t+3
             auto copies = [&](uint32_t t) {
-                st.dma(key_of(t + 3), t + 3 < ntiles, slot_of(t + 3), key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                // the words first: their store in V(t + 1) then waits for the copies of V(t) in flight longer
+                if (!GB) st.load_ks_next();
+                st.dma_next(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
-                st.load_ks(key_of(t + 3), t + 3 < ntiles);
             };
             auto v_phase = [&](uint32_t t, uint32_t (&pw)[NA][4], bool last) {
                 FMHA_SETPRIO(0);
-                st.store_ks(slot_of(t + 2));
+                if (!GB) {
+                    asm volatile("" : "+v"(st.ksr));   // the wait for the word stays here (later in the phase: +1 % on split tiles)
+                    st.store_ks(slot_of(t + 2));
+                }
                 if (SC) w.scale_s(s, mrow);   // the in-kernel softmax scale (an instantiation of its own)
                 if (w.needs_mask(key_of(t))) {
                     w.template apply_mask<KB0>(s, key_of(t));
