@@ -7,6 +7,9 @@
 //   fmha_fwd_hd128_mxfp8_v3_kvsplit_combine8h LSE-weighted merge of the partials, 8 outputs per thread
 // and extensions with the same layouts: _t128_split_tiles (t128's grid, 8 waves splitting each tile's keys),
 // _kvsplit_combine_wide (the merge for many partials), and the _scaled kernels (the softmax scale applied in the kernel).
+// The one-call entry launches the _pre_ kernels: the same bodies on preloaded parameters, one recipe option each, and two
+// of its own: _pre_packed* (short query ranges, a KV head's query heads packed into one block's rows) and
+// _pre_vs128_tail* (the 256-row grid with its last blocks split over idle CUs).
 //
 // Per wave: 32 query rows. S^T (keys x queries) = K Q^T on v_mfma_scale_f32_32x32x64_f8f6f4 with the E8M0
 // scales in the MFMA (K scale byte-selected per lane half, Q scale - 9 so S comes out x 2^-9), seeded with the
@@ -64,7 +67,7 @@ constexpr int kLdsK = 0;                      // kSlots K tiles
 constexpr int kLdsV = kSlots * kTileBytes;    // kSlots V tiles
 constexpr int kLdsKs = 2 * kSlots * kTileBytes;   // kSlots x 1 KiB of K scales: the words, then the words >> 8
 constexpr int kKsSlot = 1024;
-constexpr int kLdsKsDummy = kLdsKs + kSlots * kKsSlot;   // 1 KiB sink for the K-scale writes of threads 256..511
+constexpr int kLdsKsDummy = kLdsKs + kSlots * kKsSlot;   // 1 KiB sink for the K-scale copies of the 256-thread kernel's waves 2, 3
 // per-32-key V scales (extension): kSlots x 512 B (4 blocks of 32 keys x 128 columns), then a 2 KiB sink for the
 // copies of the waves that carry none
 constexpr int kVsSlot = 512;
@@ -403,8 +406,8 @@ template <int NT>
 struct Stager {
     static constexpr int kN = kTileBytes / (NT * 16);   // 16-byte chunks per thread per 16 KiB tile
     const uint8_t *kb, *vb, *ksb;
-    uint32_t ksoff;     // K-scale load offset: key (tid & 127) for tid < 256, out of range (zeros) beyond
-    uint32_t kswoff;    // K-scale LDS write offset in a slot (tid < 256: word tid; beyond: the sink)
+    uint32_t ksoff;     // K-scale load offset: key tid & 127 (the words are staged by threads 0..255: group A)
+    uint32_t kswoff;    // K-scale LDS write offset in a slot: word tid
     uint32_t ksshift;   // 0 for the words (tid < 128), 8 for the shifted copies (128 <= tid < 256)
     uint32_t tid, k_seq, ks_row, SK, lds;
     const uint8_t* vsb; // per-32-key V scales of this (batch, KV head) (extension; unused otherwise)
@@ -430,18 +433,6 @@ struct Stager {
         const uint32_t dst = w < 2u ? slot_base(lds, kLdsVs, slot, kVsSlot) + 256u * w : lds + kLdsVsSink + 256u * (w - 2u);
         dma4(vs_rsrc((key0 >> 5) + 2u * w, valid && w < 2u), dst, (lane >> 5) * vs_row + 4u * (lane & 31u), 0u);
     }
-    // Copy instruction i (0 .. 2 kN - 1: K chunk i / 2 for even i, V chunk i / 2 for odd i) of dma(), alone, so that a
-    // wave can spread a tile's copies between its MFMAs instead of waiting for the load path in one burst
-    __device__ __forceinline__ void dma_part(int i, uint32_t key0, bool valid, uint32_t slot) const {
-        const bool isv = (i & 1) != 0;
-        const uint8_t* base = isv ? vb : kb;
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(base + (size_t)key0 * k_seq, tile_bytes(key0, valid, k_seq, kD));
-        const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const uint32_t dst = slot_base(lds, isv ? kLdsV : kLdsK, slot, kTileBytes);
-        const uint32_t g = (uint32_t)(i >> 1) * (NT / 64) + w;
-        const uint32_t soff = __builtin_amdgcn_readfirstlane((uint32_t)(i >> 1) * (NT / 8) * k_seq);
-        dma16(r, dst + g * 1024u, dmaoff, soff);
-    }
     // Direct copy of tile [key0, key0 + 128)'s K-scale words (the words only, no shifted copy: readers use kscale_raw)
     // into K-scale slot `slot`: waves 0 and 1 copy 64 keys each (lane L: key 64 w + L, its 4 bytes at 4 (64 w + L));
     // the other waves copy from an empty resource into the sink, so that every wave issues one copy per tile.
@@ -460,8 +451,8 @@ struct Stager {
         ks_row = k_seq_ >> 5;
         SK = SK_;
         lds = lds_;
-        ksoff = tid < 256u ? (tid & 127u) * ks_row : 0x80000000u;
-        kswoff = tid < 256u ? tid * 4u : 0u;
+        ksoff = (tid & 127u) * ks_row;
+        kswoff = tid * 4u;
         ksshift = tid < 128u ? 0u : 8u;
     }
 
@@ -514,17 +505,44 @@ struct Stager {
         csstep = kTile * ks_row;
         woff = __builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
     }
-    // K's copies, then V's: alternating, or V first, cost the split-tile grids 1 % and 3 %
+    // K's copies, then V's: alternating, or V first, cost the split-tile grids 0.5 % and 3 %
     __device__ __forceinline__ void dma_next(uint32_t kslot, uint32_t vslot) {
         const __amdgpu_buffer_rsrc_t rk = make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0));
         const __amdgpu_buffer_rsrc_t rv = make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0));
         const uint32_t kbase = slot_base(lds + woff, kLdsK, kslot, kTileBytes), vbase = slot_base(lds + woff, kLdsV, vslot, kTileBytes);
 #pragma unroll
-        for (int i = 0; i < kN; ++i) dma16(rk, kbase + (uint32_t)i * (NT * 16u), dmaoff, __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
-#pragma unroll
-        for (int i = 0; i < kN; ++i) dma16(rv, vbase + (uint32_t)i * (NT * 16u), dmaoff, __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
+        for (int j = 0; j < 2 * kN; ++j) {
+            const int i = j % kN;
+            const bool isv = j >= kN;
+            dma16(isv ? rv : rk, (isv ? vbase : kbase) + (uint32_t)i * (NT * 16u), dmaoff,
+                  __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
+        }
         ck += cstep; cv += cstep;
         nk -= (int)cstep; nv -= (int)cstep;
+    }
+    // The 256-thread kernel spreads a tile's copies over its MFMAs: the resources and slots of the next tile (K and V of the
+    // same keys), and copy i of it (K chunk i / 2 for even i, V chunk i / 2 for odd i, then the K-scale words)
+    struct Next {
+        __amdgpu_buffer_rsrc_t k, v, ks;
+        uint32_t kbase, vbase, ksbase;
+    };
+    __device__ __forceinline__ Next next_tile(uint32_t slot) {
+        const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        Next n = {make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0)), make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0)),
+                  make_rsrc((const void*)(uintptr_t)cks, w < 2u ? (uint32_t)max(nks, 0) : 0u),
+                  slot_base(lds + woff, kLdsK, slot, kTileBytes), slot_base(lds + woff, kLdsV, slot, kTileBytes),
+                  w < 2u ? slot_base(lds, kLdsKs, slot, kKsSlot) + 256u * w : lds + kLdsKsDummy + 256u * ((w - 2u) & 3u)};
+        ck += cstep; cv += cstep; cks += csstep;
+        nk -= (int)cstep; nv -= (int)cstep; nks -= (int)csstep;
+        return n;
+    }
+    __device__ __forceinline__ void dma_next_part(const Next& n, int i) const {
+        if (i == 2 * kN) {
+            dma4(n.ks, n.ksbase, ksoff, 0u);
+            return;
+        }
+        dma16((i & 1) ? n.v : n.k, ((i & 1) ? n.vbase : n.kbase) + (uint32_t)(i >> 1) * (NT * 16u), dmaoff,
+              __builtin_amdgcn_readfirstlane((uint32_t)(i >> 1) * (NT / 8) * k_seq));
     }
     __device__ __forceinline__ void load_ks_next() {
         ksr = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc((const void*)(uintptr_t)cks, (uint32_t)max(nks, 0)), ksoff, 0, 0);
@@ -1628,6 +1646,7 @@ __device__ __forceinline__ void attend_single_wave(const Prm& p, uint32_t lds, u
         // VMEM operations per tile: the K and V copies, the K-scale copy and (extension) the V-scale copy
         constexpr int kOps = 2 * Stager<NT>::kN + 1 + (VS ? 1 : 0);
         FMHA_MARK(p, tblk, 2);
+        st.init_cursors(key_of(3), key_of(3), min(p.SK, ntiles * kTile));
         block_barrier_keep_dma<0, kOps>();   // tiles 0 and 1 have landed; tile 2's copies stay in flight
         FMHA_MARK(p, tblk, 3);
         v16f sa[4], sb[4];
@@ -1648,9 +1667,9 @@ __device__ __forceinline__ void attend_single_wave(const Prm& p, uint32_t lds, u
             uint32_t pw[4][4];
             // the copies of tile t+3, one instruction behind each of the phase's first MFMAs
             const uint32_t u = t + 3;
+            const typename Stager<NT>::Next next = st.next_tile(slot_of(u));
             auto copies = [&](int i) {
-                if (i < 2 * Stager<NT>::kN) st.dma_part(i, key_of(u), u < ntiles, slot_of(u));
-                else if (i == 2 * Stager<NT>::kN) st.dma_ks(key_of(u), u < ntiles, slot_of(u));
+                if (i <= 2 * Stager<NT>::kN) st.dma_next_part(next, i);
                 else if (VS && i == 2 * Stager<NT>::kN + 1) st.dma_vs(key_of(u), u < ntiles, slot_of(u));
             };
             float m = w.template m_phase_cv<LUT, VS, true>(rc, slot_of(t), slot_of(t + 1), sc, sn, pw, copies);
