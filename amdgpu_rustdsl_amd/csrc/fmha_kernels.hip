@@ -505,15 +505,17 @@ struct Stager {
         csstep = kTile * ks_row;
         woff = __builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
     }
-    // K's copies, then V's: alternating, or V first, cost the split-tile grids 0.5 % and 3 %
+    // K's copies, then V's: alternating, or V first, cost the split-tile grids 0.5 % and 3 %. ALT: alternating (the packed rows,
+    // which stream both from HBM)
+    template <bool ALT>
     __device__ __forceinline__ void dma_next(uint32_t kslot, uint32_t vslot) {
         const __amdgpu_buffer_rsrc_t rk = make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0));
         const __amdgpu_buffer_rsrc_t rv = make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0));
         const uint32_t kbase = slot_base(lds + woff, kLdsK, kslot, kTileBytes), vbase = slot_base(lds + woff, kLdsV, vslot, kTileBytes);
 #pragma unroll
         for (int j = 0; j < 2 * kN; ++j) {
-            const int i = j % kN;
-            const bool isv = j >= kN;
+            const int i = ALT ? j >> 1 : j % kN;
+            const bool isv = ALT ? (j & 1) != 0 : j >= kN;
             dma16(isv ? rv : rk, (isv ? vbase : kbase) + (uint32_t)i * (NT * 16u), dmaoff,
                   __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
         }
@@ -1498,12 +1500,10 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         const bool idle = PK && w.row0 >= p.pk_rows;
         if (idle) {
             for (uint32_t t = 0; t < ntiles; ++t) {
-                if (!GB) {
-                    st.store_ks(slot_of(t + 2));
-                    st.load_ks_next();
-                }
-                st.dma_next(slot_of(t + 3), slot_of(t + 2));
+                if (!GB) st.store_ks(slot_of(t + 2));
+                st.template dma_next<true>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                if (!GB) st.load_ks_next();
                 block_barrier_keep_dma<0, kDmaOps>();
             }
         }
@@ -1517,10 +1517,12 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
             typename Wave<NT>::QkPre pre;
             // V(t)'s copies: K tile t+3 and V tile t+2 (and the per-32-key V scales), the K-scale words of tile t+3
             auto copies = [&](uint32_t t) {
-                // the words first: their store in V(t + 1) then waits for the copies of V(t) in flight longer
-                if (!GB) st.load_ks_next();
-                st.dma_next(slot_of(t + 3), slot_of(t + 2));
+                // the K-scale words before the copies; behind them in the packed rows, where the copies come from HBM and
+                // should go out first (B1 H8 S128 SK16000, with the order of the copies, 16.3 -> 16.0 us per call)
+                if (!GB && !PK) st.load_ks_next();
+                st.template dma_next<PK>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
+                if (!GB && PK) st.load_ks_next();
             };
             auto v_phase = [&](uint32_t t, uint32_t (&pw)[NA][4], bool last) {
                 FMHA_SETPRIO(0);

@@ -211,7 +211,8 @@ int fmha_mxfp8_select_path(int64_t B, int64_t H, int64_t S, int64_t SK, int* spl
  * blocks of 512 threads, the two wave groups splitting each tile's keys and merging at the end), else 0. t128: at
  * least 7 key tiles (4 with `causal`); below that the 256-thread fmha_fwd_hd128_mxfp8_v3_t128, which is faster there
  * and keeps the reference's order. vs128: the same, and a 256-row grid of at most 128 blocks unless `causal` (the
- * 128-row grid's causal q-tile pairing); such a half-chip grid below the threshold runs on the 256-thread t128
+ * 128-row grid's causal q-tile pairing; not for S = SK with more 256-row blocks than CUs, which run the 256-row kernel
+ * with the heaviest query tiles first); such a half-chip grid below the threshold runs on the 256-thread t128
  * kernel. The split-tile order rounds differently from the reference's single stream per row; the path and its
  * recipe are the reference's. */
 int fmha_mxfp8_uses_split_tiles(int path, int64_t B, int64_t H, int64_t S, int64_t SK, int causal);
@@ -311,6 +312,7 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
  * KV head are packed into one block's rows, and the key range is spread over several blocks whose f32 partials a merge
  * kernel adds up. Every share starts from the softmax reference of the whole range's first tile, so P is quantised as
  * the unsplit kernel does; the sums are taken in another order. Without enough workspace the path's own kernel runs.
+ * A 256-row grid one round of CUs and a bit large may use it in the same way for the blocks past the last whole round.
  * fmha_mxfp8_auto_workspace_bytes: the workspace the call can use (one slot; 0 when it needs none). */
 int fmha_fwd_hd128_mxfp8_auto_ws(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes,
                                  void* stream, int* path_out, int* splits_out, char* err, size_t errlen);
