@@ -36,6 +36,7 @@
 
 #include "../../include/fmha_mxfp8.h"
 #include "pre_args.h"
+#include "tile_extent.h"
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -439,7 +440,7 @@ struct Stager {
     __device__ __forceinline__ void dma_ks(uint32_t key0, bool valid, uint32_t slot) const {
         const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63u;
         const uint32_t dst = w < 2u ? slot_base(lds, kLdsKs, slot, kKsSlot) + 256u * w : lds + kLdsKsDummy + 256u * ((w - 2u) & 3u);
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(ksb + (size_t)key0 * ks_row, tile_bytes(key0, valid && w < 2u, ks_row, 4));
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(ksb + (size_t)key0 * ks_row, tile_bytes(key0, valid && w < 2u, ks_row));
         dma4(r, dst, (64u * (w & 1u) + lane) * ks_row, 0u);
     }
 
@@ -458,10 +459,9 @@ struct Stager {
 
     uint32_t ksr;   // the K-scale word of the next tile, loaded in one VALU phase and stored in the next
 
-    // resource size of a tile starting at key0: rem = SK - 1 - key0 keys follow the first, rem stride + tail bytes
-    __device__ __forceinline__ uint32_t tile_bytes(uint32_t key0, bool valid, uint32_t stride, int tail) const {
-        const int rem = __builtin_amdgcn_readfirstlane((int)SK - 1 - (int)key0);
-        return valid ? (uint32_t)max(rem * (int)stride + tail, 0) : 0u;
+    // resource size of the tile starting at key0
+    __device__ __forceinline__ uint32_t tile_bytes(uint32_t key0, bool valid, uint32_t stride) const {
+        return valid ? tile_extent(__builtin_amdgcn_readfirstlane((int)(SK - key0)), stride) : 0u;
     }
 
     // Direct HBM -> LDS copies (buffer_load_dwordx4 ... lds), no VGPR round trip: copy i of wave w writes LDS rows
@@ -475,8 +475,8 @@ struct Stager {
         dmaoff = row * k_seq + (((tid & 7u) ^ swz(row)) << 4);
     }
     __device__ __forceinline__ void dma(uint32_t kkey0, bool kvalid, uint32_t kslot, uint32_t vkey0, bool vvalid, uint32_t vslot) const {
-        const __amdgpu_buffer_rsrc_t rk = make_rsrc(kb + (size_t)kkey0 * k_seq, tile_bytes(kkey0, kvalid, k_seq, kD));
-        const __amdgpu_buffer_rsrc_t rv = make_rsrc(vb + (size_t)vkey0 * k_seq, tile_bytes(vkey0, vvalid, k_seq, kD));
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(kb + (size_t)kkey0 * k_seq, tile_bytes(kkey0, kvalid, k_seq));
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(vb + (size_t)vkey0 * k_seq, tile_bytes(vkey0, vvalid, k_seq));
         const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
         const uint32_t kbase = slot_base(lds, kLdsK, kslot, kTileBytes), vbase = slot_base(lds, kLdsV, vslot, kTileBytes);
 #pragma unroll
@@ -487,30 +487,30 @@ struct Stager {
             dma16(rv, vbase + g * 1024u, dmaoff, soff);
         }
     }
-    // The loop's copies as running state: base and remaining bytes of the next K, V and K-scale tiles, advanced by one tile per
-    // call. `limit` ends the block's last tile, so a tile past it finds no bytes left (its size is at most -stride + one
-    // row's bytes, never positive) and needs no test. From the tile index, the three resources took ~50 scalar
-    // instructions in a row per VALU phase, during which the wave converted nothing.
+    // The loop's copies as running state: the bases and sizes of the next K, V and K-scale tiles, advanced by one tile per VALU
+    // phase. `limit` ends the block's last tile, so a tile past it has no rows left and needs no test. From the tile
+    // index, the three resources took ~50 scalar instructions in a row per VALU phase, during which the wave converted
+    // nothing. The K-scale rows are k_seq / 32 bytes of the K tile's rows.
     uint64_t ck, cv, cks;
-    int nk, nv, nks;
+    TileSizes sizes;
     uint32_t cstep, csstep, woff;
     __device__ __forceinline__ void init_cursors(uint32_t kkey, uint32_t vkey, uint32_t limit) {
         ck = (uint64_t)(uintptr_t)kb + (uint64_t)kkey * k_seq;
         cv = (uint64_t)(uintptr_t)vb + (uint64_t)vkey * k_seq;
         cks = (uint64_t)(uintptr_t)ksb + (uint64_t)kkey * ks_row;
-        nk = ((int)limit - 1 - (int)kkey) * (int)k_seq + kD;
-        nv = ((int)limit - 1 - (int)vkey) * (int)k_seq + kD;
-        nks = ((int)limit - 1 - (int)kkey) * (int)ks_row + 4;
+        sizes.init(limit, kkey, k_seq);
         cstep = kTile * k_seq;
         csstep = kTile * ks_row;
         woff = __builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
     }
+    // one VALU phase on: V one tile behind K (the ping-pong kernels)
+    __device__ __forceinline__ void advance() { sizes.template advance<1>(k_seq); }
     // K's copies, then V's: alternating, or V first, cost the split-tile grids 0.5 % and 3 %. ALT: alternating (the packed rows,
     // which stream both from HBM)
     template <bool ALT>
     __device__ __forceinline__ void dma_next(uint32_t kslot, uint32_t vslot) {
-        const __amdgpu_buffer_rsrc_t rk = make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0));
-        const __amdgpu_buffer_rsrc_t rv = make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0));
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc((const void*)(uintptr_t)ck, sizes.k);
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc((const void*)(uintptr_t)cv, sizes.v);
         const uint32_t kbase = slot_base(lds + woff, kLdsK, kslot, kTileBytes), vbase = slot_base(lds + woff, kLdsV, vslot, kTileBytes);
 #pragma unroll
         for (int j = 0; j < 2 * kN; ++j) {
@@ -520,7 +520,6 @@ struct Stager {
                   __builtin_amdgcn_readfirstlane((uint32_t)i * (NT / 8) * k_seq));
         }
         ck += cstep; cv += cstep;
-        nk -= (int)cstep; nv -= (int)cstep;
     }
     // The 256-thread kernel spreads a tile's copies over its MFMAs: the resources and slots of the next tile (K and V of the
     // same keys), and copy i of it (K chunk i / 2 for even i, V chunk i / 2 for odd i, then the K-scale words)
@@ -530,12 +529,12 @@ struct Stager {
     };
     __device__ __forceinline__ Next next_tile(uint32_t slot) {
         const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
-        Next n = {make_rsrc((const void*)(uintptr_t)ck, (uint32_t)max(nk, 0)), make_rsrc((const void*)(uintptr_t)cv, (uint32_t)max(nv, 0)),
-                  make_rsrc((const void*)(uintptr_t)cks, w < 2u ? (uint32_t)max(nks, 0) : 0u),
+        sizes.template advance<0>(k_seq);
+        Next n = {make_rsrc((const void*)(uintptr_t)ck, sizes.k), make_rsrc((const void*)(uintptr_t)cv, sizes.v),
+                  make_rsrc((const void*)(uintptr_t)cks, w < 2u ? sizes.k >> 5 : 0u),
                   slot_base(lds + woff, kLdsK, slot, kTileBytes), slot_base(lds + woff, kLdsV, slot, kTileBytes),
                   w < 2u ? slot_base(lds, kLdsKs, slot, kKsSlot) + 256u * w : lds + kLdsKsDummy + 256u * ((w - 2u) & 3u)};
         ck += cstep; cv += cstep; cks += csstep;
-        nk -= (int)cstep; nv -= (int)cstep; nks -= (int)csstep;
         return n;
     }
     __device__ __forceinline__ void dma_next_part(const Next& n, int i) const {
@@ -547,19 +546,18 @@ struct Stager {
               __builtin_amdgcn_readfirstlane((uint32_t)(i >> 1) * (NT / 8) * k_seq));
     }
     __device__ __forceinline__ void load_ks_next() {
-        ksr = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc((const void*)(uintptr_t)cks, (uint32_t)max(nks, 0)), ksoff, 0, 0);
+        ksr = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc((const void*)(uintptr_t)cks, sizes.k >> 5), ksoff, 0, 0);
         cks += csstep;
-        nks -= (int)csstep;
     }
     // The K-scale words of tile [kkey0, kkey0 + 128) into ksr (register-staged: the upper k-group's copy is shifted)
     __device__ __forceinline__ void load_ks(uint32_t kkey0, bool kvalid) {
-        const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksb + (size_t)kkey0 * ks_row, tile_bytes(kkey0, kvalid, ks_row, 4));
+        const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksb + (size_t)kkey0 * ks_row, tile_bytes(kkey0, kvalid, ks_row));
         ksr = __builtin_amdgcn_raw_buffer_load_b32(rks, ksoff, 0, 0);
     }
     __device__ __forceinline__ void store_ks(uint32_t kslot) const { store_ks_word(ksr, kslot); }
     // the same through a register the caller holds (the prologue loads several tiles' words at once)
     __device__ __forceinline__ uint32_t ks_word(uint32_t kkey0, bool kvalid) const {
-        const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksb + (size_t)kkey0 * ks_row, tile_bytes(kkey0, kvalid, ks_row, 4));
+        const __amdgpu_buffer_rsrc_t rks = make_rsrc(ksb + (size_t)kkey0 * ks_row, tile_bytes(kkey0, kvalid, ks_row));
         return __builtin_amdgcn_raw_buffer_load_b32(rks, ksoff, 0, 0);
     }
     __device__ __forceinline__ void store_ks_word(uint32_t word, uint32_t kslot) const {
@@ -1501,6 +1499,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         if (idle) {
             for (uint32_t t = 0; t < ntiles; ++t) {
                 if (!GB) st.store_ks(slot_of(t + 2));
+                st.advance();
                 st.template dma_next<true>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
                 if (!GB) st.load_ks_next();
@@ -1519,6 +1518,7 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
             auto copies = [&](uint32_t t) {
                 // the K-scale words before the copies; behind them in the packed rows, where the copies come from HBM and
                 // should go out first (B1 H8 S128 SK16000, with the order of the copies, 16.3 -> 16.0 us per call)
+                st.advance();
                 if (!GB && !PK) st.load_ks_next();
                 st.template dma_next<PK>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
