@@ -5,6 +5,7 @@
 // is not a plain torch.Tensor (subclasses, tracing and fake tensors); ops.py then runs its Python path, which raises the
 // error or serves the call. Building the ctypes structures and reading the tensors from Python cost 17 us per attention
 // call and ~12 us per quantiser call, more than most kernels take; here a call costs its launches.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
@@ -13,15 +14,12 @@
 #include <c10/hip/HIPFunctions.h>
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <exception>
 #include <map>
-#include <memory>
-#include <mutex>
+#include <optional>
 #include <utility>
-#include <vector>
 
 #include "../../include/fmha_mxfp8.h"
 #include "../../include/mxfp8_quant.h"
@@ -56,41 +54,67 @@ struct OnDevice {
     int prev, dev;
 };
 
-// The attention's workspace per (device, stream), grown on demand, with the turn word of its slots. `mu` orders the calls
-// of several threads on one stream, each of which launches kernels that hand partials to the next. A buffer that a stream
-// capture has recorded (the graph may be replayed at any time), or that was used on another stream than the allocator
-// knows it by, is kept when the workspace grows past it; growth at least doubles, so the kept ones are smaller together.
-struct Workspace {
-    std::mutex mu;
-    at::Tensor buf;
-    uint32_t turn = 0;
-    bool keep = false;
-    std::vector<at::Tensor> kept;
+// An allocation by this thread is no part of any capture, and does not disturb one that another thread has under way.
+struct RelaxedCapture {
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
 };
-std::map<std::pair<int, uintptr_t>, std::unique_ptr<Workspace>>& workspaces() {
-    static auto* m = new std::map<std::pair<int, uintptr_t>, std::unique_ptr<Workspace>>;   // outlives the allocator's teardown
-    return *m;
+
+// Whether the allocation lies in a pool that torch keeps apart from the ordinary ones (a graph's, while torch captures it).
+bool in_private_pool(const void* ptr) {
+    const size_t a = (size_t)(uintptr_t)ptr;
+    for (const auto& s : c10::hip::HIPCachingAllocator::get()->snapshot().segments)
+        if (a >= s.address && a < s.address + s.total_size) return s.owner_private_pool_id.first != 0 || s.owner_private_pool_id.second != 0;
+    return false;
 }
 
-// Called with the GIL held (which guards the map).
-Workspace& workspace(int dev, void* stream, size_t nbytes, const at::Tensor& like) {
-    std::unique_ptr<Workspace>& w = workspaces()[{dev, (uintptr_t)stream}];
-    if (!w) w = std::make_unique<Workspace>();
-    std::lock_guard<std::mutex> lk(w->mu);
-    const size_t have = w->buf.defined() ? (size_t)w->buf.numel() : 0;
-    if (have < nbytes) {
-        at::Tensor grown = at::empty({(int64_t)std::max(nbytes, w->keep ? 2 * have : 0)}, like.options().dtype(at::kByte));
-        if (have && w->keep) w->kept.push_back(std::move(w->buf));
-        w->buf = std::move(grown);
-        w->keep = stream != c10::hip::getCurrentHIPStreamMasqueradingAsCUDA((c10::DeviceIndex)dev).stream();
-    }
-    if (!w->keep) {
+// The attention's workspace: memory of one call, from torch's caching allocator by the call's stream, so that its earlier users are
+// work on that stream, and so are its next ones. Nothing is kept between calls and no two callers share a buffer. (The
+// allocator hands consecutive calls of a stream the same block, whose slots they then take in turn.)
+// Under a capture by torch the block is the graph's own, from its pool. Under any other capture nobody owns the memory that
+// the graph will use on each replay, so it is allocated for that capture and stream, and stays allocated.
+class Scratch {
+  public:
+    // Throws torch's out-of-memory error.
+    Scratch(size_t bytes, hipStream_t stream) {
+        RelaxedCapture relaxed;
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) (void)hipGetLastError();   // (the legacy stream, while another captures)
-        else w->keep = st != hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        if (hipStreamGetCaptureInfo(stream, &st, &id) != hipSuccess) {   // (the legacy stream, while another captures)
+            (void)hipGetLastError();
+            st = hipStreamCaptureStatusNone;
+        }
+        own_ = c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, stream);
+        ptr = own_;
+        if (st == hipStreamCaptureStatusActive && !in_private_pool(own_)) {
+            release();
+            ptr = of_capture(id, stream, bytes);
+        }
     }
-    return *w;
-}
+    ~Scratch() { release(); }
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+    void* ptr = nullptr;
+
+  private:
+    void release() {
+        if (own_) c10::hip::HIPCachingAllocator::raw_delete(own_);
+        own_ = nullptr;
+    }
+    // Called with the GIL held (which guards the map).
+    static void* of_capture(unsigned long long id, hipStream_t stream, size_t bytes) {
+        static auto* held = new std::map<std::pair<unsigned long long, hipStream_t>, std::pair<void*, size_t>>;
+        auto& h = (*held)[{id, stream}];
+        if (h.second < bytes) {
+            void* p = nullptr;
+            C10_HIP_CHECK(hipMalloc(&p, bytes));
+            h = {p, bytes};
+        }
+        return h.first;
+    }
+    void* own_ = nullptr;
+};
 
 void* stream_of(PyObject* o, int dev, bool& ok) {
     if (o == Py_None) return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA((c10::DeviceIndex)dev).stream();
@@ -118,6 +142,36 @@ PyObject* raise_code(int rc, const char* msg) {
 }
 
 PyObject* decline() { Py_RETURN_NONE; }
+
+// The one-call entry with its workspace -> (path, splits, partials). Called with the GIL held.
+PyObject* run_params(fmha_mxfp8_params& p, int dev, void* stream) {
+    static thread_local uint32_t turn = 0;   // which slots: any will do
+    int32_t parts = 0;
+    int path = -1, splits = 0, rc;
+    p.partials_out = &parts;
+    p.ws_turn = &turn;
+    char err[512] = "";
+    {
+        OnDevice on(dev);
+        // room for the entry's workspace slots (consecutive calls then write partials the previous combine did not just
+        // read), unless that would take more than 512 MiB
+        size_t bytes = fmha_mxfp8_auto_workspace_bytes(&p);
+        const size_t slotted = FMHA_WORKSPACE_SLOTS * ((bytes + 255) / 256 * 256);
+        if (slotted <= (512u << 20)) bytes = slotted;
+        std::optional<Scratch> ws;
+        if (bytes) ws.emplace(bytes, (hipStream_t)stream);
+        Py_BEGIN_ALLOW_THREADS
+        rc = fmha_fwd_hd128_mxfp8_auto_ws(&p, ws ? ws->ptr : nullptr, bytes, stream, &path, &splits, err, sizeof(err));
+        Py_END_ALLOW_THREADS
+    }
+    if (rc != FMHA_OK) return raise_code(rc, err);
+    PyObject* r = PyTuple_New(3);
+    if (!r) return nullptr;
+    PyTuple_SET_ITEM(r, 0, PyLong_FromLong(path));
+    PyTuple_SET_ITEM(r, 1, PyLong_FromLong(splits));
+    PyTuple_SET_ITEM(r, 2, PyLong_FromLong(parts));
+    return r;
+}
 
 // attend(q, k, v, q_scale, k_scale, v_scale, out, lse, path, splits, causal, f32_partials, softmax_scale, no_check,
 //        causal_pair, kv_fill, stream) -> (path, splits, partials), or None
@@ -165,41 +219,7 @@ PyObject* attend_impl(PyObject* const* a, Py_ssize_t n) {
     p.v_seq32 = seq32 ? 1 : 0;
     p.softmax_scale = (float)scale;
     p.no_check = iv[13]; p.causal_pair = iv[14]; p.kv_fill = iv[15];
-    int32_t parts = 0;
-    int path = -1, splits = 0, rc;
-    p.partials_out = &parts;
-    char err[512] = "";
-    {
-        OnDevice on(dev);
-        // room for the entry's workspace slots (consecutive calls then write partials the previous combine did not just
-        // read), unless that would take more than 512 MiB
-        size_t bytes = fmha_mxfp8_auto_workspace_bytes(&p);
-        const size_t slotted = FMHA_WORKSPACE_SLOTS * ((bytes + 255) / 256 * 256);
-        if (slotted <= (512u << 20)) bytes = slotted;
-        if (bytes) {
-            Workspace& w = workspace(dev, stream, bytes, q);
-            const at::Tensor hold = w.buf;   // another thread may grow the workspace while this one has released the GIL
-            void* ws = hold.data_ptr();
-            p.ws_turn = &w.turn;
-            Py_BEGIN_ALLOW_THREADS
-            {   // (released before the GIL is taken again: a thread that holds the GIL may wait for it)
-                std::lock_guard<std::mutex> lk(w.mu);
-                rc = fmha_fwd_hd128_mxfp8_auto_ws(&p, ws, bytes, stream, &path, &splits, err, sizeof(err));
-            }
-            Py_END_ALLOW_THREADS
-        } else {
-            Py_BEGIN_ALLOW_THREADS
-            rc = fmha_fwd_hd128_mxfp8_auto_ws(&p, nullptr, 0, stream, &path, &splits, err, sizeof(err));
-            Py_END_ALLOW_THREADS
-        }
-    }
-    if (rc != FMHA_OK) return raise_code(rc, err);
-    PyObject* r = PyTuple_New(3);
-    if (!r) return nullptr;
-    PyTuple_SET_ITEM(r, 0, PyLong_FromLong(path));
-    PyTuple_SET_ITEM(r, 1, PyLong_FromLong(splits));
-    PyTuple_SET_ITEM(r, 2, PyLong_FromLong(parts));
-    return r;
+    return run_params(p, dev, stream);
 }
 
 // A bf16 tensor the quantisers can read as it is.
@@ -344,6 +364,28 @@ PyObject* guarded(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
 }
 
+// run(params address, device, stream) -> (path, splits, partials): attend's call for params that Python filled
+PyObject* run_impl(PyObject* const* a, Py_ssize_t n) {
+    if (n != 3) return decline();
+    bool ok = true;
+    const int dev = (int)PyLong_AsLong(a[1]);
+    fmha_mxfp8_params p;
+    const void* src = PyLong_AsVoidPtr(a[0]);
+    if (PyErr_Occurred()) return nullptr;
+    std::memcpy(&p, src, sizeof(p));
+    void* stream = stream_of(a[2], dev, ok);
+    if (!ok) {
+        PyErr_SetString(PyExc_TypeError, "stream: expected a hipStream_t handle");
+        return nullptr;
+    }
+    try {
+        return run_params(p, dev, stream);
+    } catch (const std::exception&) {   // (out of memory)
+        torch::translate_exception_to_python(std::current_exception());
+        return nullptr;
+    }
+}
+
 // set_error(cls): the exception class of failing C calls (lib.FmhaError: code, message)
 PyObject* set_error(PyObject*, PyObject* cls) {
     Py_INCREF(cls);
@@ -356,6 +398,7 @@ PyMethodDef methods[] = {
     {"quantize_rows", (PyCFunction)(void*)guarded<quantize_rows_impl>, METH_FASTCALL, nullptr},
     {"quantize_v", (PyCFunction)(void*)guarded<quantize_v_impl>, METH_FASTCALL, nullptr},
     {"quantize_qkv", (PyCFunction)(void*)guarded<quantize_qkv_impl>, METH_FASTCALL, nullptr},
+    {"run", (PyCFunction)(void*)guarded<run_impl>, METH_FASTCALL, nullptr},
     {"set_error", set_error, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

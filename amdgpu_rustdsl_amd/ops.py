@@ -20,6 +20,7 @@ if not os.path.exists(_OPS_PATH):
 _loader = importlib.machinery.ExtensionFileLoader("_fmha_ops", _OPS_PATH)
 _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fmha_ops", _loader))
 _native.set_error(lib.FmhaError)
+_run = _native.run   # the one-call entry with its workspace, for params filled here
 
 D = 128
 FMHA_VS128 = "fmha_fwd_hd128_mxfp8_v3_vs128"
@@ -57,17 +58,9 @@ _PATH_CODES = {"auto": -1, "vs128": lib.PATH_VS128, "t128": lib.PATH_T128, "kvsp
 _PAIR_MODES = {"auto": 0, True: 1, False: 2}
 _PARTIAL_FORMATS = {"fp16": 0, "fp32": 1}
 
-_workspace = {}
 
-
-def _ws(device, stream, nbytes):
-    """Persistent KV-split workspace per (device, stream), grown on demand (ops.py:73-85), with the turn word of its
-    slots (host memory, owned by this op: calls on one stream take the slots in turn)."""
-    key = (device, stream)
-    ent = _workspace.get(key)
-    if ent is None or ent[0].numel() < nbytes:
-        ent = _workspace[key] = (torch.empty(nbytes, dtype=torch.uint8, device=device), ctypes.c_uint32(0))
-    return ent
+def _ran(r):
+    return lib.Ran(lib.PATH_NAMES[r[0]], r[1], r[2])
 
 
 def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", splits=None, specialize=True, stream=None, check=True,
@@ -111,7 +104,7 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
                                  _PARTIAL_FORMATS[partials], softmax_scale or 0.0, 0 if check else 1, _PAIR_MODES[causal_pair],
                                  0 if kv_fill else 1, stream)
             if ran is not None:
-                return lib.Ran(lib.PATH_NAMES[ran[0]], ran[1], ran[2])
+                return _ran(ran)
     pair_modes = _PAIR_MODES
     if causal_pair not in pair_modes:
         raise ValueError(f"fmha_fwd_mxfp8: causal_pair must be 'auto', True or False, got {causal_pair!r}")
@@ -163,20 +156,7 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
         if not float(softmax_scale) > 0.0:
             raise ValueError(f"fmha_fwd_mxfp8: softmax_scale must be positive, got {softmax_scale!r}")
         p.softmax_scale = float(softmax_scale)
-    # the workspace: the KV split's partials (the chunks, each spread over up to 8 blocks when the grid would leave CUs
-    # idle), or those of a short query range's shares
-    ws, ws_bytes = None, lib.auto_workspace_bytes(p)
-    if ws_bytes:
-        # room for the entry's workspace slots (consecutive calls then write partials the previous combine did not
-        # just read), unless that would take more than 512 MiB
-        slotted = lib.WORKSPACE_SLOTS * ((ws_bytes + 255) // 256 * 256)
-        if slotted <= 512 << 20:
-            ws_bytes = slotted
-        buf, turn = _ws(dev, st, ws_bytes)
-        ws = buf.data_ptr()
-        p.ws_turn = ctypes.pointer(turn)
-    with torch.cuda.device(dev):
-        return lib.run_auto_ws(p, ws, ws_bytes, st)
+    return _ran(_run(ctypes.addressof(p), dev.index, st))
 
 
 def alloc_scales(B, rows, H, device, fill=0):

@@ -1,5 +1,6 @@
 """The native form of the torch-facing calls (csrc/ops_binding.cpp) against their Python form, and the workspace that it
-keeps: other streams, threads on one stream, graphs that outlive its growth."""
+takes: other streams, threads on one stream, graphs."""
+import ctypes
 import threading
 
 import pytest
@@ -138,3 +139,117 @@ def test_graph_survives_workspace_growth(gpu):
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
         trash[0].add_(1)
     del trash
+
+
+def _eager(cases):
+    want = []
+    for t in cases:
+        o = _out(t)
+        ops.fmha_fwd_mxfp8(*t, o)
+        want.append(o)
+    torch.cuda.synchronize()
+    return want
+
+
+def test_calls_keep_no_memory(gpu):
+    """A call gives its workspace back: on streams that were never used, eager, and around a capture."""
+    t = _case(gpu, 2, 8, 2, 4, 3000, seed=1)
+    out = _out(t)
+    ops.fmha_fwd_mxfp8(*t, out)
+    torch.cuda.synchronize()
+    s, graph = torch.cuda.Stream(gpu), torch.cuda.CUDAGraph()
+    before = torch.cuda.memory_allocated(gpu)
+    with torch.cuda.stream(s):
+        ops.fmha_fwd_mxfp8(*t, out)
+    ops.fmha_fwd_mxfp8(*t, out, stream=torch.cuda.Stream(gpu).cuda_stream)
+    with torch.cuda.graph(graph):
+        ops.fmha_fwd_mxfp8(*t, out)
+    torch.cuda.synchronize()
+    # (torch keeps 1 KiB of random state for a graph; one partial of this call's 64 rows takes 33 KB)
+    assert torch.cuda.memory_allocated(gpu) - before < 4096
+
+
+def test_graphs_of_one_capture_stream_replay_together(gpu):
+    """Two graphs captured one after the other, each of more calls than the workspace has slots, replayed on two streams at
+    once, with eager calls on the capture stream between: the memory of each is its own."""
+    cases = [_case(gpu, 8, 32, 8, 1, 2048, seed=i) for i in range(12)]
+    want = _eager(cases)
+    s = torch.cuda.Stream(gpu)
+    graphs, outs = [], [_out(t) for t in cases]
+    for half in (0, 6):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            for i in range(half, half + 6):
+                ops.fmha_fwd_mxfp8(*cases[i], outs[i])
+        graphs.append(graph)
+    streams = [torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)]
+    extra = _out(cases[0])
+    for _ in range(10):
+        for o in outs:
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for st, graph in zip(streams, graphs):
+            with torch.cuda.stream(st):
+                graph.replay()
+        with torch.cuda.stream(s):
+            ops.fmha_fwd_mxfp8(*cases[0], extra)
+        torch.cuda.synchronize()
+        for i in range(12):
+            assert torch.equal(outs[i].view(torch.int16), want[i].view(torch.int16)), i
+        assert torch.equal(extra.view(torch.int16), want[0].view(torch.int16))
+
+
+def test_stream_argument_takes_no_memory_in_use(gpu):
+    """A call on another stream than torch's current one: memory that pending work of the current stream still writes is not
+    its workspace."""
+    t = _case(gpu, 2, 8, 2, 4, 3000, seed=3)
+    (want,) = _eager([t])
+    s, out = torch.cuda.Stream(gpu), _out(t)
+    torch.cuda.synchronize()
+    for size in (1 << 22, 1 << 24, 1 << 26):
+        torch.cuda.empty_cache()
+        blocks = [torch.empty(size, dtype=torch.uint8, device=gpu) for _ in range(4)]
+        torch.cuda._sleep(20_000_000)   # (a spin of about 10 ms)
+        for x in blocks:
+            x.fill_(0xff)
+        del blocks, x
+        ops.fmha_fwd_mxfp8(*t, out, stream=s.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), size
+
+
+def _hip():
+    """The HIP runtime that this process runs on."""
+    with open("/proc/self/maps") as f:
+        path = next(x.split()[-1] for x in f if "libamdhip64" in x)
+    return ctypes.CDLL(path)
+
+
+def test_capture_that_torch_does_not_know(gpu):
+    """A graph captured through HIP itself: its workspace is nobody else's when it is replayed."""
+    t, other = _case(gpu, 2, 8, 2, 4, 3000, seed=4), _case(gpu, 2, 8, 2, 4, 3000, seed=5)
+    want, want_other = _eager([t, other])
+    hip, s = _hip(), torch.cuda.Stream(gpu)
+    handle, graph, ex = ctypes.c_void_p(s.cuda_stream), ctypes.c_void_p(), ctypes.c_void_p()
+    out, o2 = _out(t), _out(other)
+    torch.cuda.synchronize()
+    assert hip.hipStreamBeginCapture(handle, 1) == 0   # thread-local mode
+    for _ in range(5):
+        ops.fmha_fwd_mxfp8(*t, out, stream=s.cuda_stream)
+    assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    torch.cuda.empty_cache()
+    trash = [torch.full((1 << 22,), 0xff, dtype=torch.uint8, device=gpu) for _ in range(8)]
+    for _ in range(3):
+        out.fill_(float("nan"))
+        o2.fill_(float("nan"))
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(ex, handle) == 0
+        with torch.cuda.stream(s):
+            ops.fmha_fwd_mxfp8(*other, o2)
+        ops.fmha_fwd_mxfp8(*other, o2)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(o2.view(torch.int16), want_other.view(torch.int16))
+        assert all(bool((x == 0xff).all()) for x in trash)
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
