@@ -108,7 +108,10 @@ class Scratch {
         auto& h = (*held)[{id, stream}];
         if (h.second < bytes) {
             void* p = nullptr;
-            C10_HIP_CHECK(hipMalloc(&p, bytes));
+            if (hipMalloc(&p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                TORCH_CHECK_WITH(OutOfMemoryError, false, "no memory for a captured call's workspace (", bytes, " bytes)");
+            }
             h = {p, bytes};
         }
         return h.first;
@@ -155,14 +158,26 @@ PyObject* run_params(fmha_mxfp8_params& p, int dev, void* stream) {
         OnDevice on(dev);
         // room for the entry's workspace slots (consecutive calls then write partials the previous combine did not just
         // read), unless that would take more than 512 MiB
-        size_t bytes = fmha_mxfp8_auto_workspace_bytes(&p);
+        const size_t one = fmha_mxfp8_auto_workspace_bytes(&p);
+        size_t bytes = one;
         const size_t slotted = FMHA_WORKSPACE_SLOTS * ((bytes + 255) / 256 * 256);
         if (slotted <= (512u << 20)) bytes = slotted;
         std::optional<Scratch> ws;
-        if (bytes) ws.emplace(bytes, (hipStream_t)stream);
+        std::exception_ptr oom;
+        for (const size_t n : {bytes, one}) {
+            if (ws || !n || (oom && n == bytes)) continue;
+            try {
+                ws.emplace(n, (hipStream_t)stream);
+                bytes = n;
+            } catch (const c10::OutOfMemoryError&) {
+                oom = std::current_exception();
+            }
+        }
+        if (!ws) bytes = 0;   // the full-sequence paths then run their own kernels, which take none
         Py_BEGIN_ALLOW_THREADS
         rc = fmha_fwd_hd128_mxfp8_auto_ws(&p, ws ? ws->ptr : nullptr, bytes, stream, &path, &splits, err, sizeof(err));
         Py_END_ALLOW_THREADS
+        if (rc == FMHA_ERR_WORKSPACE && oom) std::rethrow_exception(oom);
     }
     if (rc != FMHA_OK) return raise_code(rc, err);
     PyObject* r = PyTuple_New(3);

@@ -253,3 +253,39 @@ def test_capture_that_torch_does_not_know(gpu):
         assert torch.equal(o2.view(torch.int16), want_other.view(torch.int16))
         assert all(bool((x == 0xff).all()) for x in trash)
     assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+def test_without_memory_for_a_workspace(gpu):
+    """A full-sequence call takes a workspace where it can have one; where it can't, its own kernel runs without, as it does for
+    callers that pass none. The KV split needs its partials and says so."""
+    B, H, S = 3, 8, 3001
+    t, kv = _case(gpu, B, H, H, S, S), _case(gpu, 1, 8, 8, 2048, 2048)
+    out, own, kv_out = _out(t), _out(t), _out(kv)
+    p = lib.Params()
+    p.o, p.q, p.k, p.v = (x.data_ptr() for x in (own, *t[:3]))
+    p.q_descale, p.k_descale, p.v_descale = (x.data_ptr() for x in t[3:])
+    p.B, p.H, p.HK, p.S, p.SK, p.path, p.no_check = B, H, H, S, S, -1, 1
+    need = lib.auto_workspace_bytes(p)
+    if not need:
+        pytest.skip("this device's CU count splits no blocks of the shape")
+    lib.run_auto(p, None, 0, torch.cuda.current_stream(gpu).cuda_stream)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    spare = []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(gpu) / total, gpu)
+        with pytest.raises(torch.OutOfMemoryError):   # what the live tensors' segments have left
+            while True:
+                spare.append(torch.empty(1 << 20, dtype=torch.uint8, device=gpu))
+        ops.fmha_fwd_mxfp8(*t, out)
+        torch.cuda.synchronize()
+        with pytest.raises(torch.OutOfMemoryError):
+            ops.fmha_fwd_mxfp8(*kv, kv_out)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    assert torch.equal(out.view(torch.int16), own.view(torch.int16))
+    del spare
+    ops.fmha_fwd_mxfp8(*kv, kv_out)
+    torch.cuda.synchronize()
+    assert torch.isfinite(kv_out.float()).all()
