@@ -74,20 +74,36 @@ bool in_private_pool(const void* ptr) {
 // allocator hands consecutive calls of a stream the same block, whose slots they then take in turn.)
 // Under a capture by torch the block is the graph's own, from its pool. Under any other capture nobody owns the memory that
 // the graph will use on each replay, so it is allocated for that capture and stream, and stays allocated.
+// hipStreamPerThread is one handle for a stream of each thread, which the allocator cannot tell apart. Its calls take memory
+// of torch's current stream and wait for the work queued there, and the allocator hands the block out again behind this
+// thread's stream.
 class Scratch {
   public:
     // Throws torch's out-of-memory error.
-    Scratch(size_t bytes, hipStream_t stream) {
+    Scratch(size_t bytes, hipStream_t stream, int dev) {
         RelaxedCapture relaxed;
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        unsigned long long id = 0;
-        if (hipStreamGetCaptureInfo(stream, &st, &id) != hipSuccess) {   // (the legacy stream, while another captures)
-            (void)hipGetLastError();
-            st = hipStreamCaptureStatusNone;
+        unsigned long long id = capture_of(stream);
+        if (stream == hipStreamPerThread) {
+            const c10::hip::HIPStream cur = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev);
+            if (!id) id = capture_of(cur.stream());   // (nothing of the current stream's can be waited for then)
+            if (id) {
+                ptr = of_capture(id, stream, bytes);
+                return;
+            }
+            data_ = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+            ptr = data_.get();
+            c10::hip::HIPCachingAllocator::recordStream(data_, c10::hip::getStreamFromExternal(stream, (c10::DeviceIndex)dev));
+            hipEvent_t ev;
+            C10_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            const hipError_t e0 = hipEventRecord(ev, cur.stream()), e1 = hipStreamWaitEvent(stream, ev, 0);
+            (void)hipEventDestroy(ev);
+            C10_HIP_CHECK(e0);
+            C10_HIP_CHECK(e1);
+            return;
         }
         own_ = c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, stream);
         ptr = own_;
-        if (st == hipStreamCaptureStatusActive && !in_private_pool(own_)) {
+        if (id && !in_private_pool(own_)) {
             release();
             ptr = of_capture(id, stream, bytes);
         }
@@ -98,6 +114,14 @@ class Scratch {
     void* ptr = nullptr;
 
   private:
+    // One more than the id of the capture that the stream takes part in, or 0.
+    static unsigned long long capture_of(hipStream_t stream) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        if (hipStreamGetCaptureInfo(stream, &st, &id) != hipSuccess) (void)hipGetLastError();   // (the legacy stream, while another captures)
+        else if (st == hipStreamCaptureStatusActive) return id + 1u;
+        return 0;
+    }
     void release() {
         if (own_) c10::hip::HIPCachingAllocator::raw_delete(own_);
         own_ = nullptr;
@@ -117,6 +141,7 @@ class Scratch {
         return h.first;
     }
     void* own_ = nullptr;
+    at::DataPtr data_;
 };
 
 void* stream_of(PyObject* o, int dev, bool& ok) {
@@ -167,7 +192,7 @@ PyObject* run_params(fmha_mxfp8_params& p, int dev, void* stream) {
         for (const size_t n : {bytes, one}) {
             if (ws || !n || (oom && n == bytes)) continue;
             try {
-                ws.emplace(n, (hipStream_t)stream);
+                ws.emplace(n, (hipStream_t)stream, dev);
                 bytes = n;
             } catch (const c10::OutOfMemoryError&) {
                 oom = std::current_exception();

@@ -289,3 +289,28 @@ def test_without_memory_for_a_workspace(gpu):
     ops.fmha_fwd_mxfp8(*kv, kv_out)
     torch.cuda.synchronize()
     assert torch.isfinite(kv_out.float()).all()
+
+
+def test_per_thread_streams(gpu):
+    """hipStreamPerThread (handle 2) is one handle for as many streams as there are threads: their calls, at once."""
+    cases = [_case(gpu, 8, 32, 8, 1, 2048, seed=i) for i in range(4)]
+    want = _eager(cases)
+    outs = [[_out(t) for _ in range(10)] for t in cases]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            for o in outs[i]:
+                ops.fmha_fwd_mxfp8(*cases[i], o, stream=2)
+        except Exception as e:   # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [x.start() for x in threads]
+    [x.join() for x in threads]
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(4):
+        for o in outs[i]:
+            assert torch.equal(o.view(torch.int16), want[i].view(torch.int16)), i
