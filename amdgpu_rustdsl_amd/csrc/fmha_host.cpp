@@ -141,22 +141,26 @@ bool use_split_tiles(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
 }
 
 // The one-call entry also runs the vs128 path on the 128-row grid when its 256-row grid holds at most 128 blocks (half
-// of the 256 CUs or fewer): there the same shape fills twice the CUs. Causal (extension): always from 4 key tiles on,
-// so that the 128-row grid's causal q-tile pairing is available past one wave of blocks, except square causal shapes whose
-// 256-row grid has more blocks than CUs: there the 256-row kernel with its heaviest query tiles first balances as well
-// and takes 1.5 us per 256 rows and key tile where the split-tile kernel takes 2.1 (us per call, split-tile / 256-row:
-// B1 H32 HK8 S6144 174.3 / 146.1, S4096 82.6 / 66.5, B3 H8 S3001 63.7 / 40.0, B8 H8 S2048 62.5 / 59.2; at one round of
-// blocks it loses: B1 H8 S8192 72.2 / 86.4, B2 H8 S4096 41.9 / 47.5). 9 key tiles keep the split-tile kernel, which
-// fmha_mxfp8_uses_split_tiles has always named there (B8 H8 S1152 39.4 / 29.9). With many more keys than queries (chunked prefill,
-// S < SK) the split-tile order is kept: every row then averages many keys, and outputs of the two orders, though equally
-// close to float64, differ by 3 % from each other. The kernel is chosen as for t128 (above). Below the split-tile threshold the 256-thread t128 kernel gives the vs128 kernel's order and bits
+// of the 256 CUs or fewer): there the same shape fills twice the CUs. The kernel is chosen as for t128 (above). Below the
+// split-tile threshold the 256-thread t128 kernel gives the vs128 kernel's order and bits
 // (both take every tile whole) on twice the blocks; measured with the LUT recipe at B4H8S1024 SK256, B2H8S2048 SK384
 // and B1H8S4096 SK128: 10.4 / 12.6 / 7.7 us against 11.9 / 14.3 / 9.5 (above 128 blocks of 256 rows the vs128 kernel
 // stays ahead: B8H8S2048 SK256 25.4 against 36.4 us). The direct vs128 launcher keeps the 256-row kernel its grid names.
-bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
+// Causal (extension): always from 4 key tiles on, so that the 128-row grid's causal q-tile pairing is available past one
+// wave of blocks, except where the 256-row kernel gives the same bits sooner: grids of more 256-row blocks than CUs with
+// 4 to 8 key tiles, whose 128-row form is the 256-thread kernel. With its heaviest query tiles first the 256-row kernel
+// balances as well as the pairs do (us, 128-row / 256-row: B16 H8 S512 15.9 / 14.3, B9 H8 S1000 36.6 / 34.7, B16 H8 S1024
+// 39.3 / 37.7; S < SK: B32 H8 S256 SK1024 34.1 / 23.1, B16 H8 S768 SK1024 42.5 / 34.9). With at most 128 query rows half of
+// its block is padding (B64 H8 S128 SK1024 38.4 / 40.9). A caller that asks for the pairing has it. From 9 key tiles on the 128-row
+// form is the split-tile kernel, whose error against float64 is the smaller one (relative, split-tile / 256-row, three
+// seeds each: B8 H8 S1152 0.0241 / 0.0245, S2048 0.0249 / 0.0252, B1 H32 HK8 S6144 0.0261 / 0.0264): it stays, though the
+// 256-row kernel takes 147 us for the last of them and it 175.
+bool vs128_on_128row_grid(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal, bool pair_asked = false) {
     const int64_t blocks = (S + 255) / 256 * H * B;
     const int64_t tiles = (SK + 127) / 128;
-    return blocks <= 128 || (causal && tiles >= 4 && !(S == SK && (tiles <= 8 || tiles >= 10) && blocks > (int64_t)cu_count()));
+    if (blocks <= 128) return true;
+    if (!causal || tiles < 4) return false;
+    return tiles > 8 || S <= 128 || blocks <= (int64_t)cu_count() || pair_asked;
 }
 
 fmha_internal::ModuleCache<27> g_fmha(fmha_mxfp8_hsaco_begin, fmha_mxfp8_hsaco_end, kKernelNames);
@@ -403,8 +407,8 @@ struct Plan {
     uint32_t block, gx;
 };
 
-int kernel_of(int path, i64 B, i64 H, i64 S, i64 SK, bool causal, bool scaled, uint32_t* block, uint32_t* gx) {
-    if (path == FMHA_PATH_VS128 && !vs128_on_128row_grid(B, H, S, SK, causal)) {
+int kernel_of(int path, i64 B, i64 H, i64 S, i64 SK, bool causal, bool pair_asked, bool scaled, uint32_t* block, uint32_t* gx) {
+    if (path == FMHA_PATH_VS128 && !vs128_on_128row_grid(B, H, S, SK, causal, pair_asked)) {
         *block = 512u;
         *gx = (uint32_t)((S + 255) / 256);
         return scaled ? K_VS128_SC : K_VS128;
@@ -436,7 +440,7 @@ void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspa
         // kv_fill = 1 asks for the reference's grid
         if (any_path && !p.kv_fill) pl.sub = packed_sub(B, H, HK, S, SK, pl.parts, false, true, p.f32_partials != 0, H * B * pl.parts, fits);
     } else {
-        pl.kern = kernel_of(pl.path, B, H, S, SK, p.causal != 0, scaled, &pl.block, &pl.gx);
+        pl.kern = kernel_of(pl.path, B, H, S, SK, p.causal != 0, p.causal_pair == 1, scaled, &pl.block, &pl.gx);
         pl.whole = pl.kern != K_T128ST && pl.kern != K_T128ST_SC;
         // a forced path keeps its kernel (and its bits)
         if (any_path && p.path < 0 && p.kv_fill == 0)

@@ -211,9 +211,9 @@ int fmha_mxfp8_select_path(int64_t B, int64_t H, int64_t S, int64_t SK, int* spl
  * blocks of 512 threads, the two wave groups splitting each tile's keys and merging at the end), else 0. t128: at
  * least 7 key tiles (4 with `causal`); below that the 256-thread fmha_fwd_hd128_mxfp8_v3_t128, which is faster there
  * and keeps the reference's order. vs128: the same, and a 256-row grid of at most 128 blocks unless `causal` (the
- * 128-row grid's causal q-tile pairing; not for S = SK with more 256-row blocks than CUs, which run the 256-row kernel
- * with the heaviest query tiles first); such a half-chip grid below the threshold runs on the 256-thread t128
- * kernel. The split-tile order rounds differently from the reference's single stream per row; the path and its
+ * 128-row grid's causal q-tile pairing); such a half-chip grid below the threshold runs on the 256-thread t128
+ * kernel, and so do causal grids that the pairing halves with at most 8 key tiles (with more 256-row blocks than CUs and
+ * no pairing asked for, on the 256-row kernel: the same order and bits). The split-tile order rounds differently from the reference's single stream per row; the path and its
  * recipe are the reference's. */
 int fmha_mxfp8_uses_split_tiles(int path, int64_t B, int64_t H, int64_t S, int64_t SK, int causal);
 
@@ -277,7 +277,9 @@ typedef struct fmha_mxfp8_params {
                                   reference op's check=False does (python/amdgpu_jit/ops.py:88): the caller then
                                   vouches for the buffer extents and strides */
     int32_t causal_pair;       /* causal only (extension): 0 = the causal q-tile pairing (FMHA_FLAG_CAUSAL_PAIR) when
-                                  the unpaired grid has more blocks than the device has CUs; 1 = always; 2 = never */
+                                  the unpaired grid has more blocks than the device has CUs; 1 = always; 2 = never
+                                  (0 and 2 also leave grids of more 256-row blocks than CUs with 4 to 8 key tiles to the
+                                  256-row kernel; the bits are the same every way) */
     int32_t kv_fill;           /* KV split only (extension): 0 = each chunk spread over the blocks that
                                   fmha_mxfp8_kv_partials names, as far as the workspace holds their partials;
                                   1 = the reference's chunks only (one block per chunk and query tile) */

@@ -80,30 +80,32 @@ def test_split_last_blocks(gpu, case):
     assert rel <= 1e-3 and big <= 0.02 and ldiff <= 1e-5, (rel, big, ldiff)
 
 
-# (name, B, H, HK, S): square causal grids of more 256-row blocks than CUs; heads that divide over the 8 XCDs and not
+# (name, B, H, HK, S, SK): causal grids of more 256-row blocks than CUs with 4 to 8 key tiles; heads that divide over the 8 XCDs
+# and not
 CAUSAL = [
-    ("H32_gqa", 2, 32, 8, 1300),
-    ("H43", 1, 43, 43, 1500),
-    ("H8_batches", 17, 8, 8, 513),
+    ("H32_gqa", 3, 32, 8, 650, 650),
+    ("H43", 2, 43, 43, 1000, 1000),
+    ("H8_batches", 17, 8, 8, 513, 513),
+    ("more_keys", 33, 8, 2, 129, 1024),
 ]
 
 
 @pytest.mark.parametrize("case", CAUSAL, ids=[c[0] for c in CAUSAL])
 def test_causal_256row_grid(gpu, case):
     """Every row of the causal 256-row grid (heaviest query tiles first): the 256-thread t128 kernel takes every tile
-    whole too, on other blocks in another order, so the two must agree bit for bit, whatever the causal_pair field
-    says; and the sampled rows meet the emulation's bar (gpu_util.causal_bar)."""
-    name, B, H, HK, S = case
+    whole too, on other blocks in another order, so the two must agree bit for bit, also where the caller asks for its
+    pairs; and the sampled rows meet the emulation's bar (gpu_util.causal_bar)."""
+    name, B, H, HK, S, SK = case
     print(f"[case] causal 256-row grid {name}", flush=True)
-    assert not lib.uses_split_tiles("vs128", B, H, S, S, causal=True)
-    inp = oracle.Inputs(B, H, S, S, HK=HK, causal=True)
+    assert not lib.uses_split_tiles("vs128", B, H, S, SK, causal=True)
+    inp = oracle.Inputs(B, H, S, SK, HK=HK, causal=True)
     out, used, lse = gpu_util.run(inp, gpu, lse=True)
     assert used[0] == "vs128"
     paired, _, _ = gpu_util.run(inp, gpu, causal_pair=True)
     np.testing.assert_array_equal(out, paired)
     q, k, v, qs, ks, vs = gpu_util.upload(inp, gpu)
     o2 = torch.full((B, S, H, D), float("nan"), dtype=torch.bfloat16, device=gpu)
-    a = lib.fill_args(o2.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), qs.data_ptr(), ks.data_ptr(), vs.data_ptr(), B, H, HK, S, S)
+    a = lib.fill_args(o2.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), qs.data_ptr(), ks.data_ptr(), vs.data_ptr(), B, H, HK, S, SK)
     a.flags = lib.FLAG_CAUSAL
     st = torch.cuda.current_stream(gpu).cuda_stream
     assert lib.raw.fmha_mxfp8_launch_t128(ctypes.byref(a), math.ceil(S / 128), H, B, st) == 0
@@ -115,3 +117,18 @@ def test_causal_256row_grid(gpu, case):
     print(f"[case] causal 256-row grid {name} causal-bar={fig}", flush=True)
     assert not viol, (viol, fig)
     assert torch.isfinite(lse).all()
+
+
+def test_asked_pairing_runs_the_paired_kernel(gpu):
+    """causal_pair=True runs the query-tile pairs of the 128-row kernel also where the automatic choice is the 256-row one."""
+    from torch.profiler import ProfilerActivity, profile
+
+    inp = oracle.Inputs(40, 8, 300, 520, HK=8, causal=True)
+    names = []
+    for pair in ("auto", True):
+        gpu_util.run(inp, gpu, causal_pair=pair)
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            gpu_util.run(inp, gpu, causal_pair=pair)
+        names.append([e.key for e in prof.key_averages() if "fmha_fwd" in e.key])
+    print(f"[case] asked pairing {names}", flush=True)
+    assert names == [["fmha_fwd_hd128_mxfp8_pre_vs128"], ["fmha_fwd_hd128_mxfp8_v3_t128"]]
