@@ -492,7 +492,7 @@ struct Stager {
     // index, the three resources took ~50 scalar instructions in a row per VALU phase, during which the wave converted
     // nothing. The K-scale rows are k_seq / 32 bytes of the K tile's rows.
     uint64_t ck, cv, cks;
-    TileSizes sizes;
+    TileSizes<NT == 512 ? 1 : 0> sizes;   // V one tile behind K in the ping-pong kernels
     uint32_t cstep, csstep, woff;
     __device__ __forceinline__ void init_cursors(uint32_t kkey, uint32_t vkey, uint32_t limit) {
         ck = (uint64_t)(uintptr_t)kb + (uint64_t)kkey * k_seq;
@@ -503,8 +503,7 @@ struct Stager {
         csstep = kTile * ks_row;
         woff = __builtin_amdgcn_readfirstlane(tid >> 6) * 1024u;
     }
-    // one VALU phase on: V one tile behind K (the ping-pong kernels)
-    __device__ __forceinline__ void advance() { sizes.template advance<1>(k_seq); }
+    __device__ __forceinline__ void advance() { sizes.advance(k_seq); }
     // K's copies, then V's: alternating, or V first, cost the split-tile grids 0.5 % and 3 %. ALT: alternating (the packed rows,
     // which stream both from HBM)
     template <bool ALT>
@@ -529,12 +528,12 @@ struct Stager {
     };
     __device__ __forceinline__ Next next_tile(uint32_t slot) {
         const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
-        sizes.template advance<0>(k_seq);
         Next n = {make_rsrc((const void*)(uintptr_t)ck, sizes.k), make_rsrc((const void*)(uintptr_t)cv, sizes.v),
                   make_rsrc((const void*)(uintptr_t)cks, w < 2u ? sizes.k >> 5 : 0u),
                   slot_base(lds + woff, kLdsK, slot, kTileBytes), slot_base(lds + woff, kLdsV, slot, kTileBytes),
                   w < 2u ? slot_base(lds, kLdsKs, slot, kKsSlot) + 256u * w : lds + kLdsKsDummy + 256u * ((w - 2u) & 3u)};
         ck += cstep; cv += cstep; cks += csstep;
+        advance();
         return n;
     }
     __device__ __forceinline__ void dma_next_part(const Next& n, int i) const {
@@ -1499,10 +1498,10 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
         if (idle) {
             for (uint32_t t = 0; t < ntiles; ++t) {
                 if (!GB) st.store_ks(slot_of(t + 2));
-                st.advance();
                 st.template dma_next<true>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
                 if (!GB) st.load_ks_next();
+                st.advance();
                 block_barrier_keep_dma<0, kDmaOps>();
             }
         }
@@ -1518,11 +1517,11 @@ __device__ __forceinline__ void attend_pingpong_group(const Prm& p, uint32_t lds
             auto copies = [&](uint32_t t) {
                 // the K-scale words before the copies; behind them in the packed rows, where the copies come from HBM and
                 // should go out first (B1 H8 S128 SK16000, with the order of the copies, 16.3 -> 16.0 us per call)
-                st.advance();
                 if (!GB && !PK) st.load_ks_next();
                 st.template dma_next<PK>(slot_of(t + 3), slot_of(t + 2));
                 if (VS) st.dma_vs(key_of(t + 2), t + 2 < ntiles, slot_of(t + 2));
                 if (!GB && PK) st.load_ks_next();
+                st.advance();
             };
             auto v_phase = [&](uint32_t t, uint32_t (&pw)[NA][4], bool last) {
                 FMHA_SETPRIO(0);

@@ -23,20 +23,22 @@ FMHA_TILE_FN uint32_t tile_extent(int32_t left, uint32_t stride) {
     return (uint32_t)(rows > 128 ? 128 : rows) * stride;
 }
 
-// The sizes for consecutive tiles as running state: advance() steps to the next K tile and, `lag` tiles (0 or 1) behind it, V tile.
+// The sizes of consecutive tiles as running state: those of the current K tile and of the V tile `LAG` tiles (0 or 1) behind it.
+// advance() steps to the next ones, after the current copies are out, so that none of its instructions stands before them.
+template <int LAG>
 struct TileSizes {
-    int32_t left;    // rows from the next K tile's first one to the end of the range
+    int32_t left;    // rows from the current K tile's first one to the end of the range
     uint32_t k, v;   // the current K and V tiles' sizes
     FMHA_TILE_FN void init(uint32_t end, uint32_t kkey, uint32_t stride) {
         left = (int32_t)(end - kkey);
-        k = v = tile_extent(left + 128, stride);
+        k = tile_extent(left, stride);
+        v = LAG ? tile_extent(left + 128, stride) : k;
     }
-    template <int LAG>
     FMHA_TILE_FN void advance(uint32_t stride) {
+        left -= 128;
         if (LAG) v = k;
         k = tile_extent(left, stride);
         if (!LAG) v = k;
-        left -= 128;
     }
 };
 

@@ -11,16 +11,18 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = r"""
 #include "tile_extent.h"
 extern "C" unsigned extent(unsigned end, unsigned key, unsigned stride) { return tile_extent((int32_t)(end - key), stride); }
-// sizes[2 i], [2 i + 1]: the K tile at kkey + 128 i and the V tile `lag` tiles behind it
-extern "C" void sequence(unsigned end, unsigned kkey, unsigned stride, int lag, int n, unsigned* sizes) {
-    TileSizes t;
+template <int LAG>
+void walk(unsigned end, unsigned kkey, unsigned stride, int n, unsigned* sizes) {
+    TileSizes<LAG> t;
     t.init(end, kkey, stride);
-    for (int i = 0; i < n; ++i) {
-        if (lag) t.advance<1>(stride);
-        else t.advance<0>(stride);
+    for (int i = 0; i < n; ++i, t.advance(stride)) {
         sizes[2 * i] = t.k;
         sizes[2 * i + 1] = t.v;
     }
+}
+// sizes[2 i], [2 i + 1]: the K tile at kkey + 128 i and the V tile `lag` tiles behind it
+extern "C" void sequence(unsigned end, unsigned kkey, unsigned stride, int lag, int n, unsigned* sizes) {
+    (lag ? walk<1> : walk<0>)(end, kkey, stride, n, sizes);
 }
 """
 
