@@ -321,8 +321,8 @@ PyObject* quantize_v_impl(PyObject* const* a, Py_ssize_t n) {
         Py_BEGIN_ALLOW_THREADS
         rc = seq32 ? fmha_mxfp8_quantize_seq32(x->data_ptr(), q.data_ptr(), sc.data_ptr(), (int32_t)x->size(0), (int32_t)x->size(1),
                                                (int32_t)x->size(2), cap(*x), cap(q), cap(sc), stream, err, sizeof(err))
-                   : fmha_mxfp8_quantize_tensor(x->data_ptr(), q.data_ptr(), sc.data_ptr(), x->numel(), cap(*x), cap(q), cap(sc), stream, err,
-                                                sizeof(err));
+                   : fmha_mxfp8_quantize_v(x->data_ptr(), q.data_ptr(), sc.data_ptr(), x->numel(), cap(*x), cap(q), cap(sc), stream, err,
+                                           sizeof(err));
         Py_END_ALLOW_THREADS
     }
     if (rc != FMHA_OK) return raise_code(rc, err);

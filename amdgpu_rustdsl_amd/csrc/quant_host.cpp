@@ -43,6 +43,7 @@ struct QuantTensorArgs {
     void* q;
     void* descale;
     uint64_t n;
+    uint32_t clear, pad;
 };
 struct QuantSeq32Args {
     const void* x;
@@ -58,9 +59,9 @@ struct QuantQkvArgs {
     uint32_t q_slack_words, k_slack_words;
     uint32_t gq, gk, gv, seq32;
 };
-static_assert(sizeof(QuantQkvArgs) == 192, "qkv kernarg");
+static_assert(sizeof(QuantQkvArgs) == 200, "qkv kernarg");
 static_assert(sizeof(QuantRowsArgs) == 40, "rows kernarg");
-static_assert(sizeof(QuantTensorArgs) == 32, "tensor kernarg");
+static_assert(sizeof(QuantTensorArgs) == 40, "tensor kernarg");
 static_assert(sizeof(QuantSeq32Args) == 40, "seq32 kernarg");
 
 const char* const kQuantNames[5] = {
@@ -135,6 +136,16 @@ int check_seq32(const void* x, const void* q, const void* scale, int32_t B, int3
     return FMHA_OK;
 }
 
+int quantize_tensor(const void* x, void* q, void* descale, int64_t n, bool clear, uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_descale,
+                    void* stream, char* err, size_t errlen) {
+    int rc = check_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, err, errlen);
+    if (rc != FMHA_OK) return rc;
+    QuantTensorArgs a = {x, q, descale, (uint64_t)n, clear ? 1u : 0u, 0u};
+    rc = g_quant.launch(Q_AMAX, &a, sizeof(a), kAmaxGroups, 1, 1, 256, stream, err, errlen);
+    if (rc == FMHA_OK) rc = g_quant.launch(Q_TENSOR, &a, sizeof(a), stride_grid((uint64_t)n / 8), 1, 1, 256, stream, err, errlen);
+    return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -149,12 +160,12 @@ int fmha_mxfp8_quantize_rows(const void* x, void* q, void* scale, int64_t rows, 
 
 int fmha_mxfp8_quantize_tensor(const void* x, void* q, void* descale, int64_t n, uint64_t bytes_x, uint64_t bytes_q,
                                uint64_t bytes_descale, void* stream, char* err, size_t errlen) {
-    int rc = check_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, err, errlen);
-    if (rc != FMHA_OK) return rc;
-    QuantTensorArgs a = {x, q, descale, (uint64_t)n};
-    rc = g_quant.launch(Q_AMAX, &a, sizeof(a), kAmaxGroups, 1, 1, 256, stream, err, errlen);
-    if (rc == FMHA_OK) rc = g_quant.launch(Q_TENSOR, &a, sizeof(a), stride_grid((uint64_t)n / 8), 1, 1, 256, stream, err, errlen);
-    return rc;
+    return quantize_tensor(x, q, descale, n, false, bytes_x, bytes_q, bytes_descale, stream, err, errlen);
+}
+
+int fmha_mxfp8_quantize_v(const void* x, void* q, void* descale, int64_t n, uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_descale,
+                          void* stream, char* err, size_t errlen) {
+    return quantize_tensor(x, q, descale, n, true, bytes_x, bytes_q, bytes_descale, stream, err, errlen);
 }
 
 size_t fmha_mxfp8_seq32_scale_bytes(int64_t B, int64_t SK, int64_t HK) { return seq32_bytes(B, SK, HK); }
@@ -184,7 +195,7 @@ int fmha_mxfp8_quantize_qkv(const fmha_mxfp8_qkv_params* p, void* stream, char* 
     std::memset(&a, 0, sizeof(a));
     a.q = {p->q, p->q8, p->q_scale, (uint64_t)rq, p->q_mul, 0u};
     a.k = {p->k, p->k8, p->k_scale, (uint64_t)rk, 1.0f, 0u};
-    a.vt = {p->v, p->v8, p->v_scale, (uint64_t)rk * 128};
+    a.vt = {p->v, p->v8, p->v_scale, (uint64_t)rk * 128, 1u, 0u};
     a.vs = {p->v, p->v8, p->v_scale, (uint32_t)p->B, (uint32_t)p->SK, (uint32_t)p->HK, (uint32_t)((p->SK + 31) / 32)};
     a.q_slack = (char*)p->q_scale + rq * 4;
     a.k_slack = (char*)p->k_scale + rk * 4;

@@ -83,6 +83,7 @@ struct QuantTensorArgs {
     uint8_t* q;          // [n] e4m3
     float* descale;      // 1024 f32: [0] the descale; [kQuantPartial, +kQuantAmaxGroups) the amax pass's partials
     uint64_t n;
+    uint32_t clear, pad; // whether the words between are cleared
 };
 // The amax pass runs exactly this many workgroups (the host launches it so), one partial maximum each.
 constexpr uint32_t kQuantAmaxGroups = 512;
@@ -231,9 +232,9 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_tensor(QuantT
             if (c < nchunk) store8_system(a.q + c * 8u, out);
         }
     }
-    // descale[0] = d, and zeros up to the partial maxima (the buffer's contents do not depend on what it held)
+    // descale[0] = d, and for callers with a fresh buffer zeros up to the partial maxima
     if (blockIdx.x == 0)
-        for (uint32_t i = threadIdx.x; i < kQuantPartial; i += 256u) a.descale[i] = i == 0u ? d : 0.0f;
+        for (uint32_t i = threadIdx.x; i < (a.clear ? kQuantPartial : 1u); i += 256u) a.descale[i] = i == 0u ? d : 0.0f;
 }
 
 // Sequence blocks: one wave per tile of 32 keys x 128 columns of one (b, kv head). Lane l takes columns 8 (l & 15) .. +7 of

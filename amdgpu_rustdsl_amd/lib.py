@@ -125,6 +125,7 @@ _L.fmha_mxfp8_version.argtypes = []
 # include/mxfp8_quant.h
 _L.fmha_mxfp8_quantize_rows.argtypes = [_vp, _vp, _vp, _i64, ctypes.c_float, _u64, _u64, _u64, _vp, _cp, _sz]
 _L.fmha_mxfp8_quantize_tensor.argtypes = [_vp, _vp, _vp, _i64, _u64, _u64, _u64, _vp, _cp, _sz]
+_L.fmha_mxfp8_quantize_v.argtypes = _L.fmha_mxfp8_quantize_tensor.argtypes
 _L.fmha_mxfp8_quantize_seq32.argtypes = [_vp, _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _u64, _u64, _u64, _vp, _cp, _sz]
 _L.fmha_mxfp8_quantize_qkv.argtypes = [_P(QkvParams), _vp, _cp, _sz]
 _L.fmha_mxfp8_seq32_scale_bytes.argtypes = [_i64, _i64, _i64]
@@ -135,7 +136,7 @@ EXPORTED = ["fmha_mxfp8_validate_vs128", "fmha_mxfp8_validate_t128", "fmha_mxfp8
             "fmha_mxfp8_launch_t128", "fmha_mxfp8_launch_t128_split_tiles", "fmha_mxfp8_launch_kvsplit", "fmha_mxfp8_launch_combine", "fmha_mxfp8_launch_combine_wide", "fmha_fwd_hd128_mxfp8_auto",
             "fmha_fwd_hd128_mxfp8_auto_noalloc", "fmha_fwd_hd128_mxfp8_auto_ws", "fmha_mxfp8_auto_workspace_bytes",
             "fmha_mxfp8_init", "fmha_mxfp8_version",
-            "fmha_mxfp8_quantize_rows", "fmha_mxfp8_quantize_tensor", "fmha_mxfp8_quantize_seq32", "fmha_mxfp8_quantize_qkv", "fmha_mxfp8_seq32_scale_bytes"]
+            "fmha_mxfp8_quantize_rows", "fmha_mxfp8_quantize_tensor", "fmha_mxfp8_quantize_v", "fmha_mxfp8_quantize_seq32", "fmha_mxfp8_quantize_qkv", "fmha_mxfp8_seq32_scale_bytes"]
 
 raw = _L
 
@@ -265,6 +266,11 @@ def quantize_rows(x, q, scale, rows, mul, bytes_x, bytes_q, bytes_scale, stream=
 def quantize_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, stream=None):
     buf = _errbuf()
     check(_L.fmha_mxfp8_quantize_tensor(x, q, descale, n, bytes_x, bytes_q, bytes_descale, stream, buf, 512), buf)
+
+
+def quantize_v(x, q, descale, n, bytes_x, bytes_q, bytes_descale, stream=None):
+    buf = _errbuf()
+    check(_L.fmha_mxfp8_quantize_v(x, q, descale, n, bytes_x, bytes_q, bytes_descale, stream, buf, 512), buf)
 
 
 def quantize_seq32(x, q, scale, B, SK, HK, bytes_x, bytes_q, bytes_scale, stream=None):

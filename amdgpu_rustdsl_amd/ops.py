@@ -203,7 +203,7 @@ def quantize_mxfp8(x, scale_out, mul=1.0, stream=None):
 def quantize_v(x, stream=None):
     """On-GPU V quantisation with one f32 descale per tensor (ref_host.cpp:248-251): d = amax / 448, q = e4m3(x / d).
     Returns (q uint8 of x's shape, v_scale: a 4096-byte f32 buffer with d in element 0, the FMHA's V descale
-    argument). x may have any shape whose element count is a multiple of 8. Runs fmha_mxfp8_quantize_tensor."""
+    argument). x may have any shape whose element count is a multiple of 8. Runs fmha_mxfp8_quantize_v."""
     done = _native.quantize_v(x, False, stream)
     if done is not None:
         return done
@@ -211,7 +211,7 @@ def quantize_v(x, stream=None):
     q = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
     vs = torch.empty(1024, dtype=torch.float32, device=x.device)   # written whole: d, zeros, the partial maxima
     with torch.cuda.device(x.device):
-        lib.quantize_tensor(xb.data_ptr(), q.data_ptr(), vs.data_ptr(), xb.numel(), _cap(xb), _cap(q), _cap(vs), _stream(x.device, stream))
+        lib.quantize_v(xb.data_ptr(), q.data_ptr(), vs.data_ptr(), xb.numel(), _cap(xb), _cap(q), _cap(vs), _stream(x.device, stream))
     return q, vs
 
 

@@ -43,6 +43,12 @@ int fmha_mxfp8_quantize_tensor(const void* x, void* q, void* descale, int64_t n,
                                uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_descale,
                                void* stream, char* err, size_t errlen);
 
+/* The same for a `descale` buffer that holds nothing yet (extension): f32 words [1, 512) are cleared too, so that the
+ * buffer's contents do not depend on what the memory held. */
+int fmha_mxfp8_quantize_v(const void* x, void* q, void* descale, int64_t n,
+                          uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_descale,
+                          void* stream, char* err, size_t errlen);
+
 /* x [B, SK, HK, 128] bf16 -> q [B, SK, HK, 128] e4m3, scale [B, ceil(SK/32), HK, 128] E8M0 (8-byte aligned). */
 int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, int32_t SK, int32_t HK,
                               uint64_t bytes_x, uint64_t bytes_q, uint64_t bytes_scale,
@@ -53,8 +59,9 @@ size_t fmha_mxfp8_seq32_scale_bytes(int64_t B, int64_t SK, int64_t HK);
 
 /* Q, K and V of one attention layer from bf16 (extension): the same bytes as fmha_mxfp8_quantize_rows of Q (with
  * q_mul) and of K and fmha_mxfp8_quantize_tensor (or, v_seq32 != 0, _seq32) of V, in one launch (two with the tensor
- * scale). bytes_q_scale and bytes_k_scale are the whole allocations: what lies behind the scales is cleared (the slack
- * that the attention requires to be zero). v_scale: 4096 bytes of f32, or E8M0 [B, ceil(SK/32), HK, 128]. */
+ * scale). bytes_q_scale and bytes_k_scale are the whole allocations: what lies behind the scales is cleared, in whole
+ * 4-byte words (the slack that the attention requires to be zero). v_scale: 4096 bytes of f32, as
+ * fmha_mxfp8_quantize_v leaves them, or E8M0 [B, ceil(SK/32), HK, 128]. */
 typedef struct fmha_mxfp8_qkv_params {
     const void* q; const void* k; const void* v;        /* bf16 [B,S,H,128], [B,SK,HK,128] twice */
     void* q8; void* k8; void* v8;                       /* e4m3, same shapes */

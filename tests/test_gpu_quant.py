@@ -195,6 +195,22 @@ def test_qkv_matches_separate_quantisers(gpu, B, S, H, SK, HK, seq32):
         assert not vs2[1:512].any() and not vs[1:512].any()
 
 
+def test_tensor_leaves_the_callers_words(gpu):
+    """fmha_mxfp8_quantize_tensor writes word 0 and the partial maxima of a descale buffer and nothing between;
+    fmha_mxfp8_quantize_v, for a fresh buffer, clears the words between. Same bytes and descale."""
+    x = torch.randn(8 * 1001, device=gpu).to(torch.bfloat16)
+    res = []
+    for f in (lib.quantize_tensor, lib.quantize_v):
+        q, d = torch.empty(x.numel(), dtype=torch.uint8, device=gpu), torch.full((1026,), 7.0, device=gpu)
+        f(x.data_ptr(), q.data_ptr(), d.data_ptr(), x.numel(), 2 * x.numel(), x.numel(), 4096, torch.cuda.current_stream(gpu).cuda_stream)
+        torch.cuda.synchronize()
+        res.append((q, d))
+    (q, d), (q2, d2) = res
+    assert (d[1:512] == 7.0).all() and not d2[1:512].any()
+    assert (d[1024:] == 7.0).all() and (d2[1024:] == 7.0).all()
+    assert torch.equal(q, q2) and d[0] == d2[0] and torch.equal(d[512:], d2[512:])
+
+
 def test_rejections(gpu):
     x = torch.zeros(16, D, dtype=torch.bfloat16, device=gpu)
     q = torch.empty(16 * D, dtype=torch.uint8, device=gpu)
