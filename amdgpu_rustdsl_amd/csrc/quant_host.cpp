@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -50,6 +51,7 @@ struct QuantSeq32Args {
     void* q;
     void* scale;
     uint32_t B, SK, HK, nblk;
+    uint64_t tile0;
 };
 struct QuantQkvArgs {
     QuantRowsArgs q, k;
@@ -59,10 +61,10 @@ struct QuantQkvArgs {
     uint32_t q_slack_words, k_slack_words;
     uint32_t gq, gk, gv, seq32;
 };
-static_assert(sizeof(QuantQkvArgs) == 200, "qkv kernarg");
+static_assert(sizeof(QuantQkvArgs) == 208, "qkv kernarg");
 static_assert(sizeof(QuantRowsArgs) == 40, "rows kernarg");
 static_assert(sizeof(QuantTensorArgs) == 40, "tensor kernarg");
-static_assert(sizeof(QuantSeq32Args) == 40, "seq32 kernarg");
+static_assert(sizeof(QuantSeq32Args) == 48, "seq32 kernarg");
 
 const char* const kQuantNames[5] = {
     "fmha_mxfp8_quant_rows", "fmha_mxfp8_quant_amax", "fmha_mxfp8_quant_tensor", "fmha_mxfp8_quant_seq32", "fmha_mxfp8_quant_qkv",
@@ -119,7 +121,9 @@ size_t seq32_bytes(int64_t B, int64_t SK, int64_t HK) {
 
 // one wave per 32-key tile, four to a workgroup
 uint64_t seq32_tiles(int64_t B, int64_t SK, int64_t HK) { return (uint64_t)B * (uint64_t)((SK + 31) / 32) * (uint64_t)HK; }
-uint32_t seq32_groups(int64_t B, int64_t SK, int64_t HK) { return (uint32_t)((seq32_tiles(B, SK, HK) + 3) / 4); }
+uint64_t seq32_groups(int64_t B, int64_t SK, int64_t HK) { return (seq32_tiles(B, SK, HK) + 3) / 4; }
+// Workgroups of 256 threads that one launch can have (its threads are counted in 32 bits).
+constexpr uint64_t kMaxGroups = 0xFFFFFFFFull / 256;
 
 int check_seq32(const void* x, const void* q, const void* scale, int32_t B, int32_t SK, int32_t HK, uint64_t bytes_x, uint64_t bytes_q,
                 uint64_t bytes_scale, char* err, size_t errlen) {
@@ -132,7 +136,17 @@ int check_seq32(const void* x, const void* q, const void* scale, int32_t B, int3
     if (bytes_q < elems) return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "q: buffer smaller than B*SK*HK*128 bytes");
     if (bytes_scale < seq32_bytes(B, SK, HK))
         return fail(err, errlen, FMHA_ERR_EXTENT, "GV-HOST-EXTENT", "scale: buffer smaller than B*ceil(SK/32)*HK*128 bytes");
-    if ((seq32_tiles(B, SK, HK) + 3) / 4 > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
+    if ((seq32_tiles(B, SK, HK) + 15) / 16 > 0xFFFFFFFFull) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensor too large");
+    return FMHA_OK;
+}
+
+int launch_seq32(QuantSeq32Args a, void* stream, char* err, size_t errlen) {
+    const uint64_t groups = seq32_groups(a.B, a.SK, a.HK);
+    for (uint64_t g = 0; g < groups; g += kMaxGroups) {
+        a.tile0 = 4 * g;
+        const int rc = g_quant.launch(Q_SEQ32, &a, sizeof(a), (uint32_t)std::min(kMaxGroups, groups - g), 1, 1, 256, stream, err, errlen);
+        if (rc != FMHA_OK) return rc;
+    }
     return FMHA_OK;
 }
 
@@ -174,8 +188,7 @@ int fmha_mxfp8_quantize_seq32(const void* x, void* q, void* scale, int32_t B, in
                               uint64_t bytes_q, uint64_t bytes_scale, void* stream, char* err, size_t errlen) {
     const int rc = check_seq32(x, q, scale, B, SK, HK, bytes_x, bytes_q, bytes_scale, err, errlen);
     if (rc != FMHA_OK) return rc;
-    QuantSeq32Args a = {x, q, scale, (uint32_t)B, (uint32_t)SK, (uint32_t)HK, (uint32_t)((SK + 31) / 32)};
-    return g_quant.launch(Q_SEQ32, &a, sizeof(a), seq32_groups(B, SK, HK), 1, 1, 256, stream, err, errlen);
+    return launch_seq32({x, q, scale, (uint32_t)B, (uint32_t)SK, (uint32_t)HK, (uint32_t)((SK + 31) / 32), 0u}, stream, err, errlen);
 }
 
 int fmha_mxfp8_quantize_qkv(const fmha_mxfp8_qkv_params* p, void* stream, char* err, size_t errlen) {
@@ -196,18 +209,28 @@ int fmha_mxfp8_quantize_qkv(const fmha_mxfp8_qkv_params* p, void* stream, char* 
     a.q = {p->q, p->q8, p->q_scale, (uint64_t)rq, p->q_mul, 0u};
     a.k = {p->k, p->k8, p->k_scale, (uint64_t)rk, 1.0f, 0u};
     a.vt = {p->v, p->v8, p->v_scale, (uint64_t)rk * 128, 1u, 0u};
-    a.vs = {p->v, p->v8, p->v_scale, (uint32_t)p->B, (uint32_t)p->SK, (uint32_t)p->HK, (uint32_t)((p->SK + 31) / 32)};
+    a.vs = {p->v, p->v8, p->v_scale, (uint32_t)p->B, (uint32_t)p->SK, (uint32_t)p->HK, (uint32_t)((p->SK + 31) / 32), 0u};
     a.q_slack = (char*)p->q_scale + rq * 4;
     a.k_slack = (char*)p->k_scale + rk * 4;
     a.q_slack_words = (uint32_t)qsl;
     a.k_slack_words = (uint32_t)ksl;
-    a.gq = rows_groups(rq);
-    a.gk = rows_groups(rk);
-    a.gv = p->v_seq32 ? seq32_groups(p->B, p->SK, p->HK) : kAmaxGroups;
+    const uint64_t gq = rows_groups(rq), gk = rows_groups(rk), gv = p->v_seq32 ? seq32_groups(p->B, p->SK, p->HK) : kAmaxGroups;
+    const uint64_t gs = (qsl + 1023) / 1024 + (ksl + 1023) / 1024;
     a.seq32 = p->v_seq32 ? 1u : 0u;
-    const uint64_t grid = (uint64_t)a.gq + a.gk + a.gv + (qsl + 1023) / 1024 + (ksl + 1023) / 1024;
-    if (grid > 0xFFFFFFFFull / 256) return fail(err, errlen, FMHA_ERR_KA_RANGE, "GV-HOST-KA-RANGE", "tensors too large");
-    rc = g_quant.launch(Q_QKV, &a, sizeof(a), (uint32_t)grid, 1, 1, 256, stream, err, errlen);
+    uint64_t grid = gs;
+    if (gq + gk + gv + gs <= kMaxGroups) {
+        a.gq = (uint32_t)gq;
+        a.gk = (uint32_t)gk;
+        a.gv = (uint32_t)gv;
+        grid += gq + gk + gv;
+    } else {   // more than one launch can have: one after the other, the slack by the launch below
+        rc = g_quant.launch(Q_ROWS, &a.q, sizeof(a.q), (uint32_t)gq, 1, 1, 256, stream, err, errlen);
+        if (rc == FMHA_OK) rc = g_quant.launch(Q_ROWS, &a.k, sizeof(a.k), (uint32_t)gk, 1, 1, 256, stream, err, errlen);
+        if (rc == FMHA_OK)
+            rc = p->v_seq32 ? launch_seq32(a.vs, stream, err, errlen)
+                            : g_quant.launch(Q_AMAX, &a.vt, sizeof(a.vt), kAmaxGroups, 1, 1, 256, stream, err, errlen);
+    }
+    if (rc == FMHA_OK && grid) rc = g_quant.launch(Q_QKV, &a, sizeof(a), (uint32_t)grid, 1, 1, 256, stream, err, errlen);
     if (rc == FMHA_OK && !p->v_seq32)
         rc = g_quant.launch(Q_TENSOR, &a.vt, sizeof(a.vt), stride_grid((uint64_t)rk * 16), 1, 1, 256, stream, err, errlen);
     return rc;

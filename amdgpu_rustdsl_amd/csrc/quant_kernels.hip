@@ -94,6 +94,7 @@ struct QuantSeq32Args {
     uint8_t* q;          // [B, SK, HK, 128] e4m3
     uint8_t* scale;      // [B, ceil(SK/32), HK, 128] E8M0
     uint32_t B, SK, HK, nblk;
+    uint64_t tile0;      // the launch's first tile (tensors of more tiles than one launch can have)
 };
 
 // Rows: 16 lanes per 128-element row (8 elements per lane), 4 lanes per 32-element block. A workgroup covers
@@ -245,7 +246,7 @@ extern "C" __global__ void __launch_bounds__(256) fmha_mxfp8_quant_tensor(QuantT
 // re-read its last key, which changes no maximum, and are not stored.
 __device__ __forceinline__ void quant_seq32_group(const QuantSeq32Args& a, uint32_t group) {
     const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, r0 = lane >> 4;
-    uint64_t t = (uint64_t)group * 4u + (threadIdx.x >> 6);
+    uint64_t t = a.tile0 + (uint64_t)group * 4u + (threadIdx.x >> 6);
     const uint32_t hk = (uint32_t)(t % a.HK);
     t /= a.HK;
     const uint32_t blk = (uint32_t)(t % a.nblk);

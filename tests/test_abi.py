@@ -10,6 +10,7 @@ import os
 import re
 
 import pytest
+import torch
 
 import oracle
 from amdgpu_rustdsl_amd import lib
@@ -574,3 +575,14 @@ def test_code_objects_keep_m0_to_the_copies():
     if not os.path.exists(path):
         pytest.skip("not built")
     assert build.code_object_m0_misuse(path) == []
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the calls must end where they look for a device")
+def test_quantisers_take_more_tiles_than_one_launch_has():
+    """V with one scale per 32 keys of very many short sequences: 2^27 tiles are past what one launch can have and are not
+    refused (the call goes on to the device, which is missing here)."""
+    n, big = 1 << 27, 1 << 60
+    err = ctypes.create_string_buffer(256)
+    assert lib.raw.fmha_mxfp8_quantize_seq32(0x1000, 0x1000, 0x1000, n, 1, 1, big, big, big, None, err, 256) == lib.FMHA_ERR_NO_DEVICE, err.value
+    p = lib.QkvParams(*[0x1000] * 9, *[big] * 6, 1 << 33, 1 << 33, big, n, 1, 1, 1, 1, 1, 1.0, 0)
+    assert lib.raw.fmha_mxfp8_quantize_qkv(ctypes.byref(p), None, err, 256) == lib.FMHA_ERR_NO_DEVICE, err.value

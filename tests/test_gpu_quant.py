@@ -195,6 +195,24 @@ def test_qkv_matches_separate_quantisers(gpu, B, S, H, SK, HK, seq32):
         assert not vs2[1:512].any() and not vs[1:512].any()
 
 
+def test_seq32_more_tiles_than_one_launch(gpu):
+    """Sequences of one key, so many that their tiles take two launches: the last ones' bytes are those of a call of their own."""
+    if torch.cuda.get_device_properties(gpu).total_memory < 100 << 30:
+        pytest.skip("takes 34 GB of device memory")
+    B = (1 << 26) + 5
+    x = torch.empty(B, 1, 1, D, dtype=torch.bfloat16, device=gpu)
+    x.view(torch.int16).view(-1)[:1 << 20].random_(0x3000, 0x4000)
+    step = x.view(torch.int16).view(-1)[:1 << 20].view(-1, D)
+    x.view(torch.int16).view(B, D)[-(1 << 13):] = step
+    x.view(torch.int16).view(B, D)[(1 << 13):-(1 << 13)] = 0x3f80
+    q, sc = ops.quantize_v_seq32(x)
+    torch.cuda.synchronize()
+    for part in (slice(0, 100), slice(B - 100, B)):
+        q1, s1 = ops.quantize_v_seq32(x[part].contiguous())
+        assert torch.equal(q[part], q1) and torch.equal(sc[part], s1)
+    assert (q[1 << 13:-(1 << 13)] == q[1 << 13, 0, 0, 0]).all() and (sc[1 << 13:-(1 << 13)] == sc[1 << 13, 0, 0, 0]).all()
+
+
 def test_tensor_leaves_the_callers_words(gpu):
     """fmha_mxfp8_quantize_tensor writes word 0 and the partial maxima of a descale buffer and nothing between;
     fmha_mxfp8_quantize_v, for a fresh buffer, clears the words between. Same bytes and descale."""
