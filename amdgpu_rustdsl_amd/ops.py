@@ -96,7 +96,8 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
     so its output bits differ from the reference grid's by a few ULP; which fill runs depends on the device's CU
     count.
     """
-    if path in _PATH_CODES and causal_pair in _PAIR_MODES and partials in _PARTIAL_FORMATS:
+    known = isinstance(path, str) and path in _PATH_CODES and isinstance(partials, str) and partials in _PARTIAL_FORMATS
+    if known and causal_pair in _PAIR_MODES:
         split_path = path == "kvsplit"
         nsplit = (splits or 4) if split_path else 0
         if (not split_path or nsplit in (2, 4, 8)) and (softmax_scale is None or float(softmax_scale) > 0.0):

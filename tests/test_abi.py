@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle
-from amdgpu_rustdsl_amd import lib
+from amdgpu_rustdsl_amd import lib, ops
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADERS = [os.path.join(ROOT, "include", h) for h in ("fmha_mxfp8.h", "mxfp8_quant.h")]
@@ -531,7 +531,7 @@ def test_unchecked_split_keeps_the_32bit_guard():
 _CU_RULES = r"""
 import json, sys
 sys.path.insert(0, {root!r})
-from amdgpu_rustdsl_amd import lib
+from amdgpu_rustdsl_amd import lib, ops
 print(json.dumps({{
     "parts": [lib.kv_partials(1, 8, 128, 16384, 8), lib.kv_partials(1, 8, 512, 32768, 4), lib.kv_partials(1, 8, 2048, 2048, 4)],
     "st": [lib.uses_split_tiles("vs128", 2, 8, 1024, 1024, causal=True), lib.uses_split_tiles("t128", 16, 8, 512, 512, causal=True)],
@@ -575,6 +575,14 @@ def test_code_objects_keep_m0_to_the_copies():
     if not os.path.exists(path):
         pytest.skip("not built")
     assert build.code_object_m0_misuse(path) == []
+
+
+@pytest.mark.parametrize("kw", [dict(partials=["fp32"]), dict(path=["t128"]), dict(partials="fp64"), dict(path="t64")])
+def test_op_reports_unknown_options(kw):
+    """An option of any type that the op does not know is a ValueError."""
+    x = torch.zeros(1, 1, 1, 128, dtype=torch.uint8)
+    with pytest.raises(ValueError):
+        ops.fmha_fwd_mxfp8(x, x, x, x, x, x, x, **kw)
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the calls must end where they look for a device")
