@@ -201,9 +201,10 @@ def main():
     fl = flops_of(B, H, S, SK, causal)
     tflops = fl / (ms * 1e-3) / 1e12
 
-    # the dominant kernel alone through its C-ABI launcher, and the reference's timing method (median of 5 repetitions
+    # the dominant kernel alone, and the reference's timing method (median of 5 repetitions
     # of 100 launches) for the step and the kernel, repetitions interleaved
-    launch, kern_name = kernel_launcher(lib, q, k, v, qs, ks, vs, out, lse, used, B, H, HK, S, SK, causal, stream)
+    launch, kern_name = kernel_launcher(lib, q, k, v, qs, ks, vs, out, lse, used, B, H, HK, S, SK, causal, stream,
+                                        lambda: entry(*call_args))
     rcs = []
     kern = lambda: rcs.append(launch())
     step_reps, kern_reps = [], []
@@ -398,8 +399,9 @@ def main_quant(args, torch, lib, ops):
     print(json.dumps(line), flush=True)
 
 
-def kernel_launcher(lib, q, k, v, qs, ks, vs, out, lse, used, B, H, HK, S, SK, causal, stream):
-    """A launch of the main kernel alone (no combine) through its C-ABI launcher, validated once, and its name."""
+def kernel_launcher(lib, q, k, v, qs, ks, vs, out, lse, used, B, H, HK, S, SK, causal, stream, entry):
+    """A launch of the main kernel alone (no combine), and its name: the step's own call (`entry`) where one launch is the whole
+    step, else the split kernel through its C-ABI launcher, validated once."""
     import ctypes
     import torch
     from amdgpu_rustdsl_amd.ops import _cap
@@ -409,27 +411,26 @@ def kernel_launcher(lib, q, k, v, qs, ks, vs, out, lse, used, B, H, HK, S, SK, c
     a.ptr_lse = lse.data_ptr() if lse is not None else None
     sz = lib.BufferSizes(_cap(q), _cap(k), _cap(v), _cap(out), _cap(qs), _cap(ks), _cap(vs), 0, 0)
     st = stream.cuda_stream
-    path = used[0]
-    kernel = "fmha_fwd_hd128_mxfp8_v3_" + path
-    if path in ("vs128", "t128"):
-        split_tiles = lib.uses_split_tiles(path, B, H, S, SK, causal)
-        # the kernel the one-call entry runs: the split-tile kernel (t128's grid, 512 threads), the 256-thread t128
-        # kernel (128-row grids below the split-tile threshold) or the path's own; vs128 takes the 128-row grid when
-        # its 256-row grid is at most half the chip, and under the causal mask from 4 key tiles on
-        row128 = math.ceil(S / 256) * H * B <= 128 or (causal and math.ceil(SK / 128) >= 4)
-        on_t128 = path == "t128" or split_tiles or row128
-        grid = (math.ceil(S / (128 if on_t128 else 256)), H, B)
-        rc, msg = lib.validate("t128" if on_t128 else "vs128", a, sz, grid, HK=HK)
-        assert rc == 0, msg
+    if used[0] in ("vs128", "t128"):
+        # one launch is the whole step, so the step's own call is timed; the kernel's name follows the entry's rules
+        # (the fourteen preloaded arguments' kernels, except for the causal pairs and single waves and short recipes)
+        tiles, tiles128, tiles256 = math.ceil(SK / 128), math.ceil(S / 128), math.ceil(S / 256)
+        cus = torch.cuda.get_device_properties(q.device).multi_processor_count
+        split_tiles = lib.uses_split_tiles(used[0], B, H, S, SK, causal)
+        row128 = used[0] == "t128" or tiles256 * H * B <= 128 or (
+            causal and tiles >= 4 and not (tiles <= 8 and S > 128 and tiles256 * H * B > cus))
+        paired = causal and row128 and tiles128 > 1 and tiles128 * H * B > cus
         if split_tiles:
-            launch = lambda: lib.raw.fmha_mxfp8_launch_t128_split_tiles(ctypes.byref(a), *grid, st)
-        elif on_t128:
-            launch = lambda: lib.raw.fmha_mxfp8_launch_t128(ctypes.byref(a), *grid, st)
+            kernel = "v3_t128_split_tiles" if paired else "pre_split_tiles"
+        elif row128:
+            kernel = "v3_t128" if causal else "pre_t128_lut" if tiles < 4 else "pre_t128"
         else:
-            launch = lambda: lib.raw.fmha_mxfp8_launch_vs128(ctypes.byref(a), *grid, st)
-        if split_tiles:
-            kernel = "fmha_fwd_hd128_mxfp8_v3_t128_split_tiles"
+            kernel = "v3_vs128" if tiles < 4 else "pre_vs128"
+        kernel = "fmha_fwd_hd128_mxfp8_" + kernel
+        launch = entry
     else:
+        # the packed ABI's form of the step's split kernel, which only the entry launches
+        kernel = "fmha_fwd_hd128_mxfp8_v3_kvsplit"
         # the split kernel as the entry runs it: the partials that ran (the KV fill's), over the entry's workspace slots
         # in turn (one slot would have each launch write over the lines the previous one wrote)
         nsplit = used.partials
