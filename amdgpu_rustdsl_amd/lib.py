@@ -241,7 +241,7 @@ def run_auto(params, workspace=None, workspace_bytes=0, stream=None):
 
 
 def run_auto_ws(params, workspace=None, workspace_bytes=0, stream=None):
-    """fmha_fwd_hd128_mxfp8_auto_ws: run_auto with a workspace that the full-sequence paths may use too."""
+    """fmha_fwd_hd128_mxfp8_auto_ws: run_auto with a workspace (auto_workspace_bytes) that the full-sequence paths may use too."""
     return _run(_L.fmha_fwd_hd128_mxfp8_auto_ws, params, workspace, workspace_bytes, stream)
 
 

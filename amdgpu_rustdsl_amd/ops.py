@@ -67,8 +67,8 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
                    lse=None, causal=False, partials="fp16", softmax_scale=None, causal_pair="auto", kv_fill=True):
     """Attention forward on MXFP8 inputs with head dim 128, written into ``out``; returns the (path, splits) that ran,
     splits being the KV split's chunk count as in the reference op (0 off the KV split). The returned tuple's
-    ``.partials`` gives the partials per row that ran: the chunks times the blocks each chunk was spread over (the
-    KV fill below).
+    ``.partials`` gives the KV split's partials per row: the chunks times the blocks each chunk was spread over (the
+    KV fill below; 0 off the KV split).
 
     Scores are base-2: the kernels compute softmax2(q . k) over dequantised q and k, so a caller that wants the usual
     softmax(q k^T / sqrt(128)) multiplies q by log2(e) / sqrt(128) before quantising it (``fmha_fwd_bf16_via_mxfp8``
@@ -95,6 +95,10 @@ def fmha_fwd_mxfp8(q, k, v, q_scale, k_scale, v_scale, out, *, path="auto", spli
     per chunk. The fill changes the fp32 rounding order (each partial quantises P against its own running maximum),
     so its output bits differ from the reference grid's by a few ULP; which fill runs depends on the device's CU
     count.
+    Short query ranges (S <= 128) over many keys and grids a bit over a whole round of CUs may be spread over further
+    blocks whose partials are merged, on path="auto" (and, with ``kv_fill``, on the KV split, chosen or forced, where
+    ``.partials`` doesn't count them): P is quantised as in the path's own kernel, the sums are taken in another order. The
+    workspace for it is the call's own, taken by the stream it runs on; without memory for one the own kernel runs.
     """
     known = isinstance(path, str) and path in _PATH_CODES and isinstance(partials, str) and partials in _PARTIAL_FORMATS
     if known and causal_pair in _PAIR_MODES:

@@ -287,8 +287,8 @@ typedef struct fmha_mxfp8_params {
                                   workspace of several slots the call uses slot *ws_turn % slots and increments the
                                   word; NULL = slot 0. Calls that share a word take the slots in turn; callers with
                                   their own words (and workspaces) never affect each other's slots. */
-    int32_t* partials_out;     /* optional output (extension): the KV split's partials per row that ran (the chunks
-                                  times the KV fill; 0 off the KV split) */
+    int32_t* partials_out;     /* optional output (extension): the KV split's partials per row (the chunks times the KV
+                                  fill; 0 off the KV split). fmha_fwd_hd128_mxfp8_auto_ws may cut each of them further */
 } fmha_mxfp8_params;
 
 /* fmha_fwd_hd128_mxfp8_auto: dispatch + validate + launch (+ combine), all on
@@ -309,13 +309,15 @@ int fmha_fwd_hd128_mxfp8_auto(const fmha_mxfp8_params* p, void* workspace, size_
                               void* stream, int* path_out, int* splits_out, char* err, size_t errlen);
 
 /* Extension (no counterpart in the reference): the same entry for callers whose workspace serves one stream and every
- * shape. Same params, rules, errors and results; with path = -1 a short query range (S <= 128) over many key tiles may
- * then use the workspace on the full-sequence paths too, and on the KV split be cut further: the query heads of a
- * KV head are packed into one block's rows, and the key range is spread over several blocks whose f32 partials a merge
- * kernel adds up. Every share starts from the softmax reference of the whole range's first tile, so P is quantised as
- * the unsplit kernel does; the sums are taken in another order. Without enough workspace the path's own kernel runs.
- * A 256-row grid one round of CUs and a bit large may use it in the same way for the blocks past the last whole round.
- * fmha_mxfp8_auto_workspace_bytes: the workspace the call can use (one slot; 0 when it needs none). */
+ * shape. Same params, rules and errors. A short query range (S <= 128) over many key tiles may use the workspace on the
+ * full-sequence paths too (with path = -1), and on the KV split, chosen or forced, cut its partials further (with kv_fill =
+ * 0): the query heads of a KV head are packed into one block's rows, and the key range is spread over several blocks
+ * whose partials (f32; on the KV split in its own format) a merge kernel adds up. Every share starts from the softmax
+ * reference of the whole range's first tile, so P is quantised as the unsplit kernel does; the sums are taken in
+ * another order, so the outputs agree to a few 1e-3, not bit for bit. Without enough workspace the path's own kernel
+ * runs. A 256-row grid one round of CUs and a bit large may use it in the same way for the blocks past the last whole
+ * round (with path = -1). fmha_mxfp8_auto_workspace_bytes: the workspace the call can use (one slot; 0 when it needs
+ * none); partials_out does not tell it. Calls that may run at the same time need workspaces of their own. */
 int fmha_fwd_hd128_mxfp8_auto_ws(const fmha_mxfp8_params* p, void* workspace, size_t workspace_bytes,
                                  void* stream, int* path_out, int* splits_out, char* err, size_t errlen);
 size_t fmha_mxfp8_auto_workspace_bytes(const fmha_mxfp8_params* p);

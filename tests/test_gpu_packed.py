@@ -61,12 +61,25 @@ def _bf16(out):
     return out.float().cpu().numpy().reshape(-1).astype(np.float64)
 
 
-@pytest.mark.parametrize("f32", [0, 1], ids=["", "f32"])
-@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+GUARD = 4096
+
+
+def _workspace(need, gpu):
+    """`need` bytes of workspace (a NaN pattern) and GUARD bytes behind them, in one allocation."""
+    ws = torch.full((need + GUARD,), 0xff, dtype=torch.uint8, device=gpu)
+    ws[need:] = 0x5a
+    return ws
+
+
+def _guard_untouched(ws, need):
+    return bool((ws[need:] == 0x5a).all())
+
+
+# the partial format is the KV split's
+@pytest.mark.parametrize("case,f32", [(c, f) for c in CASES for f in ((0, 1) if c[10] == "kvsplit" else (0,))],
+                         ids=[c[0] + s for c in CASES for s in (("", "-f32") if c[10] == "kvsplit" else ("",))])
 def test_packed_matches_own_kernel(gpu, case, f32):
     name, B, H, HK, S, SK, causal, seq32, scale, want_lse, path, splits = case
-    if f32 and path != "kvsplit":
-        pytest.skip("the partial format is the KV split's")
     print(f"[case] packed {name}", flush=True)
     inp = oracle.Inputs(B, H, S, SK, HK=HK, causal=causal, v_seq32=seq32, qk_scale=scale)
     t = gpu_util.upload(inp, gpu)
@@ -80,7 +93,7 @@ def test_packed_matches_own_kernel(gpu, case, f32):
     out, lse = outputs()
     p = _params(t, out, lse, B, H, HK, S, SK, causal, seq32, scale, path, splits, f32)
     need = lib.auto_workspace_bytes(p)
-    ws = torch.full((max(need, 256),), 0xff, dtype=torch.uint8, device=gpu)
+    ws = _workspace(need, gpu)
     ran = lib.run_auto_ws(p, ws.data_ptr(), need, st)
     ref, ref_lse = outputs()
     p2 = _params(t, ref, ref_lse, B, H, HK, S, SK, causal, seq32, scale, path, splits, f32)
@@ -88,7 +101,7 @@ def test_packed_matches_own_kernel(gpu, case, f32):
         assert (need > 0) == (not name.endswith("is_not_packed")), need
         ran2 = lib.run_auto(p2, None, 0, st)     # no workspace: the path's own kernel
     else:
-        # the reference-named pair on the partials that the entry reports
+        # the reference-named pair on the partials that the entry reports (the packed rows cut each of them further)
         parts = lib.kv_partials(B, H, S, SK, splits)
         own = lib.workspace_bytes(B, H, S, parts)
         assert ran.partials == parts and (need > own or (f32 and need == own))   # f32 rows may not pay for more shares
@@ -106,9 +119,10 @@ def test_packed_matches_own_kernel(gpu, case, f32):
         assert lib.raw.fmha_mxfp8_launch_kvsplit(ctypes.byref(ka), math.ceil(S / 256), H, B * parts, st) == 0
         ca = lib.CombineArgs(ka.ptr_ohat, ka.ptr_lse, ref.data_ptr(), rows, 128, parts | fmt)
         assert lib.raw.fmha_mxfp8_launch_combine(ctypes.byref(ca), (rows * 16 + 255) // 256, st) == 0
-        ran2 = ran
+        ran2 = ("kvsplit", splits)
     torch.cuda.synchronize()
     assert tuple(ran) == tuple(ran2)
+    assert _guard_untouched(ws, need)
     x, y = _bf16(out), _bf16(ref)
     assert not np.isnan(x).any()
     rms = np.sqrt(np.mean(y * y))
@@ -137,12 +151,11 @@ def test_workspace_too_small_runs_own_kernel(gpu):
     one = lib.workspace_bytes(B, H, S, 1)
     assert need > 2 * one
     for size in (need, 2 * one, 2 * one - 1, 0):
-        ws = torch.full((max(size, 256),), 0xff, dtype=torch.uint8, device=gpu)
-        guard = torch.full((4096,), 0x5a, dtype=torch.uint8, device=gpu)
+        ws = _workspace(size, gpu)
         out.zero_()
         lib.run_auto_ws(p, ws.data_ptr() if size else None, size, st)
         torch.cuda.synchronize()
-        assert (guard == 0x5a).all()
+        assert _guard_untouched(ws, size)
         got.append(_bf16(out))
     for g in got[:-1]:
         assert np.linalg.norm(g - got[-1]) / np.linalg.norm(got[-1]) <= 6e-3

@@ -15,7 +15,7 @@ import torch
 import oracle
 from amdgpu_rustdsl_amd import lib
 from tests import gpu_util
-from tests.test_gpu_packed import _bf16, _params
+from tests.test_gpu_packed import _bf16, _guard_untouched, _params, _workspace
 
 pytestmark = pytest.mark.gpu
 D = 128
@@ -53,10 +53,10 @@ def test_split_last_blocks(gpu, case):
         p = _params(t, out, lse, B, H, HK, S, SK, False, seq32, scale, "auto", 0)
         need = lib.auto_workspace_bytes(p)
         assert need > 0
-        ws = torch.full((need,), 0xff, dtype=torch.uint8, device=gpu)
+        ws = _workspace(need, gpu)
         ran = lib.run_auto_ws(p, ws.data_ptr(), need, st) if use_ws else lib.run_auto(p, None, 0, st)
         torch.cuda.synchronize()
-        assert tuple(ran) == ("vs128", 0)
+        assert tuple(ran) == ("vs128", 0) and _guard_untouched(ws, need)
         res.append((out, lse))
     (x, xl), (y, yl) = res
     # [B, S, H] mask of the split blocks' rows: block l = (b H + h) gx + query tile, from the last whole round on
