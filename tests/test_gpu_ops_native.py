@@ -275,9 +275,10 @@ def test_without_memory_for_a_workspace(gpu):
     spare = []
     try:
         torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(gpu) / total, gpu)
-        with pytest.raises(torch.OutOfMemoryError):   # what the live tensors' segments have left
-            while True:
-                spare.append(torch.empty(1 << 20, dtype=torch.uint8, device=gpu))
+        for size in (32 << 20, 4 << 20):   # what the live tensors' segments have left, down to less than the workspaces
+            with pytest.raises(torch.OutOfMemoryError):
+                while True:
+                    spare.append(torch.empty(size, dtype=torch.uint8, device=gpu))
         ops.fmha_fwd_mxfp8(*t, out)
         torch.cuda.synchronize()
         with pytest.raises(torch.OutOfMemoryError):
