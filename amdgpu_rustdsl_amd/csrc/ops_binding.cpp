@@ -62,10 +62,14 @@ struct RelaxedCapture {
 };
 
 // Whether the allocation lies in a pool that torch keeps apart from the ordinary ones (a graph's, while torch captures it).
+// Allocators that cannot tell have none that is known here.
 bool in_private_pool(const void* ptr) {
     const size_t a = (size_t)(uintptr_t)ptr;
-    for (const auto& s : c10::hip::HIPCachingAllocator::get()->snapshot().segments)
-        if (a >= s.address && a < s.address + s.total_size) return s.owner_private_pool_id.first != 0 || s.owner_private_pool_id.second != 0;
+    try {
+        for (const auto& s : c10::hip::HIPCachingAllocator::get()->snapshot().segments)
+            if (a >= s.address && a < s.address + s.total_size) return s.owner_private_pool_id.first != 0 || s.owner_private_pool_id.second != 0;
+    } catch (const std::exception&) {
+    }
     return false;
 }
 
