@@ -422,7 +422,7 @@ int kernel_of(int path, i64 B, i64 H, i64 S, i64 SK, bool causal, bool pair_aske
 
 // Fills the plan of a shape whose path (and, for the KV split, chunk count) is resolved. `workspace` is what the call may
 // use: partials that do not fit lower the fill, then the shares. `any_path` (fmha_fwd_hd128_mxfp8_auto_ws): shares, and a
-// workspace on the full-sequence paths too; the other entries keep the kernels and the bits that they had.
+// workspace on the full-sequence paths too; the other entries run the path's own kernels.
 void make_plan(Plan& pl, const fmha_mxfp8_params& p, bool scaled, size_t workspace, bool any_path) {
     const i64 B = p.B, H = p.H, HK = p.HK, S = p.S, SK = p.SK;
     fmha_pre_args fits_pre;   // the packed rows and the split last blocks exist on preloaded parameters only

@@ -122,7 +122,8 @@ struct Prm {
 #endif
 };
 
-// Debug builds (-DFMHA_TRACE) record s_memrealtime (100 MHz) at phase boundaries: slot i of wave w of logical block
+// Debug builds (-DFMHA_TRACE) of the packed-ABI kernels, launched directly (the one-call entry's own kernels run the same
+// bodies on parameters that have no room for the pointer, and record nothing), record s_memrealtime (100 MHz) at phase boundaries: slot i of wave w of logical block
 // blk at trace[(blk * 8 + w) * 8 + i], written by lane 0 with a vector store. Release builds compile it away.
 #ifdef FMHA_TRACE
 #define FMHA_MARK(p, blk, i)                                                                                  \
