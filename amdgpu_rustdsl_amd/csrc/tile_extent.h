@@ -12,7 +12,7 @@
 #endif
 
 // Bytes from a tile's first row that its copies may read: `left` rows lie before the end of the range (none when it is negative),
-// a tile has 128. The rows are clamped before they are multiplied, so the size is below 2^31 for every stride up to 16 MiB
+// a tile has 128. The rows are clamped before they are multiplied, so the size is below 2^31 for every stride below 16 MiB
 // (65536 KV heads are 8 MiB): a whole K of 2 GiB or more, or many heads past a short range, would wrap. No copy addresses the
 // other heads' bytes behind the last row's own.
 FMHA_TILE_FN uint32_t tile_extent(int32_t left, uint32_t stride) {
