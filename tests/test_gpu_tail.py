@@ -119,6 +119,18 @@ def test_causal_256row_grid(gpu, case):
     assert torch.isfinite(lse).all()
 
 
+@pytest.mark.parametrize("seq32,scale", [(False, 0.0), (True, 0.0), (False, 0.7), (True, 0.7)], ids=["plain", "seq32", "scaled", "scaled_seq32"])
+@pytest.mark.parametrize("B,H,HK,S,SK", [(5, 56, 28, 129, 385), (40, 8, 2, 200, 1024), (2, 48, 48, 511, 640)])
+def test_causal_256row_grid_forms(gpu, B, H, HK, S, SK, seq32, scale):
+    """The 256-row kernel and the pairs it stands in for, over the forms that both take: the same bits and LSE bits."""
+    print(f"[case] causal 256-row forms B{B} H{H} S{S} SK{SK} {seq32} {scale}", flush=True)
+    inp = oracle.Inputs(B, H, S, SK, HK=HK, causal=True, v_seq32=seq32, qk_scale=scale)
+    out, _, lse = gpu_util.run(inp, gpu, lse=True)
+    paired, _, plse = gpu_util.run(inp, gpu, lse=True, causal_pair=True)
+    np.testing.assert_array_equal(out, paired)
+    assert torch.equal(lse, plse) and torch.isfinite(lse).all()
+
+
 def test_asked_pairing_runs_the_paired_kernel(gpu):
     """causal_pair=True runs the query-tile pairs of the 128-row kernel also where the automatic choice is the 256-row one."""
     from torch.profiler import ProfilerActivity, profile
