@@ -149,8 +149,9 @@ bool use_split_tiles(int64_t B, int64_t H, int64_t S, int64_t SK, bool causal) {
 // Causal (extension): always from 4 key tiles on, so that the 128-row grid's causal q-tile pairing is available past one
 // wave of blocks, except where the 256-row kernel gives the same bits sooner: grids of more 256-row blocks than CUs with
 // 4 to 8 key tiles, whose 128-row form is the 256-thread kernel. With its heaviest query tiles first the 256-row kernel
-// balances as well as the pairs do (us, 128-row / 256-row: B16 H8 S512 15.9 / 14.3, B9 H8 S1000 36.6 / 34.7, B16 H8 S1024
-// 39.3 / 37.7; S < SK: B32 H8 S256 SK1024 34.1 / 23.1, B16 H8 S768 SK1024 42.5 / 34.9). With at most 128 query rows half of
+// balances as well as the pairs do (us, 128-row / 256-row: B8 H16 S600 30.7 / 26.9, B9 H8 S1000 36.6 / 34.7, B16 H8 S1024
+// 39.3 / 37.7; S < SK: B33 H8 S400 SK512 51.2 / 36.6, B16 H8 S768 SK1024 42.5 / 34.9, B40 H8 S140 SK1000 58.0 / 36.3; with V
+// scales per 32 keys and the in-kernel scale the same way round). With at most 128 query rows half of
 // its block is padding (B64 H8 S128 SK1024 38.4 / 40.9). A caller that asks for the pairing has it. From 9 key tiles on the 128-row
 // form is the split-tile kernel, whose error against float64 is the smaller one (relative, split-tile / 256-row, three
 // seeds each: B8 H8 S1152 0.0241 / 0.0245, S2048 0.0249 / 0.0252, B1 H32 HK8 S6144 0.0261 / 0.0264): it stays, though the
